@@ -4,10 +4,12 @@
 // power spectrum and the instability verdict of the VFP solver.
 //
 // Dense layers: y = x W^T + b with W [out][in].  The products run on the
-// matrix cores (MFMA 16x16x32, BF16 operands, FP32 accumulation), one
-// wavefront per 16x16 output tile, with the bias, GELU and its derivative
-// fused into the store.  Master weights, gradients and Adam moments are
-// FP32; each step writes the BF16 copy the products read.
+// matrix cores (MFMA 16x16x32, BF16 operands, FP32 accumulation).  Networks
+// whose activations fit the LDS run as two kernels (mlp_fused.hpp); wider or
+// deeper ones layer by layer, one wavefront per 16x16 output tile, with the
+// bias, GELU and its derivative fused into the store.  Master weights,
+// gradients and Adam moments are FP32; each step writes the BF16 copy the
+// products read.
 //
 // Parameter layout (flattened FP32): for each layer W (out x in, row-major)
 // then b (out).
@@ -19,41 +21,12 @@
 #include <vector>
 
 #include "common.hpp"
+#include "mlp_fused.hpp"
 #include "reduce.hpp"
 
 namespace {
 
-typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// float -> bfloat16, round to nearest even (NaN stays NaN)
-__host__ __device__ inline uint16_t f2bf(float f)
-{
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if ((u & 0x7F800000u) == 0x7F800000u && (u & 0x007FFFFFu)) {
-        return (uint16_t)((u >> 16) | 0x0040u);
-    }
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-
-__host__ __device__ inline float bf2f(uint16_t h)
-{
-    return __builtin_bit_cast(float, (uint32_t)h << 16);
-}
-
-// GELU with the exact Gaussian CDF: x Phi(x), and its derivative
-__device__ inline float gelu(float x)
-{
-    return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
-}
-__device__ inline float gelu_grad(float x)
-{
-    const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
-    const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
-    return cdf + x * pdf;
-}
+using namespace vfps_impl;
 
 enum Epilogue : int {
     EPI_STORE = 0,       // C fp32
@@ -212,29 +185,21 @@ __global__ void colsum_kernel(const float* __restrict__ dZ, uint32_t B, uint32_t
     db[j] = s;
 }
 
-// Adam (Kingma & Ba): m = b1 m + (1-b1) g; v = b2 v + (1-b2) g^2;
-// p -= lr (m / (1 - b1^t)) / (sqrt(v / (1 - b2^t)) + eps); BF16 copy of p
 __global__ void adam_kernel(float* __restrict__ p, uint16_t* __restrict__ pb,
                             const float* __restrict__ g, float* __restrict__ m,
-                            float* __restrict__ v, size_t n, float lr, float b1,
-                            float b2, float eps, float c1, float c2)
+                            float* __restrict__ v, size_t n, AdamArgs a)
 {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x) {
-        const float gi = g[i];
-        const float mi = b1 * m[i] + (1.0f - b1) * gi;
-        const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-        m[i] = mi;
-        v[i] = vi;
-        const float mh = mi / c1;
-        const float vh = vi / c2;
-        const float pi = p[i] - lr * mh / (sqrtf(vh) + eps);
-        p[i] = pi;
-        pb[i] = f2bf(pi);
+        const float pi = adam_update(a, g[i], p + i, m + i, v + i);
+        if (pb) pb[i] = f2bf(pi);
     }
 }
 
 }  // namespace
+
+// most samples of a forward staged through pinned memory
+constexpr uint32_t MLP_STAGE_ROWS = 1024;
 
 struct vfps_mlp {
     vfps_dev* dev = nullptr;
@@ -248,6 +213,22 @@ struct vfps_mlp {
     float* m = nullptr;             // Adam moments
     float* v = nullptr;
     uint32_t t = 0;                 // Adam steps taken
+    // the two-kernel form (net.L > 0)
+    MlpNet net;
+    uint16_t* W = nullptr;          // padded BF16 weights, and transposed
+    uint16_t* WT = nullptr;
+    uint16_t* AT = nullptr;         // layer inputs and dZ [feature][sample]
+    uint16_t* GT = nullptr;
+    float* dbp = nullptr;           // bias and loss partials
+    double* lossp = nullptr;
+    // pinned staging of a forward's inputs and outputs, which the kernel
+    // reads and writes itself
+    float* stage = nullptr;
+    uint32_t stage_rows = 0;
+    // training data kept between calls of train (grown as needed)
+    void* data = nullptr;
+    size_t data_bytes = 0;
+    bool fused() const { return net.L > 0; }
     // workspace
     float* x = nullptr;             // [B][n_in]
     uint16_t* xb = nullptr;
@@ -273,9 +254,12 @@ void mlp_free(vfps_mlp* m)
     for (void* q : {(void*)m->p, (void*)m->pb, (void*)m->g, (void*)m->m,
                     (void*)m->v, (void*)m->x, (void*)m->xb, (void*)m->dy,
                     (void*)m->dyb, (void*)m->dz2, (void*)m->dzb2,
-                    (void*)m->tgt, (void*)m->lab, (void*)m->loss}) {
+                    (void*)m->tgt, (void*)m->lab, (void*)m->loss,
+                    (void*)m->W, (void*)m->WT, (void*)m->AT, (void*)m->GT,
+                    (void*)m->dbp, (void*)m->lossp, m->data}) {
         (void)hipFree(q);
     }
+    if (m->stage) (void)hipHostFree(m->stage);
     for (auto* q : m->z) (void)hipFree(q);
     for (auto* q : m->ab) (void)hipFree(q);
     delete m;
@@ -378,42 +362,131 @@ int backward(vfps_mlp* m, uint32_t B)
     return VFPS_OK;
 }
 
-int upload_inputs(vfps_mlp* m, const float* x, uint32_t B, bool host)
+// ---- the two-kernel form ------------------------------------------------------
+
+// a batch's samples on the device: rows idx (null: 0, 1, ...) of x, T, lab
+struct Batch {
+    const float *x, *T, *lab;
+    const uint32_t* idx;
+    uint32_t B;
+};
+
+int fused_forward(vfps_mlp* m, const float* x, uint32_t B, float* y)
 {
-    hipStream_t st = m->dev->stream;
-    const size_t n = (size_t)B * m->dims[0];
-    if (host) {
-        VFPS_HIP(hipMemcpyAsync(m->x, x, sizeof(float) * n, hipMemcpyHostToDevice, st));
-    }
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(std::min<size_t>((n + 255) / 256, 1024)),
-                       dim3(256), 0, st, m->x, m->xb, n);
+    MlpRowsArgs a{};
+    a.W = m->W;
+    a.p = m->p;
+    a.x = x;
+    a.B = B;
+    a.Y = y;
+    hipLaunchKernelGGL(mlp_rows_kernel<false>, dim3((B + MLP_ROWS - 1) / MLP_ROWS),
+                       dim3(MLP_THREADS), sizeof(float) * m->net.lds_words,
+                       m->dev->stream, m->net, a);
     VFPS_HIP(hipGetLastError());
     return VFPS_OK;
 }
 
-int loss_and_grad(vfps_mlp* m, uint32_t B, float wl)
+// loss and gradients of a batch; with `adam` also the update
+int fused_step(vfps_mlp* m, const Batch& b, float wl, float* loss,
+               const AdamArgs* adam)
+{
+    hipStream_t st = m->dev->stream;
+    const uint32_t blocks = ((b.B + 31u) & ~31u) / MLP_ROWS;
+    MlpRowsArgs a{};
+    a.W = m->W;
+    a.WT = m->WT;
+    a.p = m->p;
+    a.x = b.x;
+    a.idx = b.idx;
+    a.B = b.B;
+    a.T = b.T;
+    a.labels = b.lab;
+    a.wl = wl;
+    a.AT = m->AT;
+    a.GT = m->GT;
+    a.dbp = m->dbp;
+    a.lossp = m->lossp;
+    hipLaunchKernelGGL(mlp_rows_kernel<true>, dim3(blocks), dim3(MLP_THREADS),
+                       sizeof(float) * m->net.lds_words, st, m->net, a);
+    MlpGradArgs g{};
+    g.AT = m->AT;
+    g.GT = m->GT;
+    g.dbp = m->dbp;
+    g.lossp = m->lossp;
+    g.B = b.B;
+    g.g = m->g;
+    g.loss = loss;
+    uint32_t tiles = 0;
+    for (uint32_t l = 0; l < m->net.L; l++) tiles += mlp_grad_tiles(m->net, l);
+    const uint32_t tb = (tiles + 3u) / 4u;
+    const uint32_t bb = (m->net.nbias + MLP_GRAD_THREADS - 1) / MLP_GRAD_THREADS;
+    if (adam) {
+        g.p = m->p;
+        g.m = m->m;
+        g.v = m->v;
+        g.W = m->W;
+        g.WT = m->WT;
+        g.adam = *adam;
+        hipLaunchKernelGGL(mlp_grad_kernel<true>, dim3(tb + bb),
+                           dim3(MLP_GRAD_THREADS), 0, st, m->net, g, tb);
+    } else {
+        hipLaunchKernelGGL(mlp_grad_kernel<false>, dim3(tb + bb),
+                           dim3(MLP_GRAD_THREADS), 0, st, m->net, g, tb);
+    }
+    VFPS_HIP(hipGetLastError());
+    return VFPS_OK;
+}
+
+int fused_pack(vfps_mlp* m)
+{
+    hipLaunchKernelGGL(mlp_pack_kernel,
+                       dim3(std::min(1024u, (m->net.wsize + 255u) / 256u)),
+                       dim3(256), 0, m->dev->stream, m->net, m->p, m->W, m->WT);
+    VFPS_HIP(hipGetLastError());
+    return VFPS_OK;
+}
+
+// ---- layer by layer ------------------------------------------------------------
+
+int upload_inputs(vfps_mlp* m, uint32_t B)
+{
+    const size_t n = (size_t)B * m->dims[0];
+    hipLaunchKernelGGL(to_bf16_kernel, dim3(std::min<size_t>((n + 255) / 256, 1024)),
+                       dim3(256), 0, m->dev->stream, m->x, m->xb, n);
+    VFPS_HIP(hipGetLastError());
+    return VFPS_OK;
+}
+
+int loss_and_grad(vfps_mlp* m, uint32_t B, float wl, float* loss)
 {
     hipStream_t st = m->dev->stream;
     const uint32_t S = m->dims.back() - 1;
-    int rc = forward(m, B);
+    int rc = upload_inputs(m, B);
     if (rc != VFPS_OK) return rc;
+    if ((rc = forward(m, B)) != VFPS_OK) return rc;
     hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, st,
                        m->z[m->nlayers() - 1], m->tgt, m->lab, B, S, wl, m->dy,
-                       m->dyb, m->loss);
+                       m->dyb, loss);
     VFPS_HIP(hipGetLastError());
     return backward(m, B);
 }
 
-int adam(vfps_mlp* m, float lr, float b1, float b2, float eps)
+AdamArgs next_adam(vfps_mlp* m, float lr, float b1, float b2, float eps)
 {
     m->t++;
-    const float c1 = 1.0f - std::pow(b1, (float)m->t);
-    const float c2 = 1.0f - std::pow(b2, (float)m->t);
+    return {lr, b1, b2, eps, 1.0f - std::pow(b1, (float)m->t),
+            1.0f - std::pow(b2, (float)m->t)};
+}
+
+// the update of all parameters from the gradients in m->g
+int adam(vfps_mlp* m, float lr, float b1, float b2, float eps)
+{
+    const AdamArgs a = next_adam(m, lr, b1, b2, eps);
     hipLaunchKernelGGL(adam_kernel, dim3(std::min<size_t>((m->nparams + 255) / 256, 1024)),
                        dim3(256), 0, m->dev->stream, m->p, m->pb, m->g, m->m,
-                       m->v, m->nparams, lr, b1, b2, eps, c1, c2);
+                       m->v, m->nparams, a);
     VFPS_HIP(hipGetLastError());
-    return VFPS_OK;
+    return m->fused() ? fused_pack(m) : VFPS_OK;
 }
 
 uint64_t splitmix(uint64_t& s)
@@ -465,8 +538,11 @@ int vfps_mlp_create(vfps_dev* dev, const uint32_t* dims, uint32_t ndims,
         }
     }
     const size_t n = off;
+    m->net = mlp_net(dims, ndims, max_batch);
+    if (m->fused() && sizeof(float) * m->net.lds_words > dev->lds_max) {
+        m->net = MlpNet{};
+    }
     VFPS_HIP(hipMalloc(&m->p, sizeof(float) * n));
-    VFPS_HIP(hipMalloc(&m->pb, sizeof(uint16_t) * n));
     VFPS_HIP(hipMalloc(&m->g, sizeof(float) * n));
     VFPS_HIP(hipMalloc(&m->m, sizeof(float) * n));
     VFPS_HIP(hipMalloc(&m->v, sizeof(float) * n));
@@ -476,6 +552,38 @@ int vfps_mlp_create(vfps_dev* dev, const uint32_t* dims, uint32_t ndims,
     const size_t B = max_batch;
     const uint32_t W = m->maxw();
     VFPS_HIP(hipMalloc(&m->x, sizeof(float) * B * dims[0]));
+    VFPS_HIP(hipMalloc(&m->tgt, sizeof(float) * B * (dims[ndims - 1] - 1)));
+    VFPS_HIP(hipMalloc(&m->lab, sizeof(float) * B));
+    VFPS_HIP(hipMalloc(&m->loss, sizeof(float)));
+    if (m->fused()) {
+        const MlpNet& k = m->net;
+        const int lds = (int)(sizeof(float) * k.lds_words);
+        if (lds > 65536) {
+            for (const void* fn : {(const void*)&mlp_rows_kernel<false>,
+                                   (const void*)&mlp_rows_kernel<true>}) {
+                VFPS_HIP(hipFuncSetAttribute(
+                    fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                    (int)MLP_LDS_MAX));
+            }
+        }
+        const size_t nwg = k.bmax / MLP_ROWS;
+        VFPS_HIP(hipMalloc(&m->W, sizeof(uint16_t) * k.wsize));
+        VFPS_HIP(hipMalloc(&m->WT, sizeof(uint16_t) * k.wsize));
+        VFPS_HIP(hipMalloc(&m->AT, sizeof(uint16_t) * k.arows * k.bmax));
+        VFPS_HIP(hipMalloc(&m->GT, sizeof(uint16_t) * k.grows * k.bmax));
+        VFPS_HIP(hipMalloc(&m->dbp, sizeof(float) * nwg * k.nbias));
+        VFPS_HIP(hipMalloc(&m->lossp, sizeof(double) * nwg));
+        // (the outputs of a forward longer than the staging)
+        VFPS_HIP(hipMalloc(&m->dy, sizeof(float) * B * dims[ndims - 1]));
+        m->stage_rows = std::min(max_batch, MLP_STAGE_ROWS);
+        VFPS_HIP(hipHostMalloc((void**)&m->stage,
+                               sizeof(float) * (size_t)m->stage_rows *
+                                   (dims[0] + dims[ndims - 1]),
+                               hipHostMallocDefault));
+        *out = guard.release();
+        return vfps_mlp_set_params(*out, p.data(), n);
+    }
+    VFPS_HIP(hipMalloc(&m->pb, sizeof(uint16_t) * n));
     VFPS_HIP(hipMalloc(&m->xb, sizeof(uint16_t) * B * dims[0]));
     for (uint32_t l = 0; l + 1 < ndims; l++) {
         float* z = nullptr;
@@ -491,9 +599,6 @@ int vfps_mlp_create(vfps_dev* dev, const uint32_t* dims, uint32_t ndims,
     VFPS_HIP(hipMalloc(&m->dyb, sizeof(uint16_t) * B * W));
     VFPS_HIP(hipMalloc(&m->dz2, sizeof(float) * B * W));
     VFPS_HIP(hipMalloc(&m->dzb2, sizeof(uint16_t) * B * W));
-    VFPS_HIP(hipMalloc(&m->tgt, sizeof(float) * B * (dims[ndims - 1] - 1)));
-    VFPS_HIP(hipMalloc(&m->lab, sizeof(float) * B));
-    VFPS_HIP(hipMalloc(&m->loss, sizeof(float)));
     *out = guard.release();
     return vfps_mlp_set_params(*out, p.data(), n);
     VFPS_TRY_END
@@ -518,8 +623,14 @@ int vfps_mlp_set_params(vfps_mlp* m, const float* params, size_t n)
                    "vfps_mlp_set_params: size mismatch");
     hipStream_t st = m->dev->stream;
     VFPS_HIP(hipMemcpyAsync(m->p, params, sizeof(float) * n, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(std::min<size_t>((n + 255) / 256, 1024)),
-                       dim3(256), 0, st, m->p, m->pb, n);
+    if (m->fused()) {
+        int rc = fused_pack(m);
+        if (rc != VFPS_OK) return rc;
+    } else {
+        hipLaunchKernelGGL(to_bf16_kernel,
+                           dim3(std::min<size_t>((n + 255) / 256, 1024)),
+                           dim3(256), 0, st, m->p, m->pb, n);
+    }
     VFPS_HIP(hipGetLastError());
     VFPS_HIP(hipMemsetAsync(m->m, 0, sizeof(float) * n, st));
     VFPS_HIP(hipMemsetAsync(m->v, 0, sizeof(float) * n, st));
@@ -545,13 +656,34 @@ int vfps_mlp_forward(vfps_mlp* m, const float* x, uint32_t B, float* y)
 {
     VFPS_CHECK_ARG(m && x && y && B >= 1 && B <= m->max_batch,
                    "vfps_mlp_forward: bad argument");
-    int rc = upload_inputs(m, x, B, true);
+    hipStream_t st = m->dev->stream;
+    const uint32_t no = m->dims.back();
+    const size_t nx = (size_t)B * m->dims[0], ny = (size_t)B * no;
+    int rc;
+    if (m->fused() && B <= m->stage_rows) {
+        // the kernel reads the inputs from and writes the outputs to pinned
+        // host memory: no copy launches around it (3-256-256-256-65, 512
+        // samples: two copies were half of the call)
+        float* ys = m->stage + (size_t)m->stage_rows * m->dims[0];
+        std::memcpy(m->stage, x, sizeof(float) * nx);
+        if ((rc = fused_forward(m, m->stage, B, ys)) != VFPS_OK) return rc;
+        VFPS_HIP(hipStreamSynchronize(st));
+        std::memcpy(y, ys, sizeof(float) * ny);
+        return VFPS_OK;
+    }
+    VFPS_HIP(hipMemcpyAsync(m->x, x, sizeof(float) * nx, hipMemcpyHostToDevice,
+                            st));
+    const float* yd = m->dy;
+    if (m->fused()) {
+        rc = fused_forward(m, m->x, B, m->dy);
+    } else {
+        yd = m->z[m->nlayers() - 1];
+        rc = upload_inputs(m, B);
+        if (rc == VFPS_OK) rc = forward(m, B);
+    }
     if (rc != VFPS_OK) return rc;
-    if ((rc = forward(m, B)) != VFPS_OK) return rc;
-    VFPS_HIP(hipMemcpyAsync(y, m->z[m->nlayers() - 1],
-                            sizeof(float) * B * m->dims.back(),
-                            hipMemcpyDeviceToHost, m->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(m->dev->stream));
+    VFPS_HIP(hipMemcpyAsync(y, yd, sizeof(float) * ny, hipMemcpyDeviceToHost, st));
+    VFPS_HIP(hipStreamSynchronize(st));
     return VFPS_OK;
 }
 
@@ -563,13 +695,17 @@ int vfps_mlp_loss_grad(vfps_mlp* m, const float* x, const float* target,
                    "vfps_mlp_loss_grad: bad argument");
     hipStream_t st = m->dev->stream;
     const uint32_t S = m->dims.back() - 1;
-    int rc = upload_inputs(m, x, B, true);
-    if (rc != VFPS_OK) return rc;
+    VFPS_HIP(hipMemcpyAsync(m->x, x, sizeof(float) * B * m->dims[0],
+                            hipMemcpyHostToDevice, st));
     VFPS_HIP(hipMemcpyAsync(m->tgt, target, sizeof(float) * B * S,
                             hipMemcpyHostToDevice, st));
     VFPS_HIP(hipMemcpyAsync(m->lab, label, sizeof(float) * B,
                             hipMemcpyHostToDevice, st));
-    if ((rc = loss_and_grad(m, B, label_weight)) != VFPS_OK) return rc;
+    const int rc = m->fused()
+                       ? fused_step(m, {m->x, m->tgt, m->lab, nullptr, B},
+                                    label_weight, m->loss, nullptr)
+                       : loss_and_grad(m, B, label_weight, m->loss);
+    if (rc != VFPS_OK) return rc;
     if (loss) {
         VFPS_HIP(hipMemcpyAsync(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost, st));
     }
@@ -600,72 +736,71 @@ int vfps_mlp_train(vfps_mlp* m, const float* x, const float* target,
     VFPS_TRY_BEGIN
     hipStream_t st = m->dev->stream;
     const uint32_t nin = m->dims[0], S = m->dims.back() - 1;
-    float *dx = nullptr, *dt = nullptr, *dl = nullptr, *losses = nullptr;
-    uint32_t* didx = nullptr;
     const uint32_t nb = (N + batch - 1) / batch;
-    int rc = VFPS_OK;
-    auto cleanup = [&]() {
-        (void)hipFree(dx);
-        (void)hipFree(dt);
-        (void)hipFree(dl);
-        (void)hipFree(didx);
-        (void)hipFree(losses);
-    };
-    if (hipMalloc(&dx, sizeof(float) * N * nin) != hipSuccess ||
-        hipMalloc(&dt, sizeof(float) * N * S) != hipSuccess ||
-        hipMalloc(&dl, sizeof(float) * N) != hipSuccess ||
-        hipMalloc(&didx, sizeof(uint32_t) * N) != hipSuccess ||
-        hipMalloc(&losses, sizeof(float) * nb) != hipSuccess) {
-        cleanup();
-        return vfps_impl::fail(VFPS_ERR_NOMEM, "vfps_mlp_train: device memory");
+    // samples, targets, labels, the epoch's order and losses
+    const size_t fx = (size_t)N * nin, ft = (size_t)N * S;
+    const size_t need = sizeof(float) * (fx + ft + 2 * (size_t)N + nb);
+    if (need > m->data_bytes) {
+        VFPS_HIP(hipStreamSynchronize(st));
+        VFPS_HIP(hipFree(m->data));
+        m->data = nullptr;
+        m->data_bytes = 0;
+        if (hipMalloc(&m->data, need) != hipSuccess) {
+            return fail(VFPS_ERR_NOMEM, "vfps_mlp_train: device memory");
+        }
+        m->data_bytes = need;
     }
-    if (hipMemcpy(dx, x, sizeof(float) * N * nin, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dt, target, sizeof(float) * N * S, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dl, label, sizeof(float) * N, hipMemcpyHostToDevice) != hipSuccess) {
-        cleanup();
-        return vfps_impl::fail(VFPS_ERR_HIP, "vfps_mlp_train: upload failed");
-    }
+    float* dx = (float*)m->data;
+    float* dt = dx + fx;
+    float* dl = dt + ft;
+    uint32_t* didx = (uint32_t*)(dl + N);
+    float* losses = (float*)(didx + N);
+    VFPS_HIP(hipMemcpyAsync(dx, x, sizeof(float) * fx, hipMemcpyHostToDevice, st));
+    VFPS_HIP(hipMemcpyAsync(dt, target, sizeof(float) * ft, hipMemcpyHostToDevice, st));
+    VFPS_HIP(hipMemcpyAsync(dl, label, sizeof(float) * N, hipMemcpyHostToDevice, st));
     std::vector<uint32_t> perm(N);
     std::vector<float> lh(nb);
     uint64_t s = seed;
+    int rc = VFPS_OK;
     for (uint32_t e = 0; e < epochs && rc == VFPS_OK; e++) {
         std::iota(perm.begin(), perm.end(), 0u);
         for (uint32_t i = N - 1; i > 0; i--) {
             std::swap(perm[i], perm[splitmix(s) % (i + 1)]);
         }
-        hipMemcpyAsync(didx, perm.data(), sizeof(uint32_t) * N,
-                       hipMemcpyHostToDevice, st);
+        VFPS_HIP(hipMemcpyAsync(didx, perm.data(), sizeof(uint32_t) * N,
+                                hipMemcpyHostToDevice, st));
         for (uint32_t bi = 0; bi < nb && rc == VFPS_OK; bi++) {
             const uint32_t b0 = bi * batch;
             const uint32_t B = std::min(batch, N - b0);
+            if (m->fused()) {
+                const AdamArgs a = next_adam(m, lr, 0.9f, 0.999f, 1e-8f);
+                rc = fused_step(m, {dx, dt, dl, didx + b0, B}, label_weight,
+                                losses + bi, &a);
+                continue;
+            }
             hipLaunchKernelGGL(gather_kernel, dim3(64), dim3(256), 0, st, dx,
                                didx + b0, B, nin, m->x);
             hipLaunchKernelGGL(gather_kernel, dim3(64), dim3(256), 0, st, dt,
                                didx + b0, B, S, m->tgt);
             hipLaunchKernelGGL(gather_kernel, dim3(64), dim3(256), 0, st, dl,
                                didx + b0, B, 1u, m->lab);
-            rc = upload_inputs(m, nullptr, B, false);
-            if (rc == VFPS_OK) rc = loss_and_grad(m, B, label_weight);
+            rc = loss_and_grad(m, B, label_weight, losses + bi);
             if (rc == VFPS_OK) rc = adam(m, lr, 0.9f, 0.999f, 1e-8f);
-            if (rc == VFPS_OK) {
-                hipMemcpyAsync(losses + bi, m->loss, sizeof(float),
-                               hipMemcpyDeviceToDevice, st);
-            }
         }
         if (rc == VFPS_OK && epoch_loss) {
-            hipMemcpyAsync(lh.data(), losses, sizeof(float) * nb,
-                           hipMemcpyDeviceToHost, st);
-            hipStreamSynchronize(st);
+            VFPS_HIP(hipMemcpyAsync(lh.data(), losses, sizeof(float) * nb,
+                                    hipMemcpyDeviceToHost, st));
+        }
+        // (the next epoch shuffles perm again)
+        VFPS_HIP(hipStreamSynchronize(st));
+        if (rc == VFPS_OK && epoch_loss) {
             double a = 0;
             for (float v : lh) a += v;
             epoch_loss[e] = (float)(a / nb);
         }
     }
-    hipStreamSynchronize(st);
-    cleanup();
-    if (rc != VFPS_OK) return rc;
-    VFPS_HIP(hipGetLastError());
-    return VFPS_OK;
+    VFPS_HIP(hipStreamSynchronize(st));
+    return rc;
     VFPS_TRY_END
 }
 

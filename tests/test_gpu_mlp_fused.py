@@ -1,0 +1,81 @@
+"""The two-kernel form of the network at the edges of its tiles (16 samples,
+16 columns, 32-deep products), the layer-by-layer form of networks that do
+not fit it, and the update fused into the gradients."""
+import numpy as np
+import pytest
+
+from oracle import mlp_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def V():
+    import inovesa_amd as V
+    return V
+
+
+def _rel(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+def _data(B, dims, seed=1):
+    rng = np.random.default_rng(seed)
+    return (rng.uniform(-1, 1, (B, dims[0])).astype(np.float32),
+            rng.standard_normal((B, dims[-1] - 1)).astype(np.float32),
+            (rng.random(B) > 0.5).astype(np.float32))
+
+
+# the last three do not fit (activations, layers): layer by layer
+NETS = [(3, 2), (1, 5, 2), (3, 48, 33, 9), (33, 100, 17), (40, 256, 300, 65),
+        (3, 31, 32, 33, 16, 17, 64, 65, 3), (3, 1200, 1100, 9),
+        (3, 1600, 5), (3, 8, 8, 8, 8, 8, 8, 8, 8, 4)]
+
+
+@pytest.mark.parametrize("dims", NETS)
+@pytest.mark.parametrize("B", [1, 16, 33])
+def test_network_edges_match_oracle(V, dims, B):
+    # bounds of test_gpu_mlp.py: one BF16 rounding of an activation that
+    # falls to the other side is 2^-9 of it
+    net = V.MLP(dims, max_batch=48, seed=3)
+    x, t, lab = _data(B, dims, seed=B)
+    layers = mo.split(net.params(), dims)
+    ref, _ = mo.forward(layers, x, emulate=True)
+    assert _rel(net.forward(x), ref) <= 2e-3
+    loss = net.loss_grad(x, t, lab, 0.5)
+    rloss, rg = mo.loss_and_grads(layers, x, t, lab, 0.5, emulate=True)
+    assert loss == pytest.approx(rloss, rel=1e-3)
+    for (dW, db), (rW, rb) in zip(net.layers(net.grads()), rg):
+        assert _rel(dW, rW) <= 2e-2
+        assert _rel(db, rb) <= 2e-2
+
+
+def test_forward_beyond_the_staging(V):
+    dims = (3, 64, 9)
+    net = V.MLP(dims, max_batch=3000, seed=5)
+    x, _, _ = _data(2501, dims)
+    y = net.forward(x)
+    for k in (0, 1023, 1024, 2500):
+        np.testing.assert_array_equal(y[k:k + 1], net.forward(x[k:k + 1]))
+
+
+@pytest.mark.parametrize("dims", [(3, 48, 33, 9), (3, 1200, 1100, 9)])
+def test_train_is_gradients_and_adam(V, dims):
+    """One update over the whole set, fused, against loss_grad + adam_step.
+    The sums run over the samples in another order: gradients differ by a
+    few 2^-24 of their terms, and Adam's first update is lr g / (|g| + eps),
+    which only differs where |g| is itself of that size."""
+    x, t, lab = _data(45, dims, seed=8)
+    a = V.MLP(dims, max_batch=48, seed=6)
+    b = V.MLP(dims, max_batch=48, seed=6)
+    loss = a.train(x, t, lab, batch=45, epochs=1, lr=1e-3, seed=4)
+    assert loss[0] == pytest.approx(b.loss_grad(x, t, lab), rel=1e-6)
+    assert _rel(a.grads(), b.grads()) <= 1e-5
+    b.adam_step(lr=1e-3)
+    d = np.abs(a.params() - b.params())
+    assert d.max() <= 2.1e-3 and d.mean() <= 1e-5
+    # the padded copies follow the parameters
+    c = V.MLP(dims, max_batch=48, seed=1)
+    c.set_params(a.params())
+    np.testing.assert_array_equal(a.forward(x), c.forward(x))
