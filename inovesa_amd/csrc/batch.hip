@@ -47,7 +47,8 @@ struct Group {
 // workgroup per member, ahead of the step kernels of the same step.
 struct FieldLaunch {
     bool wake = false, csr = false;
-    uint32_t ninst = 0, Mmax = 0;
+    uint32_t ninst = 0;
+    size_t lds = 0;       // the most any member's transform needs
     FieldParams* params_d = nullptr;
 };
 
@@ -102,23 +103,23 @@ int build_fields(vfps_batch* b)
     for (int pair = 0; pair < 4; pair++) {
         const bool wake = (pair & 1) != 0, csr = (pair & 2) != 0;
         std::vector<FieldParams> ps;
-        uint32_t Mmax = 0;
+        size_t lds = 0;
         for (const vfps_step* s : b->members) {
             if (s->direct || (s->desc.use_wake != 0) != wake ||
                 (s->desc.use_csr != 0) != csr) {
                 continue;
             }
             ps.push_back(s->fparams_h);
-            Mmax = std::max(Mmax, s->M);
+            lds = std::max(lds, field_lds_bytes(s->M));
         }
         if (ps.empty()) continue;
-        VFPS_CHECK_ARG(field_lds_bytes(Mmax) <= b->dev->lds_max,
+        VFPS_CHECK_ARG(lds <= b->dev->lds_max,
                        "batch: an FFT length exceeds the LDS of one CU");
         FieldLaunch f;
         f.wake = wake;
         f.csr = csr;
         f.ninst = (uint32_t)ps.size();
-        f.Mmax = Mmax;
+        f.lds = lds;
         b->fields.push_back(f);
         FieldLaunch& fl = b->fields.back();
         VFPS_HIP(hipMalloc(&fl.params_d, sizeof(FieldParams) * ps.size()));
@@ -244,7 +245,7 @@ int launch_step(vfps_batch* b, uint32_t parity)
     hipStream_t main = b->dev->stream;
     // the FFT-wake members' wake potentials, CSR powers and step counts
     for (const auto& f : b->fields) {
-        int rc = launch_fields(f.wake, f.csr, f.params_d, f.ninst, f.Mmax,
+        int rc = launch_fields(f.wake, f.csr, f.params_d, f.ninst, f.lds,
                                parity, main);
         if (rc != VFPS_OK) return rc;
     }

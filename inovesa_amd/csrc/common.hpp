@@ -150,7 +150,8 @@ struct vfps_field {
     float* wake = nullptr;       // [nb][n]
     float* wake_padded = nullptr;  // [nmax] unscaled C2R output
     float* padded = nullptr;     // [nmax]
-    double2* tw_m = nullptr;     // e^{-2 pi i t/M}, t < M (M = nmax/2)
+    double2* tw_m = nullptr;     // e^{-2 pi i t/M}, t < M (M = nmax/2), or
+                                 // the chirp table
     double2* tw_n = nullptr;     // e^{-2 pi i k/nmax}, k < M
     float* csr_renorm = nullptr; // [nmax]
     float* spectrum = nullptr;   // [nb][nmax]

@@ -4,7 +4,9 @@
 // of length M (even samples in the real parts, odd samples in the
 // imaginary parts).  The complex FFT is a Stockham autosort with radix-8
 // passes (and one radix-4 or radix-2 pass), in place in one LDS buffer
-// with a spare slot after every 8 elements, with no bit reversal.
+// with a spare slot after every 8 elements, with no bit reversal.  A length
+// M that is no power of two goes through two transforms of a power-of-two
+// length (Bluestein's chirp algorithm).
 //
 // The butterflies run in FP64.  Inputs and outputs stay FP32 exactly where
 // the reference's arrays are float (profile, spectrum F, W = Z F, wake
@@ -47,6 +49,25 @@ __host__ __device__ constexpr uint32_t fft_slots(uint32_t M)
     return M + M / 8;
 }
 
+// Twiddles exp(-2 pi i t / P), t < P/2, of a transform of P elements: the
+// half table itself, or, where it would not fit the LDS beside the data, two
+// factors exp(-2 pi i (t mod 64) / P) and exp(-2 pi i 64 (t / 64) / P) (one
+// more FP64 product, 1e-16).
+struct TwTable {
+    const double2* tw;
+    __device__ __forceinline__ double2 operator()(uint32_t t) const
+    {
+        return tw[t];
+    }
+};
+struct TwFactors {
+    const double2* lo;  // 64 entries, then P/128 of the second factor
+    __device__ __forceinline__ double2 operator()(uint32_t t) const
+    {
+        return cmul(lo[64u + (t >> 6)], lo[t & 63u]);
+    }
+};
+
 // The butterflies' DFT of 4 (forward exp(-i..), INV exp(+i..)), in place
 template <bool INV>
 __device__ __forceinline__ void dft4(double2& c0, double2& c1, double2& c2,
@@ -68,15 +89,15 @@ __device__ __forceinline__ void dft4(double2& c0, double2& c1, double2& c2,
 // (j < M/R) of the pass with Ns = 2^lgNs takes inputs j + k M/R, scales
 // input k by w^(k jm M/(Ns R)) (jm = j mod Ns, w = exp(-2 pi i / M)), and
 // writes output q to (j - jm) R + jm + q Ns.  The twiddle w^(jm M/(Ns R))
-// comes from the half table tw (its index is below M/2), its powers by
-// complex products in FP64.
-template <bool INV, int R>
+// comes from tw (its index is below M/2), its powers by complex products in
+// FP64.  MAXM: the longest M.
+template <bool INV, int R, uint32_t MAXM, typename Tw>
 __device__ __forceinline__ void fft_pass(double2* a, uint32_t lgM,
-                                         uint32_t lgNs, const double2* tw)
+                                         uint32_t lgNs, const Tw& tw)
 {
     constexpr int LGR = R == 8 ? 3 : (R == 4 ? 2 : 1);
-    // butterflies per thread: M/R <= FFT_MAX_M/R over FFT_THREADS threads
-    constexpr int NB = (int)((FFT_MAX_M / R + FFT_THREADS - 1) / FFT_THREADS);
+    // butterflies per thread: M/R <= MAXM/R over FFT_THREADS threads
+    constexpr int NB = (int)((MAXM / R + FFT_THREADS - 1) / FFT_THREADS);
     const uint32_t nbf = 1u << (lgM - LGR);
     const uint32_t Ns = 1u << lgNs;
     const uint32_t lgts = lgM - lgNs - LGR;
@@ -101,7 +122,7 @@ __device__ __forceinline__ void fft_pass(double2* a, uint32_t lgM,
         double2* x = v[b];
         const uint32_t jm = j & (Ns - 1u);
         if (jm != 0u) {
-            double2 w1 = tw[jm << lgts];
+            double2 w1 = tw(jm << lgts);
             if (INV) {
                 w1 = cconj(w1);
             }
@@ -162,62 +183,95 @@ __device__ __forceinline__ void fft_pass(double2* a, uint32_t lgM,
     __syncthreads();
 }
 
-// Complex FFT of length M (power of two, 2 <= M <= FFT_MAX_M) in place in
+// Complex FFT of length M (power of two, 2 <= M <= MAXM) in place in
 // the slots (fft_slot) of the LDS buffer `a`: Stockham autosort, radix-8
 // passes with a radix-4 or radix-2 pass where log2(M) is not a multiple of
-// 3, so the output is in natural order without a bit reversal.  tw: LDS
-// half table exp(-2 pi i t / M), t < M/2.  Forward uses exp(-i..), INV
-// exp(+i..); unnormalised.  Must be called by the whole workgroup of
-// FFT_THREADS threads.
-template <bool INV>
-__device__ void fft_lds(double2* a, uint32_t M, const double2* tw)
+// 3, so the output is in natural order without a bit reversal.  Forward uses
+// exp(-i..), INV exp(+i..); unnormalised.  Must be called by the whole
+// workgroup of FFT_THREADS threads.
+template <bool INV, uint32_t MAXM = FFT_MAX_M, typename Tw>
+__device__ __forceinline__ void fft_lds(double2* a, uint32_t M, const Tw& tw)
 {
     const uint32_t lgM = 31u - (uint32_t)__clz(M);
     uint32_t lgNs = 0;
     while (lgNs < lgM) {
         const uint32_t left = lgM - lgNs;
         if (left >= 3u && (left % 3u == 0u || left > 4u)) {
-            fft_pass<INV, 8>(a, lgM, lgNs, tw);
+            fft_pass<INV, 8, MAXM>(a, lgM, lgNs, tw);
             lgNs += 3;
         } else if (left >= 2u) {
-            fft_pass<INV, 4>(a, lgM, lgNs, tw);
+            fft_pass<INV, 4, MAXM>(a, lgM, lgNs, tw);
             lgNs += 2;
         } else {
-            fft_pass<INV, 2>(a, lgM, lgNs, tw);
+            fft_pass<INV, 2, MAXM>(a, lgM, lgNs, tw);
             lgNs += 1;
         }
     }
 }
 
-// Complex DFT of length M (any M) in place in the LDS buffer `a`, by the
-// direct sum out[k] = sum_j a[j] w^(j k) in FP64, for the lengths the
-// radix-4/2 FFT does not take (the reference's FFTW plans any length, e.g.
-// nmax = 768 = 3 * 256 when RoundPadding is off).  tmp: LDS scratch of M
-// entries; tw: the full table exp(-2 pi i t / M), t < M (global memory: the
-// powers of w are picked by index, (j k) mod M, so no rounding accumulates
-// across the sum).  Forward uses exp(-i..), INV exp(+i..); unnormalised.
-// Must be called by the whole workgroup.
-template <bool INV>
-__device__ void dft_lds(double2* a, double2* tmp, uint32_t M,
-                        const double2* __restrict__ tw)
+// Length of the two transforms behind a DFT of M elements, M no power of
+// two: the next power of two from 2 M - 1 on.
+__host__ __device__ __forceinline__ uint32_t chirp_len(uint32_t M)
 {
-    for (uint32_t i = threadIdx.x; i < M; i += FFT_THREADS) {
-        tmp[i] = a[i];
+    uint32_t P = 8;
+    while (P < 2u * M - 1u) P <<= 1;
+    return P;
+}
+// longest of them
+constexpr uint32_t CHIRP_MAX_P = 2 * FFT_MAX_M;
+// entries of the twiddle factors of a transform of P elements
+__host__ __device__ __forceinline__ uint32_t chirp_tw(uint32_t P)
+{
+    return 64u + (P / 2u + 63u) / 64u;
+}
+// Table of a chirp DFT: the chirp c[j] = exp(-pi i j^2 / M) (M entries),
+// the transform of the filter conj(c[|d|]) over P (P entries, divided by P),
+// the twiddle factors of TwFactors.
+__host__ __device__ __forceinline__ uint32_t chirp_table(uint32_t M)
+{
+    const uint32_t P = chirp_len(M);
+    return M + P + chirp_tw(P);
+}
+
+// Complex DFT of length M (no power of two; M <= FFT_MAX_M) in place in the
+// slots of the LDS buffer `a` (chirp_len(M) elements), for the lengths the
+// FFT does not take (the reference's FFTW plans any length, e.g. nmax = 768 =
+// 3 * 256 when RoundPadding is off).  With j k = (j^2 + k^2 - (k - j)^2) / 2,
+//   X_k = c_k sum_j (x_j c_j) conj(c_{k-j}):
+// a convolution, made by an FFT of P >= 2 M - 1 elements, the product with
+// the filter's transform and the inverse FFT, all FP64.  Wake potential and
+// CSR spectra of two bunches with M = 1500: 119 us a call, with the direct
+// sums of M^2 terms it was 1884.
+// The inverse DFT is the conjugate of the DFT of the conjugate.  tw: LDS
+// copy of the table's twiddle factors; tab: the table in global memory (it
+// stays in L2).  Forward uses exp(-i..), INV exp(+i..); unnormalised.
+// Must be called by the whole workgroup of FFT_THREADS threads.
+template <bool INV>
+__device__ void dft_lds(double2* a, uint32_t M, const double2* tw,
+                        const double2* __restrict__ tab)
+{
+    const uint32_t P = chirp_len(M);
+    const double2* filt = tab + M;
+    for (uint32_t j = threadIdx.x; j < P; j += FFT_THREADS) {
+        double2 v = make_double2(0.0, 0.0);
+        if (j < M) {
+            v = a[fft_slot(j)];
+            if (INV) v = cconj(v);
+            v = cmul(v, tab[j]);
+        }
+        a[fft_slot(j)] = v;
     }
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < M; k += FFT_THREADS) {
-        double re = 0.0, im = 0.0;
-        uint32_t t = 0;
-        for (uint32_t j = 0; j < M; j++) {
-            const double2 x = tmp[j];
-            const double2 w = tw[t];
-            const double wy = INV ? -w.y : w.y;
-            re += x.x * w.x - x.y * wy;
-            im += x.x * wy + x.y * w.x;
-            t += k;
-            if (t >= M) t -= M;
-        }
-        a[k] = make_double2(re, im);
+    fft_lds<false, CHIRP_MAX_P>(a, P, TwFactors{tw});
+    for (uint32_t j = threadIdx.x; j < P; j += FFT_THREADS) {
+        a[fft_slot(j)] = cmul(a[fft_slot(j)], filt[j]);
+    }
+    __syncthreads();
+    fft_lds<true, CHIRP_MAX_P>(a, P, TwFactors{tw});
+    for (uint32_t j = threadIdx.x; j < M; j += FFT_THREADS) {
+        double2 v = cmul(a[fft_slot(j)], tab[j]);
+        if (INV) v = cconj(v);
+        a[fft_slot(j)] = v;
     }
     __syncthreads();
 }

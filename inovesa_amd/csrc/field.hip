@@ -26,7 +26,11 @@ field_kernel(FieldParams p)
 
 size_t field_lds_bytes(uint32_t M)
 {
-    return sizeof(double2) * (fft_pow2(M) ? fft_slots(M) + M / 2 : 2 * M);
+    if (fft_pow2(M)) {
+        return sizeof(double2) * (fft_slots(M) + M / 2);
+    }
+    const uint32_t P = chirp_len(M);
+    return sizeof(double2) * (fft_slots(P) + chirp_tw(P));
 }
 
 int launch_field(const FieldParams& p, bool wake, bool csr, uint32_t blocks,
@@ -64,19 +68,73 @@ int field_set_lds_limit(size_t bytes)
     return VFPS_OK;
 }
 
-// twiddle tables: e^{-2 pi i t/M} (t < M) and e^{-2 pi i k/N} (k < M),
-// in double
+// in-place radix-2 FFT (host, exp(-i..)) of a power-of-two length
+static void fft_host(std::vector<double2>& a)
+{
+    const size_t n = a.size();
+    for (size_t i = 1, j = 0; i < n; i++) {
+        size_t bit = n >> 1;
+        for (; j & bit; bit >>= 1) j ^= bit;
+        j ^= bit;
+        if (i < j) std::swap(a[i], a[j]);
+    }
+    std::vector<double2> w(n / 2);
+    for (size_t t = 0; t < n / 2; t++) {
+        sincos(-2.0 * M_PI * (double)t / (double)n, &w[t].y, &w[t].x);
+    }
+    for (size_t h = 1; h < n; h <<= 1) {
+        for (size_t i = 0; i < n; i += 2 * h) {
+            for (size_t k = 0; k < h; k++) {
+                const double2 c = w[k * (n / (2 * h))], u = a[i + k],
+                              v = a[i + k + h];
+                const double2 x = make_double2(v.x * c.x - v.y * c.y,
+                                               v.x * c.y + v.y * c.x);
+                a[i + k] = make_double2(u.x + x.x, u.y + x.y);
+                a[i + k + h] = make_double2(u.x - x.x, u.y - x.y);
+            }
+        }
+    }
+}
+
+// the chirp table of dft_lds (fft.hpp)
+static std::vector<double2> chirp_tables(uint32_t M)
+{
+    const uint32_t P = chirp_len(M);
+    std::vector<double2> t(chirp_table(M)), b(P, make_double2(0.0, 0.0));
+    for (uint32_t j = 0; j < M; j++) {
+        // j^2 modulo 2 M: the angle stays small and exact
+        const uint64_t q = (uint64_t)j * j % (2ull * M);
+        sincos(-M_PI * (double)q / (double)M, &t[j].y, &t[j].x);
+        b[j] = make_double2(t[j].x, -t[j].y);
+        if (j) b[P - j] = b[j];
+    }
+    fft_host(b);
+    for (uint32_t k = 0; k < P; k++) {
+        t[M + k] = make_double2(b[k].x / P, b[k].y / P);
+    }
+    double2* f = t.data() + M + P;
+    for (uint32_t k = 0; k < chirp_tw(P); k++) {
+        const uint64_t e = k < 64u ? k : 64ull * (k - 64u);
+        sincos(-2.0 * M_PI * (double)e / (double)P, &f[k].y, &f[k].x);
+    }
+    return t;
+}
+
 void make_twiddles(uint32_t M, std::vector<double2>& tw_m,
                    std::vector<double2>& tw_n)
 {
     const double pi = 3.141592653589793238462643383279502884;
-    tw_m.resize(M);
+    if (fft_pow2(M)) {
+        tw_m.resize(M);
+        for (uint32_t t = 0; t < M; t++) {
+            sincos(-2.0 * pi * (double)t / (double)M, &tw_m[t].y, &tw_m[t].x);
+        }
+    } else {
+        tw_m = chirp_tables(M);
+    }
     tw_n.resize(M);
     for (uint32_t t = 0; t < M; t++) {
-        double a = -2.0 * pi * (double)t / (double)M;
-        tw_m[t] = make_double2(std::cos(a), std::sin(a));
-        double b = -2.0 * pi * (double)t / (2.0 * (double)M);
-        tw_n[t] = make_double2(std::cos(b), std::sin(b));
+        sincos(-2.0 * pi * (double)t / (2.0 * (double)M), &tw_n[t].y, &tw_n[t].x);
     }
 }
 
@@ -313,7 +371,7 @@ int vfps_field_create(vfps_mesh* ps, vfps_impedance* z,
     e = e ? e : hipMalloc(&f->wake, sizeof(float) * nb * n);
     e = e ? e : hipMalloc(&f->padded, sizeof(float) * nmax);
     e = e ? e : hipMalloc(&f->wake_padded, sizeof(float) * nmax);
-    e = e ? e : hipMalloc(&f->tw_m, sizeof(double2) * M);
+    e = e ? e : hipMalloc(&f->tw_m, sizeof(double2) * twm.size());
     e = e ? e : hipMalloc(&f->tw_n, sizeof(double2) * M);
     e = e ? e : hipMalloc(&f->csr_renorm, sizeof(float) * nmax);
     e = e ? e : hipMalloc(&f->spectrum, sizeof(float) * nb * nmax);
@@ -328,7 +386,7 @@ int vfps_field_create(vfps_mesh* ps, vfps_impedance* z,
     hipMemsetAsync(f->wake, 0, sizeof(float) * nb * n, st);
     hipMemsetAsync(f->padded, 0, sizeof(float) * nmax, st);
     hipMemsetAsync(f->wake_padded, 0, sizeof(float) * nmax, st);
-    hipMemcpyAsync(f->tw_m, twm.data(), sizeof(double2) * M,
+    hipMemcpyAsync(f->tw_m, twm.data(), sizeof(double2) * twm.size(),
                    hipMemcpyHostToDevice, st);
     hipMemcpyAsync(f->tw_n, twn.data(), sizeof(double2) * M,
                    hipMemcpyHostToDevice, st);

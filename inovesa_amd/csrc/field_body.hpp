@@ -18,7 +18,8 @@ namespace vfps_impl {
 // holds them as float, and the float arithmetic on them follows the
 // reference.  lds: field_lds_bytes(M): fft_slots(M) + M/2 double2 (data
 // with a spare slot after every 8 elements, twiddle half table) for a
-// power-of-two M, else 2 M (data, DFT scratch).  Runs with FFT_THREADS
+// power-of-two M, else those of the chirp transform's length and its twiddle
+// factors.  Runs with FFT_THREADS
 // threads (the loops step by that constant: blockDim would be a load from
 // the dispatch packet, waited for after every barrier).
 constexpr int FIELD_PAIRS = 3;  // (k, M-k) pairs per thread: M <= 4096
@@ -49,16 +50,14 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     VFPS_FSTAMP(0);
     const uint32_t M = p.M;
     // power-of-two M: radix-8 FFT with the half twiddle table in LDS;
-    // other M: direct DFT with M entries of LDS scratch
+    // other M: chirp DFT
     const bool pow2 = fft_pow2(M);
-    // element i of the transform buffer: a spare slot after every 8
-    // elements for the FFT (fft_slot), dense for the DFT
-    const uint32_t psh = pow2 ? 3u : 31u;
-    auto slot = [psh](uint32_t i) { return i + (i >> psh); };
+    const uint32_t P = pow2 ? M : chirp_len(M);
+    auto slot = [](uint32_t i) { return fft_slot(i); };
     // real sample i of the padded array: element i/2, real part for even i
     auto rslot = [&](uint32_t i) { return 2u * slot(i >> 1) + (i & 1u); };
     double2* A = lds;
-    double2* twl = lds + (pow2 ? fft_slots(M) : M);
+    double2* twl = lds + fft_slots(P);
     double* Ad = reinterpret_cast<double*>(A);
     // one bunch (the step's case): its profile and Simpson weights are
     // fetched first, with the tables and the step counter below, so that
@@ -89,9 +88,11 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     for (uint32_t i = threadIdx.x; i < M; i += FFT_THREADS) {
         A[slot(i)] = make_double2(0.0, 0.0);
     }
-    if ((WAKE || CSR) && pow2) {
-        for (uint32_t i = threadIdx.x; i < M / 2; i += FFT_THREADS) {
-            twl[i] = p.tw_m[i];
+    if (WAKE || CSR) {
+        const uint32_t ntw = pow2 ? M / 2 : chirp_tw(P);
+        const double2* src = pow2 ? p.tw_m : p.tw_m + M + P;
+        for (uint32_t i = threadIdx.x; i < ntw; i += FFT_THREADS) {
+            twl[i] = src[i];
         }
     }
     // this thread's (k, M-k) pairs: tables fetched before the transform so
@@ -196,9 +197,9 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     }
     VFPS_FSTAMP(1);
     if (pow2) {
-        fft_lds<false>(A, M, twl);
+        fft_lds<false>(A, M, TwTable{twl});
     } else {
-        dft_lds<false>(A, twl, M, p.tw_m);
+        dft_lds<false>(A, M, twl, p.tw_m);
     }
     VFPS_FSTAMP(2);
     double2* Zf = A;
@@ -288,9 +289,9 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     __syncthreads();
     VFPS_FSTAMP(3);
     if (pow2) {
-        fft_lds<true>(A, M, twl);
+        fft_lds<true>(A, M, TwTable{twl});
     } else {
-        dft_lds<true>(A, twl, M, p.tw_m);
+        dft_lds<true>(A, M, twl, p.tw_m);
     }
     VFPS_FSTAMP(4);
     const double* yd = reinterpret_cast<const double*>(A);

@@ -265,10 +265,9 @@ static const void* fields_fn(bool one)
 }
 
 int launch_fields(bool wake, bool csr, const FieldParams* params_d,
-                  uint32_t ninst, uint32_t Mmax, uint32_t parity,
+                  uint32_t ninst, size_t lds, uint32_t parity,
                   hipStream_t st, const FieldParams* params_h)
 {
-    const size_t lds = field_lds_bytes(Mmax);
     const bool one = ninst == 1 && params_h;
     const void* fn;
     if (wake && csr) {
@@ -368,7 +367,7 @@ static int step_launch_fused(vfps_step* s, uint32_t parity, hipStream_t st)
 {
     if (!s->direct) {
         int rc = launch_fields(s->desc.use_wake != 0, s->desc.use_csr != 0,
-                               s->fparams_d, 1, s->M, parity, st,
+                               s->fparams_d, 1, field_lds_bytes(s->M), parity, st,
                                &s->fparams_h);
         if (rc != VFPS_OK) return rc;
     }
@@ -401,7 +400,7 @@ static int step_launch_maps(vfps_step* s, uint32_t parity)
         return step_launch_fused(s, parity, st);
     }
     // per-map path, the loop body of src/main.cpp:948-1053
-    int rc = launch_fields(wake, csr, s->fparams_d, 1, s->M, 0, st,
+    int rc = launch_fields(wake, csr, s->fparams_d, 1, field_lds_bytes(s->M), 0, st,
                            &s->fparams_h);
     if (rc != VFPS_OK) return rc;
     vfps_mesh *t1 = s->t1, *t2 = s->t2, *t3 = s->t3;
@@ -565,7 +564,7 @@ static int step_upload_desc(vfps_step* s)
         if (!s->wfield) {
             // CSR only: twiddles from a field-less table
             p.tw_m = s->csr_tw;
-            p.tw_n = s->csr_tw + s->M;
+            p.tw_n = s->csr_tw + s->csr_tw_m;
         }
     }
     s->fparams_h = p;
@@ -899,10 +898,11 @@ int vfps_step_create(vfps_dev* dev, const vfps_step_desc* desc,
         VFPS_HIP(hipMalloc(&s->csr_renorm, sizeof(float) * nmax));
         VFPS_HIP(hipMemcpy(s->csr_renorm, renorm.data(), sizeof(float) * nmax,
                            hipMemcpyHostToDevice));
-        VFPS_HIP(hipMalloc(&s->csr_tw, sizeof(double2) * 2 * s->M));
-        VFPS_HIP(hipMemcpy(s->csr_tw, twm.data(), sizeof(double2) * s->M,
+        s->csr_tw_m = twm.size();
+        VFPS_HIP(hipMalloc(&s->csr_tw, sizeof(double2) * (twm.size() + s->M)));
+        VFPS_HIP(hipMemcpy(s->csr_tw, twm.data(), sizeof(double2) * twm.size(),
                            hipMemcpyHostToDevice));
-        VFPS_HIP(hipMemcpy(s->csr_tw + s->M, twn.data(),
+        VFPS_HIP(hipMemcpy(s->csr_tw + s->csr_tw_m, twn.data(),
                            sizeof(double2) * s->M, hipMemcpyHostToDevice));
     }
     VFPS_HIP(hipMalloc(&s->filling, sizeof(double) * 2));
@@ -1392,7 +1392,8 @@ int vfps_step_timing(vfps_step* s, uint32_t nsteps, float* ms_wake,
             const uint32_t par = s->parity;
             hipEventRecord(e0, st);
             rc = launch_fields(s->desc.use_wake != 0, s->desc.use_csr != 0,
-                               s->fparams_d, 1, s->M, par, st, &s->fparams_h);
+                               s->fparams_d, 1, field_lds_bytes(s->M), par, st,
+                               &s->fparams_h);
             hipEventRecord(e1, st);
             if (rc == VFPS_OK) {
                 rc = launch_step_kernel(s->variant, s->inst_d, nullptr,

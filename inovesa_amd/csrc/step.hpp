@@ -107,11 +107,12 @@ void toeplitz_tables(uint32_t n, uint32_t M, const float2* Z,
                      const float2* Zc, const float* renorm, float fdelta,
                      std::vector<double>* g, std::vector<double>* h);
 
-// Field kernel over `ninst` instances (one workgroup each).  params_h:
+// Field kernel over `ninst` instances (one workgroup each), with the LDS
+// the longest of their transforms needs.  params_h:
 // the host copy of the parameters of a single instance, passed by value,
 // or null to read them from params_d.
 int launch_fields(bool wake, bool csr, const FieldParams* params_d,
-                  uint32_t ninst, uint32_t Mmax, uint32_t parity,
+                  uint32_t ninst, size_t lds, uint32_t parity,
                   hipStream_t st, const FieldParams* params_h = nullptr);
 // close a run: with close_csr, the last step's CSR power from the tiles'
 // shares (direct form; the next step's closing workgroup does this
@@ -142,6 +143,7 @@ struct vfps_step {
     vfps_impedance* zcsr = nullptr;
     float* csr_renorm = nullptr;
     double2* csr_tw = nullptr;
+    size_t csr_tw_m = 0;          // entries of the transform's table in it
     float csr_fdelta = 0;
     double* filling = nullptr;  // [2]
     uint32_t* counter = nullptr;    // [2] (ping-pong in the fused step)
