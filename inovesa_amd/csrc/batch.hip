@@ -68,6 +68,11 @@ struct vfps_batch {
     std::vector<vfps_step*> members;
     std::vector<Group> groups;
     std::vector<FieldLaunch> fields;
+    // every member's descriptor in batch order and where its profile starts
+    // in the concatenated ones; built when a run or a read-back first needs
+    // them
+    InstDesc* all_d = nullptr;
+    uint32_t* start_d = nullptr;
     bool merge = false;   // one launch per variant, workgroup size and form
                           // (LDS classes merged: every tile gets the largest
                           // tile's LDS)
@@ -93,6 +98,10 @@ void free_groups(vfps_batch* b)
 {
     for (auto& g : b->groups) group_free(g);
     b->groups.clear();
+    hipFree(b->all_d);
+    hipFree(b->start_d);
+    b->all_d = nullptr;
+    b->start_d = nullptr;
     for (auto& f : b->fields) hipFree(f.params_d);
     b->fields.clear();
 }
@@ -276,6 +285,63 @@ int launch_step(vfps_batch* b, uint32_t parity)
     return VFPS_OK;
 }
 
+// ---- results of all instances in one transfer -----------------------------------
+// A copy per instance costs about 10 us on the host, whatever its size: 64
+// instances of 128^2 spent 1.9 ms a call on their profiles, CSR histories and
+// error flags beside 2.0 ms for 128 steps.  A workgroup per instance writes
+// them into the device handle's pinned buffer instead: one launch and one
+// wait for all; what is longer than the buffer goes through it in parts.
+
+// the current profile of instances i0 + blockIdx.x, each at its start
+__global__ void __launch_bounds__(256)
+batch_profiles_kernel(const InstDesc* __restrict__ descs,
+                      const uint32_t* __restrict__ start, uint32_t i0,
+                      uint32_t parity, float* __restrict__ out)
+{
+    const uint32_t i = i0 + blockIdx.x;
+    const float* src = descs[i].proj[parity];
+    float* dst = out + (start[i] - start[i0]);
+    for (uint32_t x = threadIdx.x; x < descs[i].n; x += 256u) {
+        dst[x] = src[x];
+    }
+}
+
+// recorded CSR power [first, first + count) of instances i0 + blockIdx.y
+__global__ void __launch_bounds__(256)
+batch_csr_kernel(const InstDesc* __restrict__ descs, uint32_t i0,
+                 uint32_t first, uint32_t count, float* __restrict__ out)
+{
+    const float* src = descs[i0 + blockIdx.y].csr_hist + first;
+    float* dst = out + (size_t)blockIdx.y * count;
+    for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < count;
+         t += gridDim.x * 256u) {
+        dst[t] = src[t];
+    }
+}
+
+int ensure_all(vfps_batch* b)
+{
+    if (b->all_d) return VFPS_OK;
+    const size_t k = b->members.size();
+    std::vector<InstDesc> descs(k);
+    std::vector<uint32_t> start(k);
+    uint32_t o = 0;
+    for (size_t i = 0; i < k; i++) {
+        descs[i] = b->members[i]->inst_h;
+        start[i] = o;
+        o += descs[i].n;
+    }
+    VFPS_HIP(hipMalloc(&b->start_d, sizeof(uint32_t) * k));
+    VFPS_HIP(hipMemcpy(b->start_d, start.data(), sizeof(uint32_t) * k,
+                       hipMemcpyHostToDevice));
+    InstDesc* d = nullptr;
+    VFPS_HIP(hipMalloc(&d, sizeof(InstDesc) * k));
+    b->all_d = d;
+    VFPS_HIP(hipMemcpy(d, descs.data(), sizeof(InstDesc) * k,
+                       hipMemcpyHostToDevice));
+    return VFPS_OK;
+}
+
 // longest captured run; a run of nsteps replays it nsteps / BATCH_GRAPH
 // times, then one captured run of the remaining steps
 constexpr uint32_t BATCH_GRAPH = 64;
@@ -430,7 +496,8 @@ int vfps_batch_run(vfps_batch* b, uint32_t nsteps)
     VFPS_CHECK_ARG(b, "vfps_batch_run: NULL batch");
     hipStream_t st = b->dev->stream;
     uint32_t left = nsteps;
-    int rc;
+    int rc = ensure_all(b);
+    if (rc != VFPS_OK) return rc;
     // host launches when the members ask for them (no_graph)
     const bool host = !b->members.empty() && b->members[0]->desc.no_graph;
     while (host && left > 0) {
@@ -448,25 +515,21 @@ int vfps_batch_run(vfps_batch* b, uint32_t nsteps)
         left -= k;
         b->parity ^= (k & 1u);
     }
-    if (nsteps > 0) {
-        for (auto& g : b->groups) {
-            // (the FFT form's field kernel has recorded each step's power)
-            if (!g.variant.direct) continue;
-            rc = launch_step_finalize(g.descs_d, (uint32_t)g.members.size(),
-                                      b->parity, st);
-            if (rc != VFPS_OK) return rc;
-        }
-    }
-    // every member's error flag comes back in the same stream: one wait
-    for (auto* s : b->members) {
-        VFPS_HIP(hipMemcpyAsync(s->err_h, s->err, sizeof(uint32_t),
-                                hipMemcpyDeviceToHost, st));
+    // the last step's CSR powers (the FFT form's field kernel has recorded
+    // its own) and every member's error flag, in one launch
+    static_assert(DEV_STAGE_BYTES >= sizeof(uint32_t) * 0xFFFFu,
+                  "an error flag per instance");
+    DevStage stage(b->dev);
+    uint32_t* err = stage.get<uint32_t>();
+    if (!err) return fail(VFPS_ERR_NOMEM, "batch: pinned memory");
+    if ((rc = launch_step_finalize(b->all_d, (uint32_t)b->members.size(),
+                                   b->parity, st, err, nsteps > 0)) != VFPS_OK) {
+        return rc;
     }
     VFPS_HIP(hipStreamSynchronize(st));
     sync_parity(b);
-    for (auto* s : b->members) {
-        const uint32_t err = *s->err_h;
-        if (err) {
+    for (size_t i = 0; i < b->members.size(); i++) {
+        if (err[i]) {
             return fail(VFPS_ERR_INVALID, "batch step: a tap fell outside the "
                                           "halo rows (internal error)");
         }
@@ -523,38 +586,78 @@ int vfps_batch_get_mesh(vfps_batch* b, uint32_t inst, float* mesh,
 int vfps_batch_get_projections(vfps_batch* b, float* out)
 {
     VFPS_CHECK_ARG(b && out, "vfps_batch_get_projections: NULL argument");
+    VFPS_TRY_BEGIN
     hipStream_t st = b->dev->stream;
-    VFPS_HIP(hipStreamSynchronize(st));
     sync_parity(b);
-    size_t o = 0;
-    for (auto* s : b->members) {
-        const vfps_mesh* cur = (s->parity & 1u) ? s->t2 : s->t1;
-        VFPS_HIP(hipMemcpyAsync(out + o, cur->proj, sizeof(float) * s->desc.n,
-                                hipMemcpyDeviceToHost, st));
-        o += s->desc.n;
+    int rc = ensure_all(b);
+    if (rc != VFPS_OK) return rc;
+    constexpr size_t most = DEV_STAGE_BYTES / sizeof(float);
+    DevStage stage(b->dev);
+    float* buf = stage.get<float>();
+    if (!buf) return fail(VFPS_ERR_NOMEM, "batch: pinned memory");
+    const uint32_t k = (uint32_t)b->members.size();
+    for (uint32_t i = 0; i < k;) {
+        uint32_t e = i;
+        size_t words = 0;
+        while (e < k && words + b->members[e]->desc.n <= most) {
+            words += b->members[e++]->desc.n;
+        }
+        hipLaunchKernelGGL(batch_profiles_kernel, dim3(e - i), dim3(256), 0, st,
+                           b->all_d, b->start_d, i, b->parity & 1u, buf);
+        VFPS_HIP(hipGetLastError());
+        VFPS_HIP(hipStreamSynchronize(st));
+        std::copy(buf, buf + words, out);
+        out += words;
+        i = e;
     }
-    VFPS_HIP(hipStreamSynchronize(st));
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 int vfps_batch_get_csr_histories(vfps_batch* b, uint32_t first, uint32_t count,
                                  float* out)
 {
     VFPS_CHECK_ARG(b && out, "vfps_batch_get_csr_histories: NULL argument");
-    hipStream_t st = b->dev->stream;
-    VFPS_HIP(hipStreamSynchronize(st));
-    size_t o = 0;
     for (auto* s : b->members) {
-        VFPS_CHECK_ARG(s->csr_hist && first + count <= s->hist_cap,
+        VFPS_CHECK_ARG(s->csr_hist && (size_t)first + count <= s->hist_cap,
                        "vfps_batch_get_csr_histories: outside the recorded "
                        "capacity");
-        VFPS_HIP(hipMemcpyAsync(out + o, s->csr_hist + first,
-                                sizeof(float) * count, hipMemcpyDeviceToHost,
-                                st));
-        o += count;
     }
-    VFPS_HIP(hipStreamSynchronize(st));
+    if (count == 0) return VFPS_OK;
+    VFPS_TRY_BEGIN
+    hipStream_t st = b->dev->stream;
+    int rc = ensure_all(b);
+    if (rc != VFPS_OK) return rc;
+    const uint32_t k = (uint32_t)b->members.size();
+    const size_t most = DEV_STAGE_BYTES / sizeof(float) / count;
+    if (most == 0) {
+        // a history longer than the staging: a copy per instance
+        for (auto* s : b->members) {
+            VFPS_HIP(hipMemcpyAsync(out, s->csr_hist + first,
+                                    sizeof(float) * count,
+                                    hipMemcpyDeviceToHost, st));
+            out += count;
+        }
+        VFPS_HIP(hipStreamSynchronize(st));
+        return VFPS_OK;
+    }
+    DevStage stage(b->dev);
+    float* buf = stage.get<float>();
+    if (!buf) return fail(VFPS_ERR_NOMEM, "batch: pinned memory");
+    for (uint32_t i = 0; i < k;) {
+        const uint32_t m = (uint32_t)std::min<size_t>(most, k - i);
+        hipLaunchKernelGGL(batch_csr_kernel,
+                           dim3(std::min(ceil_div(count, 256u), 64u), m),
+                           dim3(256), 0, st, b->all_d, i, first, count,
+                           buf);
+        VFPS_HIP(hipGetLastError());
+        VFPS_HIP(hipStreamSynchronize(st));
+        std::copy(buf, buf + (size_t)m * count, out);
+        out += (size_t)m * count;
+        i += m;
+    }
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 int vfps_batch_info(vfps_batch* b, uint32_t* ninst, uint32_t* ngroups,

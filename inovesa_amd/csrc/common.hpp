@@ -9,6 +9,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -68,7 +69,41 @@ struct vfps_dev {
     int ncu = 0;
     size_t lds_max = 65536;
     std::string arch;
+    // pinned memory results are read back through (DevStage)
+    std::mutex stage_mu;
+    void* stage = nullptr;
 };
+
+namespace vfps_impl {
+
+// The device handle's pinned buffer, held by one caller at a time from the
+// launch that fills it to the copy out of it.  A kernel writes its results
+// there itself, so that a call returning a few arrays costs one launch and
+// one wait where a copy per array costs about 10 us each.  Allocated on first
+// use, freed with the handle.
+constexpr size_t DEV_STAGE_BYTES = 4u << 20;
+
+class DevStage {
+public:
+    explicit DevStage(vfps_dev* dev) : lock_(dev->stage_mu), dev_(dev) {}
+    // null if the allocation failed
+    template <typename T>
+    T* get()
+    {
+        if (!dev_->stage &&
+            hipHostMalloc(&dev_->stage, DEV_STAGE_BYTES,
+                          hipHostMallocDefault) != hipSuccess) {
+            dev_->stage = nullptr;
+        }
+        return static_cast<T*>(dev_->stage);
+    }
+
+private:
+    std::unique_lock<std::mutex> lock_;
+    vfps_dev* dev_;
+};
+
+}  // namespace vfps_impl
 
 struct vfps_mesh {
     vfps_dev* dev = nullptr;

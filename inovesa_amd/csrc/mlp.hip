@@ -198,9 +198,6 @@ __global__ void adam_kernel(float* __restrict__ p, uint16_t* __restrict__ pb,
 
 }  // namespace
 
-// most samples of a forward staged through pinned memory
-constexpr uint32_t MLP_STAGE_ROWS = 1024;
-
 struct vfps_mlp {
     vfps_dev* dev = nullptr;
     std::vector<uint32_t> dims;     // n_in, hidden..., n_out
@@ -221,10 +218,6 @@ struct vfps_mlp {
     uint16_t* GT = nullptr;
     float* dbp = nullptr;           // bias and loss partials
     double* lossp = nullptr;
-    // pinned staging of a forward's inputs and outputs, which the kernel
-    // reads and writes itself
-    float* stage = nullptr;
-    uint32_t stage_rows = 0;
     // training data kept between calls of train (grown as needed)
     void* data = nullptr;
     size_t data_bytes = 0;
@@ -259,7 +252,6 @@ void mlp_free(vfps_mlp* m)
                     (void*)m->dbp, (void*)m->lossp, m->data}) {
         (void)hipFree(q);
     }
-    if (m->stage) (void)hipHostFree(m->stage);
     for (auto* q : m->z) (void)hipFree(q);
     for (auto* q : m->ab) (void)hipFree(q);
     delete m;
@@ -575,11 +567,6 @@ int vfps_mlp_create(vfps_dev* dev, const uint32_t* dims, uint32_t ndims,
         VFPS_HIP(hipMalloc(&m->lossp, sizeof(double) * nwg));
         // (the outputs of a forward longer than the staging)
         VFPS_HIP(hipMalloc(&m->dy, sizeof(float) * B * dims[ndims - 1]));
-        m->stage_rows = std::min(max_batch, MLP_STAGE_ROWS);
-        VFPS_HIP(hipHostMalloc((void**)&m->stage,
-                               sizeof(float) * (size_t)m->stage_rows *
-                                   (dims[0] + dims[ndims - 1]),
-                               hipHostMallocDefault));
         *out = guard.release();
         return vfps_mlp_set_params(*out, p.data(), n);
     }
@@ -660,13 +647,16 @@ int vfps_mlp_forward(vfps_mlp* m, const float* x, uint32_t B, float* y)
     const uint32_t no = m->dims.back();
     const size_t nx = (size_t)B * m->dims[0], ny = (size_t)B * no;
     int rc;
-    if (m->fused() && B <= m->stage_rows) {
+    if (m->fused() && sizeof(float) * (nx + ny) <= DEV_STAGE_BYTES) {
         // the kernel reads the inputs from and writes the outputs to pinned
         // host memory: no copy launches around it (3-256-256-256-65, 512
         // samples: two copies were half of the call)
-        float* ys = m->stage + (size_t)m->stage_rows * m->dims[0];
-        std::memcpy(m->stage, x, sizeof(float) * nx);
-        if ((rc = fused_forward(m, m->stage, B, ys)) != VFPS_OK) return rc;
+        DevStage stage(m->dev);
+        float* xs = stage.get<float>();
+        if (!xs) return fail(VFPS_ERR_NOMEM, "vfps_mlp_forward: pinned memory");
+        float* ys = xs + nx;
+        std::memcpy(xs, x, sizeof(float) * nx);
+        if ((rc = fused_forward(m, xs, B, ys)) != VFPS_OK) return rc;
         VFPS_HIP(hipStreamSynchronize(st));
         std::memcpy(y, ys, sizeof(float) * ny);
         return VFPS_OK;

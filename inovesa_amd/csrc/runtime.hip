@@ -393,6 +393,7 @@ int vfps_dev_close(vfps_dev* dev)
     hipSetDevice(dev->ordinal);
     hipStreamSynchronize(dev->stream);
     hipStreamDestroy(dev->stream);
+    if (dev->stage) hipHostFree(dev->stage);
     delete dev;
     return VFPS_OK;
 }

@@ -748,7 +748,8 @@ int step_retile(vfps_step* s, uint32_t T, uint32_t threads, bool reset)
 }
 
 // The CSR power of the last step of a direct-form run (the shares at
-// parity^1), one workgroup per instance; the counter is at parity.
+// parity^1), one workgroup per instance; the counter is at parity.  An
+// FFT-wake instance has no shares: its field kernel records every step.
 __global__ void __launch_bounds__(256)
 step_finalize_kernel(const InstDesc* __restrict__ descs, uint32_t parity,
                      uint32_t* err_host, uint32_t close_csr)
@@ -758,7 +759,7 @@ step_finalize_kernel(const InstDesc* __restrict__ descs, uint32_t parity,
     if (err_host && threadIdx.x == 0) {
         err_host[blockIdx.x] = *d.err;
     }
-    if (!close_csr || !d.use_csr || !d.counter) {
+    if (!close_csr || !d.use_csr || !d.counter || !d.csr_part) {
         return;
     }
     const uint32_t cnt = d.counter[parity];

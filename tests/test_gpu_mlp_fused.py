@@ -52,11 +52,11 @@ def test_network_edges_match_oracle(V, dims, B):
 
 
 def test_forward_beyond_the_staging(V):
-    dims = (3, 64, 9)
-    net = V.MLP(dims, max_batch=3000, seed=5)
-    x, _, _ = _data(2501, dims)
+    dims = (3, 64, 65)
+    net = V.MLP(dims, max_batch=16000, seed=5)
+    x, _, _ = _data(15500, dims)   # 4.2 MB of inputs and outputs
     y = net.forward(x)
-    for k in (0, 1023, 1024, 2500):
+    for k in (0, 1023, 1024, 15499):
         np.testing.assert_array_equal(y[k:k + 1], net.forward(x[k:k + 1]))
 
 
