@@ -72,6 +72,9 @@ struct vfps_dev {
     // pinned memory results are read back through (DevStage)
     std::mutex stage_mu;
     void* stage = nullptr;
+    // node table of the Airy functions (impedance.hip)
+    std::mutex airy_mu;
+    double* airy = nullptr;
 };
 
 namespace vfps_impl {

@@ -162,8 +162,7 @@ __global__ void airy_kernel(uint32_t n, const double* x, const double* tab,
 // Bi, Bi' increase with u, so that is exactly the set dropped).
 __global__ void __launch_bounds__(256)
 pp_csr_kernel(uint32_t nfreqs, double delta, double r_bend, double f0,
-              double g, const double* __restrict__ tab, float2* z,
-              unsigned long long* nterms)
+              double g, const double* __restrict__ tab, float2* z)
 {
     __shared__ double red[16];
     const uint32_t i = blockIdx.x + 1;
@@ -177,7 +176,6 @@ pp_csr_kernel(uint32_t nfreqs, double delta, double r_bend, double f0,
     const double p23 = pow(2.0, 2. / 3.);
     const uint32_t nodd = (maxp + 1) / 2;  // p = 2t+1 <= maxp
     double zr = 0.0, zi = 0.0;
-    unsigned long long cnt = 0;
     for (uint32_t t = threadIdx.x; t < nodd; t += blockDim.x) {
         const uint32_t p = 2 * t + 1;
         const double u = pi2 * p * p / p23 * b;
@@ -191,17 +189,13 @@ pp_csr_kernel(uint32_t nfreqs, double delta, double r_bend, double f0,
         const double uai = u * ai;
         zr += aip * aip + uai * ai;
         zi += aip * (-bip) + uai * (-bi);
-        cnt++;
     }
     zr = block_sum(zr, red);
     zi = block_sum(zi, red);
-    double c = (double)cnt;
-    c = block_sum(c, red);
     if (threadIdx.x == 0) {
         const double sc = 4.0 * b * n * g / r_bend * pi2 * pow(2.0, 1. / 3.) * z0;
         const float2 old = z[i];
         z[i] = make_float2(old.x + (float)(zr * sc), old.y + (float)(zi * sc));
-        atomicAdd(nterms, (unsigned long long)c);
     }
 }
 
@@ -251,11 +245,26 @@ __global__ void add_kernel(uint32_t n, const float2* a, float2* z)
     z[i] = make_float2(z[i].x + a[i].x, z[i].y + a[i].y);
 }
 
-static int airy_table(hipStream_t st, double** tab)
+// The node table of a device handle: made on its stream by the first call
+// that needs it and kept with the handle.  Its Taylor steps follow one
+// another (two threads, 128 us), and a scan builds an impedance per run: 64
+// tables cost it 8 ms.
+static int airy_table(vfps_dev* dev, double** tab)
 {
-    VFPS_HIP(hipMalloc(tab, sizeof(double) * 4 * AIRY_NODES));
-    hipLaunchKernelGGL(airy_nodes_kernel, dim3(1), dim3(64), 0, st, *tab);
-    VFPS_HIP(hipGetLastError());
+    std::lock_guard<std::mutex> lock(dev->airy_mu);
+    if (!dev->airy) {
+        double* t = nullptr;
+        VFPS_HIP(hipMalloc(&t, sizeof(double) * 4 * AIRY_NODES));
+        hipLaunchKernelGGL(airy_nodes_kernel, dim3(1), dim3(64), 0,
+                           dev->stream, t);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) {
+            hipFree(t);
+            return fail(VFPS_ERR_HIP, hipGetErrorString(e));
+        }
+        dev->airy = t;
+    }
+    *tab = dev->airy;
     return VFPS_OK;
 }
 
@@ -324,23 +333,18 @@ int vfps_impedance_add_parallel_plates(vfps_impedance* z, float f0,
 {
     VFPS_CHECK_ARG(z && f0 > 0 && g > 0, "ParallelPlatesCSR: bad argument");
     double* tab = nullptr;
-    unsigned long long* cnt = nullptr;
     hipStream_t st = z->dev->stream;
-    int rc = airy_table(st, &tab);
+    int rc = airy_table(z->dev, &tab);
     if (rc != VFPS_OK) return rc;
-    VFPS_HIP(hipMalloc(&cnt, sizeof(unsigned long long)));
-    hipMemsetAsync(cnt, 0, sizeof(unsigned long long), st);
     // delta = f_max/f0/(nfreqs-1.0): float quotient, then double
     const double delta = (double)(f_max / f0) / ((double)z->n - 1.0);
     const double r_bend = 2.99792458e8 / (2 * PI_D * (double)f0);
     if (z->n / 2 >= 1) {
         hipLaunchKernelGGL(pp_csr_kernel, dim3(z->n / 2), dim3(256), 0, st,
-                           z->n, delta, r_bend, (double)f0, g, tab, z->z, cnt);
+                           z->n, delta, r_bend, (double)f0, g, tab, z->z);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    hipFree(tab);
-    hipFree(cnt);
     if (e != hipSuccess) {
         return fail(VFPS_ERR_HIP, hipGetErrorString(e));
     }
@@ -416,7 +420,7 @@ int vfps_airy(vfps_dev* dev, const double* x, uint32_t n, double* out,
     double* dx = nullptr;
     double* dout = nullptr;
     int32_t* dovf = nullptr;
-    int rc = airy_table(st, &tab);
+    int rc = airy_table(dev, &tab);
     if (rc != VFPS_OK) return rc;
     hipError_t e = hipMalloc(&dx, sizeof(double) * n);
     if (e == hipSuccess) e = hipMalloc(&dout, sizeof(double) * 4 * n);
@@ -434,7 +438,6 @@ int vfps_airy(vfps_dev* dev, const double* x, uint32_t n, double* out,
                        st);
         e = hipStreamSynchronize(st);
     }
-    hipFree(tab);
     hipFree(dx);
     hipFree(dout);
     hipFree(dovf);

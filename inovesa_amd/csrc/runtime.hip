@@ -394,6 +394,7 @@ int vfps_dev_close(vfps_dev* dev)
     hipStreamSynchronize(dev->stream);
     hipStreamDestroy(dev->stream);
     if (dev->stage) hipHostFree(dev->stage);
+    if (dev->airy) hipFree(dev->airy);
     delete dev;
     return VFPS_OK;
 }
