@@ -363,6 +363,27 @@ struct Batch {
     uint32_t B;
 };
 
+// the rows kernel; returns its workgroups
+template <bool TRAIN>
+uint32_t launch_rows(vfps_mlp* m, const MlpRowsArgs& a)
+{
+    const uint32_t rr = mlp_rows_per_lane(a.B, (uint32_t)m->dev->ncu);
+    // (training: whole 32s of samples, the depth of the gradient products)
+    const uint32_t rows = TRAIN ? (a.B + 31u) & ~31u : a.B;
+    const uint32_t blocks = (rows + 4u * rr - 1) / (4u * rr);
+    const size_t lds = sizeof(float) * m->net.lds_words;
+    const dim3 g(blocks), t(MLP_THREADS);
+    hipStream_t st = m->dev->stream;
+    if (rr == 1) {
+        hipLaunchKernelGGL((mlp_rows_kernel<TRAIN, 1>), g, t, lds, st, m->net, a);
+    } else if (rr == 2) {
+        hipLaunchKernelGGL((mlp_rows_kernel<TRAIN, 2>), g, t, lds, st, m->net, a);
+    } else {
+        hipLaunchKernelGGL((mlp_rows_kernel<TRAIN, 4>), g, t, lds, st, m->net, a);
+    }
+    return blocks;
+}
+
 int fused_forward(vfps_mlp* m, const float* x, uint32_t B, float* y)
 {
     MlpRowsArgs a{};
@@ -371,9 +392,7 @@ int fused_forward(vfps_mlp* m, const float* x, uint32_t B, float* y)
     a.x = x;
     a.B = B;
     a.Y = y;
-    hipLaunchKernelGGL(mlp_rows_kernel<false>, dim3((B + MLP_ROWS - 1) / MLP_ROWS),
-                       dim3(MLP_THREADS), sizeof(float) * m->net.lds_words,
-                       m->dev->stream, m->net, a);
+    launch_rows<false>(m, a);
     VFPS_HIP(hipGetLastError());
     return VFPS_OK;
 }
@@ -383,7 +402,6 @@ int fused_step(vfps_mlp* m, const Batch& b, float wl, float* loss,
                const AdamArgs* adam)
 {
     hipStream_t st = m->dev->stream;
-    const uint32_t blocks = ((b.B + 31u) & ~31u) / MLP_ROWS;
     MlpRowsArgs a{};
     a.W = m->W;
     a.WT = m->WT;
@@ -398,9 +416,8 @@ int fused_step(vfps_mlp* m, const Batch& b, float wl, float* loss,
     a.GT = m->GT;
     a.dbp = m->dbp;
     a.lossp = m->lossp;
-    hipLaunchKernelGGL(mlp_rows_kernel<true>, dim3(blocks), dim3(MLP_THREADS),
-                       sizeof(float) * m->net.lds_words, st, m->net, a);
     MlpGradArgs g{};
+    g.nwg = launch_rows<true>(m, a);
     g.AT = m->AT;
     g.GT = m->GT;
     g.dbp = m->dbp;
@@ -551,14 +568,18 @@ int vfps_mlp_create(vfps_dev* dev, const uint32_t* dims, uint32_t ndims,
         const MlpNet& k = m->net;
         const int lds = (int)(sizeof(float) * k.lds_words);
         if (lds > 65536) {
-            for (const void* fn : {(const void*)&mlp_rows_kernel<false>,
-                                   (const void*)&mlp_rows_kernel<true>}) {
+            for (const void* fn : {(const void*)&mlp_rows_kernel<false, 1>,
+                                   (const void*)&mlp_rows_kernel<false, 2>,
+                                   (const void*)&mlp_rows_kernel<false, 4>,
+                                   (const void*)&mlp_rows_kernel<true, 1>,
+                                   (const void*)&mlp_rows_kernel<true, 2>,
+                                   (const void*)&mlp_rows_kernel<true, 4>}) {
                 VFPS_HIP(hipFuncSetAttribute(
                     fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                     (int)MLP_LDS_MAX));
             }
         }
-        const size_t nwg = k.bmax / MLP_ROWS;
+        const size_t nwg = mlp_max_blocks(k.bmax, (uint32_t)dev->ncu);
         VFPS_HIP(hipMalloc(&m->W, sizeof(uint16_t) * k.wsize));
         VFPS_HIP(hipMalloc(&m->WT, sizeof(uint16_t) * k.wsize));
         VFPS_HIP(hipMalloc(&m->AT, sizeof(uint16_t) * k.arows * k.bmax));

@@ -1,7 +1,7 @@
 // The network in two kernels, for nets whose activations fit the LDS of a
 // CU (every width the surrogate uses).
 //
-//   mlp_rows_kernel   one workgroup takes 16 samples through the whole
+//   mlp_rows_kernel   one workgroup takes 4, 8 or 16 samples through the whole
 //                     network: every layer's product (MFMA 16x16x32 BF16),
 //                     bias, GELU, and, when training, the loss and the
 //                     backward products.  Activations never leave the LDS.
@@ -12,17 +12,19 @@
 //
 // The layer-by-layer form they replace launched 15 kernels a training step
 // (gathers, products, column sums, loss, Adam), most of them one to a few
-// workgroups long: 422 us a step for 256 samples of 3-256-256-256-65, 47 us
-// with the two (an epoch of 8192 samples, uploads included: 13.49 ms before,
-// 1.51 ms).  A forward of 512 samples went from 89.0 to 34.6 us.
+// workgroups long: 422 us a step for 256 samples of 3-256-256-256-65; the two
+// take 20.5 and 5.7 us (an epoch of 8192 samples, uploads included: 13.6 ms
+// before, 1.03 ms).  A forward of 512 samples went from 88.6 to 27.7 us.
 //
 // Operand layout.  v_mfma_f32_16x16x32_bf16 wants 8 consecutive k per lane
-// from both operands, so everything a product reads is kept with its
-// contraction index contiguous and padded with zeros to a multiple of 32:
-// the weights twice, [out][in] for the forward and [in][out] for the
-// backward products; the layer inputs and the output gradients of a batch
-// as [feature][sample] for the weight gradients.  Every operand load is then
-// one aligned 16-byte load per lane without a bounds check.
+// from both operands: lane l holds column (or row) l % 16, k = 8 (l / 16) ...
+// + 7 of a 16 x 32 fragment.  Everything a product reads from memory is kept
+// in that order, a fragment after the other (mlp_frag), padded with zeros to
+// whole fragments: the weights twice, once per direction, and the layer
+// inputs and output gradients of a batch (samples as the contraction).  A
+// fragment load is then 1 KB in a row and needs no bounds check.  With
+// row-major matrices a load touched 16 rows, and the 128 KB of a layer took
+// a workgroup 4 us (30 us a launch for the training kernel, 20.5 now).
 #pragma once
 
 #include "common.hpp"
@@ -55,6 +57,14 @@ __host__ __device__ inline float bf2f(uint16_t h)
 __device__ inline float gelu(float x)
 {
     return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
+}
+// both, from one error function
+__device__ inline float gelu_both(float x, float* grad)
+{
+    const float e = 1.0f + erff(x * 0.70710678118654752f);
+    const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
+    *grad = 0.5f * e + x * pdf;
+    return 0.5f * x * e;
 }
 __device__ inline float gelu_grad(float x)
 {
@@ -90,8 +100,17 @@ __device__ __forceinline__ float adam_update(const AdamArgs& a, float g,
     return pi;
 }
 
+// place of (column c, contraction index k) in a matrix of K contraction
+// indexes (K % 32 == 0) held as fragments
+__host__ __device__ __forceinline__ size_t mlp_frag(uint32_t c, uint32_t k,
+                                                    uint32_t K)
+{
+    return ((size_t)(c >> 4) * (K >> 5) + (k >> 5)) * 512u +
+           (((k & 31u) >> 3) * 16u + (c & 15u)) * 8u + (k & 7u);
+}
+
 constexpr uint32_t MLP_MAX_LAYERS = 8;
-constexpr uint32_t MLP_ROWS = 16;        // samples per workgroup
+constexpr uint32_t MLP_ROWS = 16;        // most samples per workgroup
 constexpr uint32_t MLP_THREADS = 1024;
 constexpr uint32_t MLP_WAVES = MLP_THREADS / 64;
 constexpr uint32_t MLP_FRAGS = 8;        // operand loads in flight per tile
@@ -111,10 +130,12 @@ struct MlpNet {
     uint32_t nbias = 0;                   // bias partials per workgroup
     uint32_t to[MLP_MAX_LAYERS] = {};     // a layer's bias partials
     // LDS (4-byte words)
-    uint32_t zo[MLP_MAX_LAYERS] = {};     // hidden pre-activations [16][wp+4]
+    uint32_t zo[MLP_MAX_LAYERS] = {};     // gelu' of the hidden layers [.][wp+4]
     uint32_t yo = 0;                      // outputs [16][w + 1]
     uint32_t tgt = 0, lab = 0;            // targets [16][w - 1], labels [16]
     uint32_t act[2] = {};                 // BF16 activations [16][as]
+    uint32_t tr = 0;                      // layer inputs, then dZ [feature][.]
+    uint32_t db = 0;                      // bias partials [nbias]
     uint32_t as = 0;                      // their row stride (halves)
     uint32_t lds_words = 0;
     uint32_t wsize = 0, arows = 0, grows = 0;
@@ -165,6 +186,10 @@ inline MlpNet mlp_net(const uint32_t* dims, uint32_t ndims, uint32_t max_batch)
         n.act[k] = z;
         z += MLP_ROWS * n.as / 2;
     }
+    n.tr = z;
+    z += (n.arows + n.grows) * MLP_ROWS / 2;
+    n.db = z;
+    z += n.nbias;
     n.lds_words = z;
     n.bmax = up32(max_batch);
     if ((size_t)z * 4 > MLP_LDS_MAX) return MlpNet{};
@@ -172,8 +197,8 @@ inline MlpNet mlp_net(const uint32_t* dims, uint32_t ndims, uint32_t max_batch)
 }
 
 struct MlpRowsArgs {
-    const uint16_t* W;       // padded BF16 weights [out][in] per layer
-    const uint16_t* WT;      // the same, [in][out]
+    const uint16_t* W;       // BF16 weights per layer: columns out, k in
+    const uint16_t* WT;      // the same, columns in, k out
     const float* p;          // parameters (biases)
     const float* x;          // samples [.][w0]
     const uint32_t* idx;     // rows of the batch in x, T, lab (null: 0, 1, ..)
@@ -183,33 +208,34 @@ struct MlpRowsArgs {
     const float* T;          // [.][out - 1]
     const float* labels;     // [.]
     float wl;                // weight of the label's loss
-    uint16_t* AT;            // layer inputs [feature][bmax]
-    uint16_t* GT;            // layer dZ [feature][bmax]
+    uint16_t* AT;            // layer inputs: columns features, k samples
+    uint16_t* GT;            // layer dZ, the same way
     float* dbp;              // bias partials [workgroup][nbias]
     double* lossp;           // loss partials [workgroup]
 };
 
-// up to MLP_FRAGS operand fragments of one 16-column tile, k from 0: 16
-// bytes per lane each (a fragment past K rereads the last one, unused)
+// up to MLP_FRAGS fragments from q on, of `count` (one past them rereads the
+// last, unused)
 __device__ __forceinline__ void mlp_frags(u16x8 (&f)[MLP_FRAGS],
-                                          const uint16_t* q, uint32_t K)
+                                          const uint16_t* q, uint32_t count,
+                                          uint32_t lane)
 {
 #pragma unroll
     for (uint32_t t = 0; t < MLP_FRAGS; t++) {
-        const uint32_t k = t * 32u < K ? t * 32u : K - 32u;
-        f[t] = *reinterpret_cast<const u16x8*>(q + k);
+        const uint32_t e = t < count ? t : count - 1u;
+        f[t] = *reinterpret_cast<const u16x8*>(q + e * 512u + lane * 8u);
     }
 }
 
 // 16 rows through one product: act [16][as] (BF16, LDS) times the 16
-// columns of the fragments f (the first MLP_FRAGS of the column block q)
+// columns whose fragments are f (the first MLP_FRAGS of the K / 32 at q).
 __device__ __forceinline__ f32x4 mlp_tile(const uint16_t* act, uint32_t as,
-                                          uint32_t r16, uint32_t kq,
+                                          uint32_t lane,
                                           const u16x8 (&f)[MLP_FRAGS],
                                           const uint16_t* q, uint32_t K)
 {
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const uint16_t* a = act + r16 * as + kq;
+    const uint16_t* a = act + (lane & 15u) * as + (lane >> 4) * 8u;
 #pragma unroll
     for (uint32_t t = 0; t < MLP_FRAGS; t++) {
         if (t * 32u < K) {
@@ -219,116 +245,163 @@ __device__ __forceinline__ f32x4 mlp_tile(const uint16_t* act, uint32_t as,
     }
     for (uint32_t k = MLP_FRAGS * 32u; k < K; k += 32u) {
         acc = mfma_bf16(*reinterpret_cast<const u16x8*>(a + k),
-                        *reinterpret_cast<const u16x8*>(q + k), acc);
+                        *reinterpret_cast<const u16x8*>(q + k * 16u + lane * 8u),
+                        acc);
     }
     return acc;
 }
 
-// Bound: the latency of one pass through the layers (16 workgroups for 256
-// samples: the smallest MFMA tile is 16 rows, and 16 rows of the surrogate
-// are 4.8 M products, 1 us of a CU's matrix cores).  Each wavefront owns
-// 16-column tiles and loads the next layer's first operand fragments (8 KB)
-// before the barrier that ends this one, so that the weights' trip from the
-// other XCDs' writes overlaps the epilogue.  3-256-256-256-65: forward of
-// 512 samples, all layers and the transfer, in one launch (was six).
-template <bool TRAIN>
+// Bound: the latency of one pass through the layers.  Samples per workgroup:
+// 4 RR, the fewest that still need no more workgroups than the GPU has CUs
+// (mlp_rows_per_lane).  The products cost a CU 1 us whatever of their 16 rows
+// is in use, but a GELU with its derivative is about 130 instructions: with
+// 16 samples a workgroup's four wavefronts per SIMD spend 3 us a layer on
+// them, and a batch of 256 is 16 workgroups; with 4 samples it is 64 (256
+// samples: 34 us a launch before, 30 after).
+// A lane of a product's result holds rows 4 q .. 4 q + 3 of one column, so
+// sample s = q RR + r is given MFMA row 4 q + r: every lane then has RR
+// samples (the rows between hold stale values that no other row sees).
+// Each wavefront owns 16-column tiles and loads the next layer's first
+// operand fragments (8 KB) and bias before the epilogue of its last tile, so
+// that their trip overlaps it.  What the gradient products read is kept in
+// LDS and stored at the end: a store in between would be waited for by the
+// next use of a load (the counter drains in order).
+template <bool TRAIN, int RR>
 __global__ void __launch_bounds__(MLP_THREADS)
 mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
 {
     extern __shared__ __align__(16) float lds[];
     __shared__ double red[16];
+    constexpr uint32_t R = 4u * RR;  // samples of this workgroup
+    typedef uint16_t packed_t __attribute__((ext_vector_type(RR == 1 ? 2 : RR)));
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t r16 = lane & 15u, q4 = lane >> 4, kq = q4 * 8u;
-    const uint32_t r0 = blockIdx.x * MLP_ROWS;
+    const uint32_t r16 = lane & 15u, q4 = lane >> 4;
+    const uint32_t r0 = blockIdx.x * R;
+    const uint32_t s0 = q4 * RR;     // this lane's first sample
     const uint32_t L = n.L, out = n.w[L];
     uint16_t* act = reinterpret_cast<uint16_t*>(lds + n.act[0]);
     uint16_t* nxt = reinterpret_cast<uint16_t*>(lds + n.act[1]);
     float* y = lds + n.yo;
     u16x8 f[MLP_FRAGS];
+    float bias0 = 0.0f;  // bias of this lane's column of the first tile
 
-    // this wavefront's first tile of a product with weights q [N][K]
-    auto fetch = [&](const uint16_t* q, uint32_t N, uint32_t K) {
-        if (wave * 16u < N) {
-            mlp_frags(f, q + (size_t)(wave * 16u + r16) * K + kq, K);
+    // act row of sample s
+    auto row = [](uint32_t s) { return s / RR * 4u + s % RR; };
+    // layer inputs (arows features), then dZ (grows), R samples each
+    uint16_t* tr = reinterpret_cast<uint16_t*>(lds + n.tr);
+    // this lane's RR samples of one feature
+    auto keep = [&](uint32_t feature, packed_t v) {
+        if constexpr (RR == 1) {
+            tr[feature * R + s0] = v[0];
+        } else {
+            *reinterpret_cast<packed_t*>(tr + feature * R + s0) = v;
         }
     };
-    // the product of the 16 rows in act with q [N][K]; then(acc, column)
-    // per tile; the fragments of the first tile are in f
-    auto product = [&](const uint16_t* q, uint32_t N, uint32_t K, auto&& then) {
-        for (uint32_t tj = wave * 16u; tj < N; tj += MLP_WAVES * 16u) {
-            const uint16_t* col = q + (size_t)(tj + r16) * K + kq;
-            if (tj != wave * 16u) {
-                mlp_frags(f, col, K);
-            }
-            then(mlp_tile(act, n.as, r16, kq, f, col, K), tj + r16);
+    // this wavefront's tile tj of a product with the fragments q of N columns
+    // and K contraction indexes (bias: of the columns, the first nb)
+    auto fetch = [&](const uint16_t* q, uint32_t tj, uint32_t N, uint32_t K,
+                     const float* bias, uint32_t nb) {
+        if (tj < N) {
+            mlp_frags(f, q + (size_t)tj * K, K / 32u, lane);
+            bias0 = tj + r16 < nb ? bias[tj + r16] : 0.0f;
+        }
+    };
+    auto fetch_forward = [&](uint32_t l, uint32_t tj) {
+        fetch(a.W + n.wo[l], tj, n.wp[l + 1], n.wp[l], a.p + n.bo[l], n.w[l + 1]);
+    };
+    auto fetch_backward = [&](uint32_t l, uint32_t tj) {
+        fetch(a.WT + n.wo[l], tj, n.wp[l], n.wp[l + 1], nullptr, 0);
+    };
+    // the product of the rows in act with q (N columns, K contraction
+    // indexes); then(acc, column, bias) per tile.  The operands of the first
+    // tile are in f and bias0; here(tj) fetches those of a later one, next()
+    // those of the product that follows.
+    auto product = [&](const uint16_t* q, uint32_t N, uint32_t K, auto&& here,
+                       auto&& next, auto&& then) {
+        constexpr uint32_t step = MLP_WAVES * 16u;
+        if (wave * 16u >= N) next();
+        for (uint32_t tj = wave * 16u; tj < N; tj += step) {
+            if (tj != wave * 16u) here(tj);
+            const f32x4 acc =
+                mlp_tile(act, n.as, lane, f, q + (size_t)tj * K, K);
+            const float b = bias0;
+            if (tj + step >= N) next();
+            then(acc, tj + r16, b);
         }
     };
 
-    fetch(a.W + n.wo[0], n.wp[1], n.wp[0]);
-    auto sample = [&](uint32_t r) -> size_t {
-        return a.idx ? a.idx[r0 + r] : r0 + r;
+    auto sample = [&](uint32_t s) -> size_t {
+        return a.idx ? a.idx[r0 + s] : r0 + s;
     };
-    // inputs (rows past the batch: zeros), targets and labels
-    for (uint32_t t = tid; t < MLP_ROWS * n.wp[0]; t += MLP_THREADS) {
-        const uint32_t r = t / n.wp[0], c = t % n.wp[0];
-        act[r * n.as + c] = r0 + r < a.B && c < n.w[0]
-                                ? f2bf(a.x[sample(r) * n.w[0] + c])
-                                : (uint16_t)0;
+    // inputs (samples past the batch: zeros), targets and labels
+    for (uint32_t t = tid; t < R * n.wp[0]; t += MLP_THREADS) {
+        const uint32_t s = t / n.wp[0], c = t % n.wp[0];
+        act[row(s) * n.as + c] = r0 + s < a.B && c < n.w[0]
+                                     ? f2bf(a.x[sample(s) * n.w[0] + c])
+                                     : (uint16_t)0;
     }
+    fetch_forward(0, wave * 16u);
     if constexpr (TRAIN) {
         const uint32_t S = out - 1;
-        for (uint32_t t = tid; t < MLP_ROWS * S; t += MLP_THREADS) {
-            const uint32_t r = t / S, c = t % S;
-            lds[n.tgt + t] = r0 + r < a.B ? a.T[sample(r) * S + c] : 0.0f;
+        for (uint32_t t = tid; t < R * S; t += MLP_THREADS) {
+            const uint32_t s = t / S, c = t % S;
+            lds[n.tgt + t] = r0 + s < a.B ? a.T[sample(s) * S + c] : 0.0f;
         }
-        if (tid < MLP_ROWS) {
+        if (tid < R) {
             lds[n.lab + tid] = r0 + tid < a.B ? a.labels[sample(tid)] : 0.0f;
         }
     }
     __syncthreads();
     if constexpr (TRAIN) {
-        for (uint32_t t = tid; t < MLP_ROWS * n.wp[0]; t += MLP_THREADS) {
-            const uint32_t c = t / MLP_ROWS, r = t % MLP_ROWS;
-            a.AT[(size_t)(n.ao[0] + c) * n.bmax + r0 + r] = act[r * n.as + c];
+        for (uint32_t t = tid; t < R * n.wp[0]; t += MLP_THREADS) {
+            const uint32_t c = t / R, s = t % R;
+            tr[(n.ao[0] + c) * R + s] = act[row(s) * n.as + c];
         }
     }
 
     // ---- forward -------------------------------------------------------------
     for (uint32_t l = 0; l < L; l++) {
         const uint32_t N = n.w[l + 1], NP = n.wp[l + 1];
-        const float* bias = a.p + n.bo[l];
         const bool last = l + 1 == L;
-        product(a.W + n.wo[l], NP, n.wp[l], [&](f32x4 acc, uint32_t j) {
-            const float b = j < N ? bias[j] : 0.0f;
-            u16x4 packed;
+        auto next = [&]() {
+            if (!last) {
+                fetch_forward(l + 1, wave * 16u);
+            } else if (TRAIN && L > 1) {
+                fetch_backward(l, wave * 16u);
+            }
+        };
+        product(a.W + n.wo[l], NP, n.wp[l],
+                [&](uint32_t tj) { fetch_forward(l, tj); }, next,
+                [&](f32x4 acc, uint32_t j, float b) {
+            packed_t packed;
 #pragma unroll
-            for (uint32_t r = 0; r < 4; r++) {
-                const uint32_t i = q4 * 4u + r;
+            for (uint32_t r = 0; r < (uint32_t)RR; r++) {
+                const uint32_t s = s0 + r;
                 const float z = acc[r] + b;
                 if (!last) {
-                    const uint16_t h = f2bf(gelu(z));
-                    nxt[i * n.as + j] = h;
-                    // (rows past the batch add nothing to the gradients)
-                    packed[r] = r0 + i < a.B ? h : (uint16_t)0;
-                    if (TRAIN) lds[n.zo[l] + i * (NP + 4u) + j] = z;
+                    float h, grad = 0.0f;
+                    if (TRAIN) {
+                        h = gelu_both(z, &grad);
+                        lds[n.zo[l] + s * (NP + 4u) + j] = grad;
+                    } else {
+                        h = gelu(z);
+                    }
+                    const uint16_t hb = f2bf(h);
+                    nxt[row(s) * n.as + j] = hb;
+                    // (samples past the batch add nothing to the gradients)
+                    packed[r] = r0 + s < a.B ? hb : (uint16_t)0;
                 } else if (j < N) {
                     if (TRAIN) {
-                        y[i * (N + 1u) + j] = z;
-                    } else if (r0 + i < a.B) {
-                        a.Y[(size_t)(r0 + i) * N + j] = z;
+                        y[s * (N + 1u) + j] = z;
+                    } else if (r0 + s < a.B) {
+                        a.Y[(size_t)(r0 + s) * N + j] = z;
                     }
                 }
             }
             if (TRAIN && !last) {
-                *reinterpret_cast<u16x4*>(a.AT + (size_t)(n.ao[l + 1] + j) * n.bmax +
-                                          r0 + q4 * 4u) = packed;
+                keep(n.ao[l + 1] + j, packed);
             }
         });
-        if (!last) {
-            fetch(a.W + n.wo[l + 1], n.wp[l + 2], NP);
-        } else if (TRAIN && L > 1) {
-            fetch(a.WT + n.wo[l], n.wp[l], NP);
-        }
         __syncthreads();
         uint16_t* t = act;
         act = nxt;
@@ -345,17 +418,17 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
     {
         const uint32_t S = out - 1, NP = n.wp[L];
         double loss = 0.0;
-        for (uint32_t t = tid; t < MLP_ROWS * NP; t += MLP_THREADS) {
-            const uint32_t r = t / NP, k = t % NP;
+        for (uint32_t t = tid; t < R * NP; t += MLP_THREADS) {
+            const uint32_t s = t / NP, k = t % NP;
             float g = 0.0f;
-            if (k < out && r0 + r < a.B) {
-                const float v = y[r * (out + 1u) + k];
+            if (k < out && r0 + s < a.B) {
+                const float v = y[s * (out + 1u) + k];
                 if (k < S) {
-                    const float d = v - lds[n.tgt + r * S + k];
+                    const float d = v - lds[n.tgt + s * S + k];
                     loss += (double)d * (double)d / (double)S;
                     g = 2.0f * d / (float)(S * a.B);
                 } else {
-                    const float lab = lds[n.lab + r];
+                    const float lab = lds[n.lab + s];
                     // BCE with logits: max(y,0) - y*lab + log(1 + exp(-|y|))
                     loss += (double)a.wl *
                             ((double)fmaxf(v, 0.0f) - (double)v * lab +
@@ -364,62 +437,82 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
                     g = a.wl * (sg - lab) / (float)a.B;
                 }
             }
-            if (k < out) y[r * (out + 1u) + k] = g;
-            act[r * n.as + k] = f2bf(g);
+            if (k < out) y[s * (out + 1u) + k] = g;
+            act[row(s) * n.as + k] = f2bf(g);
         }
         loss = block_sum(loss, red);  // (its barriers order act and y too)
-        if (tid == 0) {
-            a.lossp[blockIdx.x] = loss;
-        }
-        float* db = a.dbp + (size_t)blockIdx.x * n.nbias + n.to[L - 1];
+        if (tid == 0) red[0] = loss;
         for (uint32_t k = tid; k < NP; k += MLP_THREADS) {
-            u16x8 h[2];
-            float s = 0.0f;
+            float sum = 0.0f;
 #pragma unroll
-            for (uint32_t r = 0; r < MLP_ROWS; r++) {
-                h[r >> 3][r & 7u] = act[r * n.as + k];
-                if (k < out) s += y[r * (out + 1u) + k];
+            for (uint32_t s = 0; s < R; s++) {
+                tr[(n.arows + n.go[L - 1] + k) * R + s] = act[row(s) * n.as + k];
+                if (k < out) sum += y[s * (out + 1u) + k];
             }
-            db[k] = s;
-            u16x8* dst = reinterpret_cast<u16x8*>(
-                a.GT + (size_t)(n.go[L - 1] + k) * n.bmax + r0);
-            dst[0] = h[0];
-            dst[1] = h[1];
+            lds[n.db + n.to[L - 1] + k] = sum;
         }
     }
 
     // ---- backward: dZ of layer l - 1 from dZ of layer l ---------------------------
     for (uint32_t l = L - 1; l > 0; l--) {
         const uint32_t NP = n.wp[l];
-        const float* z = lds + n.zo[l - 1];
-        float* db = a.dbp + (size_t)blockIdx.x * n.nbias + n.to[l - 1];
-        product(a.WT + n.wo[l], NP, n.wp[l + 1], [&](f32x4 acc, uint32_t j) {
-            u16x4 packed;
-            float s = 0.0f;
+        const float* grad = lds + n.zo[l - 1];
+        auto next = [&]() {
+            if (l > 1) fetch_backward(l - 1, wave * 16u);
+        };
+        product(a.WT + n.wo[l], NP, n.wp[l + 1],
+                [&](uint32_t tj) { fetch_backward(l, tj); }, next,
+                [&](f32x4 acc, uint32_t j, float) {
+            packed_t packed;
+            float sum = 0.0f;
 #pragma unroll
-            for (uint32_t r = 0; r < 4; r++) {
-                const uint32_t i = q4 * 4u + r;
-                const float dz = r0 + i < a.B
-                                     ? acc[r] * gelu_grad(z[i * (NP + 4u) + j])
+            for (uint32_t r = 0; r < (uint32_t)RR; r++) {
+                const uint32_t s = s0 + r;
+                const float dz = r0 + s < a.B
+                                     ? acc[r] * grad[s * (NP + 4u) + j]
                                      : 0.0f;
-                s += dz;
+                sum += dz;
                 packed[r] = f2bf(dz);
-                nxt[i * n.as + j] = packed[r];
+                nxt[row(s) * n.as + j] = packed[r];
             }
-            *reinterpret_cast<u16x4*>(a.GT + (size_t)(n.go[l - 1] + j) * n.bmax +
-                                      r0 + q4 * 4u) = packed;
-            s += __shfl_xor(s, 16, 64);
-            s += __shfl_xor(s, 32, 64);
-            if (q4 == 0) db[j] = s;
+            keep(n.arows + n.go[l - 1] + j, packed);
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            if (q4 == 0) lds[n.db + n.to[l - 1] + j] = sum;
         });
-        if (l > 1) {
-            fetch(a.WT + n.wo[l - 1], n.wp[l - 1], NP);
-        }
         __syncthreads();
         uint16_t* t = act;
         act = nxt;
         nxt = t;
     }
+    if (L == 1) __syncthreads();
+    // ---- what the gradient products and biases read -------------------------------
+    for (uint32_t t = tid; t < (n.arows + n.grows) * RR; t += MLP_THREADS) {
+        const uint32_t feature = t / RR, c = t % RR;
+        const bool in = feature < n.arows;
+        *reinterpret_cast<u16x4*>(
+            (in ? a.AT : a.GT) +
+            mlp_frag(in ? feature : feature - n.arows, r0 + 4u * c, n.bmax)) =
+            *reinterpret_cast<const u16x4*>(tr + feature * R + 4u * c);
+    }
+    if (tid == 0) {
+        a.lossp[blockIdx.x] = red[0];
+    }
+    for (uint32_t t = tid; t < n.nbias; t += MLP_THREADS) {
+        a.dbp[(size_t)blockIdx.x * n.nbias + t] = lds[n.db + t];
+    }
+}
+
+// Samples per lane (RR) of a batch of B samples on a GPU of ncu CUs.
+inline uint32_t mlp_rows_per_lane(uint32_t B, uint32_t ncu)
+{
+    const uint32_t rows = (B + 31u) & ~31u;
+    return rows <= 4u * ncu ? 1u : rows <= 8u * ncu ? 2u : 4u;
+}
+// most workgroups of the rows kernel for any batch of at most bmax samples
+inline uint32_t mlp_max_blocks(uint32_t bmax, uint32_t ncu)
+{
+    return std::max(std::min(bmax / 4u, ncu), bmax / MLP_ROWS);
 }
 
 struct MlpGradArgs {
@@ -427,6 +520,7 @@ struct MlpGradArgs {
     const uint16_t* GT;
     const float* dbp;
     const double* lossp;
+    uint32_t nwg;            // workgroups of the rows kernel
     uint32_t B;
     float* g;                // gradients
     float* loss;             // [1] the batch's loss
@@ -457,7 +551,7 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
 {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t K = (a.B + 31u) & ~31u;
-    const uint32_t nwg = K / MLP_ROWS;  // workgroups of the rows kernel
+    const uint32_t nwg = a.nwg;
     if (blockIdx.x < tile_blocks) {
         uint32_t tile = blockIdx.x * (MLP_GRAD_THREADS / 64u) + wave;
         uint32_t l = 0;
@@ -470,8 +564,8 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
         const uint32_t tk = (ni + 15u) / 16u;
         const uint32_t j0 = (tile / tk) * 16u, k0 = (tile % tk) * 16u;
         const uint32_t r16 = lane & 15u, q4 = lane >> 4;
-        const uint16_t* ga = a.GT + (size_t)(n.go[l] + j0 + r16) * n.bmax + q4 * 8u;
-        const uint16_t* xa = a.AT + (size_t)(n.ao[l] + k0 + r16) * n.bmax + q4 * 8u;
+        const uint16_t* ga = a.GT + (size_t)(n.go[l] + j0) * n.bmax;
+        const uint16_t* xa = a.AT + (size_t)(n.ao[l] + k0) * n.bmax;
         const uint32_t k = k0 + r16;
         // the parameters and moments of this lane's four entries, fetched
         // beside the operands
@@ -490,8 +584,8 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         for (uint32_t b = 0; b < K; b += MLP_FRAGS * 32u) {
             u16x8 fg[MLP_FRAGS], fx[MLP_FRAGS];
-            mlp_frags(fg, ga + b, K - b);
-            mlp_frags(fx, xa + b, K - b);
+            mlp_frags(fg, ga + b * 16u, (K - b) / 32u, lane);
+            mlp_frags(fx, xa + b * 16u, (K - b) / 32u, lane);
 #pragma unroll
             for (uint32_t t = 0; t < MLP_FRAGS; t++) {
                 if (b + t * 32u < K) acc = mfma_bf16(fg[t], fx[t], acc);
@@ -509,13 +603,13 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
                 a.p[o] = pv[r];
                 a.m[o] = mv[r];
                 a.v[o] = vv[r];
-                a.W[n.wo[l] + (size_t)j * n.wp[l] + k] = packed[r];
+                a.W[n.wo[l] + mlp_frag(j, k, n.wp[l])] = packed[r];
             }
         }
         if (ADAM && k < ni) {
             // (rows past the layer's last keep their zeros)
-            *reinterpret_cast<u16x4*>(a.WT + n.wo[l] + (size_t)k * n.wp[l + 1] +
-                                      j0 + q4 * 4u) = packed;
+            *reinterpret_cast<u16x4*>(
+                a.WT + n.wo[l] + mlp_frag(k, j0 + q4 * 4u, n.wp[l + 1])) = packed;
         }
         return;
     }
@@ -526,6 +620,7 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
         const uint32_t j = t - n.to[l];
         if (j < n.w[l + 1]) {
             float s = 0.0f;
+#pragma unroll 16
             for (uint32_t w = 0; w < nwg; w++) {
                 s += a.dbp[(size_t)w * n.nbias + t];
             }
@@ -538,6 +633,7 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
     }
     if (blockIdx.x == gridDim.x - 1 && tid == MLP_GRAD_THREADS - 1) {
         double s = 0.0;
+#pragma unroll 16
         for (uint32_t w = 0; w < nwg; w++) s += a.lossp[w];
         *a.loss = (float)(s / (double)a.B);
     }
@@ -557,8 +653,8 @@ mlp_pack_kernel(MlpNet n, const float* __restrict__ p, uint16_t* __restrict__ W,
         const bool in = j < n.w[l + 1] && k < n.w[l];
         const uint16_t h = in ? f2bf(p[n.po[l] + (size_t)j * n.w[l] + k])
                               : (uint16_t)0;
-        W[t] = h;
-        WT[n.wo[l] + (size_t)k * n.wp[l + 1] + j] = h;
+        W[n.wo[l] + mlp_frag(j, k, n.wp[l])] = h;
+        WT[n.wo[l] + mlp_frag(k, j, n.wp[l + 1])] = h;
     }
 }
 

@@ -60,6 +60,26 @@ def test_forward_beyond_the_staging(V):
         np.testing.assert_array_equal(y[k:k + 1], net.forward(x[k:k + 1]))
 
 
+@pytest.mark.parametrize("B", [1030, 2100, 4200])
+def test_samples_per_workgroup(V, B):
+    """4, 8 and 16 samples per workgroup (by the batch and 256 CUs): the
+    same sums per sample, so the same outputs as a small batch; gradients
+    against the oracle."""
+    dims = (3, 40, 17, 9)
+    net = V.MLP(dims, max_batch=B, seed=7)
+    x, t, lab = _data(B, dims, seed=2)
+    y = net.forward(x)
+    for k in (0, 500, B - 3):
+        np.testing.assert_array_equal(y[k:k + 3], net.forward(x[k:k + 3]))
+    loss = net.loss_grad(x, t, lab, 0.5)
+    rloss, rg = mo.loss_and_grads(mo.split(net.params(), dims), x, t, lab, 0.5,
+                                  emulate=True)
+    assert loss == pytest.approx(rloss, rel=1e-3)
+    for (dW, db), (rW, rb) in zip(net.layers(net.grads()), rg):
+        assert _rel(dW, rW) <= 2e-2
+        assert _rel(db, rb) <= 2e-2
+
+
 @pytest.mark.parametrize("dims", [(3, 48, 33, 9), (3, 1200, 1100, 9)])
 def test_train_is_gradients_and_adam(V, dims):
     """One update over the whole set, fused, against loss_grad + adam_step.
