@@ -91,21 +91,28 @@ __global__ void outer_kernel(uint32_t nb, uint32_t n, const float* g,
 // projection equals the reference's bit for bit (the wake potential
 // amplifies the last bits of the profile through the high-frequency
 // impedance).  A workgroup takes PX_ROWS rows: all its threads form the
-// products data*ws with coalesced loads into LDS (rows padded by 4 words),
-// then one lane per row adds its row in order from LDS.
+// products data*ws with coalesced loads into LDS (rows filled up with +0 to
+// 16 words, which changes no sum that starts at +0, and 4 words apart), then
+// one lane per row adds its row in order from LDS, 16 bytes a load.
 constexpr uint32_t PX_ROWS = 16;
 constexpr uint32_t PX_THREADS = 256;
 constexpr int PX_BATCH = 8;   // float4 loads in flight per thread
+
+__host__ __device__ constexpr uint32_t px_stride(uint32_t n)
+{
+    return ((n + 15u) & ~15u) + 4u;
+}
 
 __global__ void __launch_bounds__(PX_THREADS)
 project_x_kernel(uint32_t rows, uint32_t n, uint32_t rows_per_wg,
                  const float* __restrict__ data,
                  const float* __restrict__ ws, float* __restrict__ proj)
 {
-    extern __shared__ __align__(16) float px[];   // rows_per_wg * (n + 4)
+    extern __shared__ __align__(16) float px[];   // rows_per_wg * px_stride(n)
     const uint32_t r0 = blockIdx.x * rows_per_wg;
     const uint32_t nr = min(rows_per_wg, rows - r0);
-    const uint32_t stride = n + 4;
+    const uint32_t stride = px_stride(n);
+    const uint32_t np = stride - 4u;
     const float* src = data + (size_t)r0 * n;
     if ((n & 3u) == 0u) {
         // PX_BATCH float4s of the rows (and their weights) in flight per
@@ -152,34 +159,34 @@ project_x_kernel(uint32_t rows, uint32_t n, uint32_t rows_per_wg,
             px[r * stride + y] = src[i] * ws[y];
         }
     }
+    if (np != n) {
+        for (uint32_t i = threadIdx.x; i < nr * 16u; i += blockDim.x) {
+            const uint32_t y = np - 16u + (i & 15u);
+            if (y >= n) px[(i >> 4) * stride + y] = 0.0f;
+        }
+    }
     __syncthreads();
     if (threadIdx.x < nr) {
-        const float* p = px + threadIdx.x * stride;
         float acc = 0.0f;
-        uint32_t y = 0;
-        if ((n & 15u) == 0u) {
-            // the next 16 products load while the current 16 are added
-            const float4* p4 = reinterpret_cast<const float4*>(p);
-            float4 q[4], nq[4];
+        // the next 16 products load while the current 16 are added
+        const float4* p4 =
+            reinterpret_cast<const float4*>(px + threadIdx.x * stride);
+        float4 q[4], nq[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) q[k] = p4[k];
-            for (; y < n; y += 16) {
-                const uint32_t yn = y + 16 < n ? y + 16 : y;
+        for (int k = 0; k < 4; k++) q[k] = p4[k];
+        for (uint32_t y = 0; y < np; y += 16) {
+            const uint32_t yn = y + 16 < np ? y + 16 : y;
 #pragma unroll
-                for (int k = 0; k < 4; k++) nq[k] = p4[(yn >> 2) + k];
+            for (int k = 0; k < 4; k++) nq[k] = p4[(yn >> 2) + k];
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    acc = acc + q[k].x;
-                    acc = acc + q[k].y;
-                    acc = acc + q[k].z;
-                    acc = acc + q[k].w;
-                }
-#pragma unroll
-                for (int k = 0; k < 4; k++) q[k] = nq[k];
+            for (int k = 0; k < 4; k++) {
+                acc = acc + q[k].x;
+                acc = acc + q[k].y;
+                acc = acc + q[k].z;
+                acc = acc + q[k].w;
             }
-        }
-        for (; y < n; y++) {
-            acc = acc + p[y];
+#pragma unroll
+            for (int k = 0; k < 4; k++) q[k] = nq[k];
         }
         proj[r0 + threadIdx.x] = acc;
     }
@@ -315,10 +322,12 @@ __global__ void variance_kernel(uint32_t n, const float* proj,
 int launch_project_x(vfps_mesh* m, const float* src, float* proj)
 {
     const uint32_t rows = m->nb * m->n;
-    // as many rows per workgroup as the LDS holds, up to PX_ROWS
-    const size_t row_bytes = sizeof(float) * (m->n + 4);
+    // rows per workgroup: enough workgroups for the CUs (two meshes of 256^2
+    // in rows of 16 were 32 of them), at most PX_ROWS and what the LDS holds
+    const size_t row_bytes = sizeof(float) * px_stride(m->n);
+    const size_t share = ceil_div(rows, (size_t)std::max(m->dev->ncu, 1));
     const uint32_t rpw = (uint32_t)std::max<size_t>(
-        1, std::min<size_t>(PX_ROWS, m->dev->lds_max / row_bytes));
+        1, std::min({share, (size_t)PX_ROWS, m->dev->lds_max / row_bytes}));
     const size_t lds = row_bytes * rpw;
     VFPS_CHECK_ARG(lds <= m->dev->lds_max,
                    "updateXProjection: a mesh row exceeds the LDS");

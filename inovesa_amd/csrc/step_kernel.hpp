@@ -1081,32 +1081,62 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                         acc = acc + qb[k].w;
                     }
                 }
-            } else if ((n & 15u) == 0u) {
-                // the next 16 values load while the current 16 are added
+            } else if (vec_rows) {
+                // other lengths: the same with the loads held inside the row,
+                // and the last n % 64 values' loads together (one word at a
+                // time the last n % 16 took 30 cycles each: the projection of
+                // two rows of 388 took 11.9 us, now 2.2)
                 const vec4f* r4 = reinterpret_cast<const vec4f*>(r);
-                vec4f q[4], nq[4];
+                const uint32_t n4 = n >> 2;
+                vec4f qa[8], qb[8];
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    q[k] = r4[k];
+                for (uint32_t k = 0; k < 8; k++) {
+                    qa[k] = r4[min(k, n4 - 1u)];
                 }
-                for (; y < n; y += 16) {
-                    const uint32_t yn = y + 16 < n ? y + 16 : y;
+#pragma unroll 1
+                for (; y + 64 <= n; y += 64) {
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        nq[k] = r4[(yn >> 2) + k];
+                    for (int k = 0; k < 8; k++) {
+                        qb[k] = r4[((y + 32) >> 2) + k];
                     }
+                    if constexpr (ONE_MESH) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        acc = acc + q[k].x;
-                        acc = acc + q[k].y;
-                        acc = acc + q[k].z;
-                        acc = acc + q[k].w;
+                    for (int k = 0; k < 8; k++) {
+                        acc = acc + qa[k].x;
+                        acc = acc + qa[k].y;
+                        acc = acc + qa[k].z;
+                        acc = acc + qa[k].w;
                     }
+                    if constexpr (ONE_MESH) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        q[k] = nq[k];
+                    for (uint32_t k = 0; k < 8; k++) {
+                        qa[k] = r4[min(((y + 64) >> 2) + k, n4 - 1u)];
+                    }
+                    if constexpr (ONE_MESH) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        acc = acc + qb[k].x;
+                        acc = acc + qb[k].y;
+                        acc = acc + qb[k].z;
+                        acc = acc + qb[k].w;
                     }
                 }
+                const uint32_t left4 = (n - y) >> 2;
+#pragma unroll
+                for (uint32_t k = 0; k < 8; k++) {
+                    qb[k] = r4[min(((y + 32) >> 2) + k, n4 - 1u)];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < 16; k++) {
+                    if (k < left4) {
+                        const vec4f q = k < 8u ? qa[k & 7u] : qb[k & 7u];
+                        acc = acc + q.x;
+                        acc = acc + q.y;
+                        acc = acc + q.z;
+                        acc = acc + q.w;
+                    }
+                }
+                y = n;
             }
             for (; y < n; y++) {
                 acc = acc + r[y];
