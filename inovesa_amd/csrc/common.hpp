@@ -106,6 +106,28 @@ private:
     vfps_dev* dev_;
 };
 
+// Device arrays to host memory (src, dst and bytes multiples of 4), after
+// everything on the stream so far; returns when they are there.  Up to
+// READ_BACK_MAX bytes one kernel copies all of them into the pinned buffer:
+// one launch and one wait (about 8 us) where a pageable copy takes 10 us per
+// array.  Longer ones are copied by the runtime.
+struct ReadBack {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+constexpr size_t READ_BACK_ARRAYS = 4;
+constexpr size_t READ_BACK_MAX = 64u << 10;
+int read_back(vfps_dev* dev, const ReadBack* arrays, size_t count);
+
+// n floats of host memory to the device, in stream order; src may be reused
+// when the call returns.  Up to UPLOAD_MAX of them travel as arguments of a
+// kernel that stores them: nothing is waited for (a pageable copy and the
+// wait for it take 16 us).
+constexpr size_t UPLOAD_ARGS = 960;   // floats in the arguments of one launch
+constexpr size_t UPLOAD_MAX = 4 * UPLOAD_ARGS;
+int upload_floats(vfps_dev* dev, float* dst, const float* src, size_t n);
+
 }  // namespace vfps_impl
 
 struct vfps_mesh {
@@ -164,8 +186,6 @@ struct vfps_map {
     float rf_syncphase = 0;
     std::vector<float> modulation;  // [steps][2]: phase, amplitude
     uint32_t mod_next = 0;          // entries applied so far
-    float* stage_h = nullptr;       // pinned host offsets of the next apply
-    hipEvent_t stage_done = nullptr;  // the last upload from stage_h
 };
 
 struct vfps_impedance {
@@ -192,7 +212,8 @@ struct vfps_field {
                                  // the chirp table
     double2* tw_n = nullptr;     // e^{-2 pi i k/nmax}, k < M
     float* csr_renorm = nullptr; // [nmax]
-    float* spectrum = nullptr;   // [nb][nmax]
+    float* spectrum = nullptr;   // [nb][nmax] (only where the pinned buffer
+                                 // of the device handle is too small)
     float* power = nullptr;      // [nb]
     float csr_fc = -1;           // fc the renorm table was built for
     float fdelta = 0;            // frequency ruler step (1/(dq (nmax-1)))

@@ -374,7 +374,6 @@ int vfps_field_create(vfps_mesh* ps, vfps_impedance* z,
     e = e ? e : hipMalloc(&f->tw_m, sizeof(double2) * twm.size());
     e = e ? e : hipMalloc(&f->tw_n, sizeof(double2) * M);
     e = e ? e : hipMalloc(&f->csr_renorm, sizeof(float) * nmax);
-    e = e ? e : hipMalloc(&f->spectrum, sizeof(float) * nb * nmax);
     e = e ? e : hipMalloc(&f->power, sizeof(float) * nb);
     if (e != hipSuccess) {
         vfps_field_destroy(f);
@@ -392,7 +391,6 @@ int vfps_field_create(vfps_mesh* ps, vfps_impedance* z,
                    hipMemcpyHostToDevice, st);
     hipMemcpyAsync(f->csr_renorm, renorm.data(), sizeof(float) * nmax,
                    hipMemcpyHostToDevice, st);
-    hipMemsetAsync(f->spectrum, 0, sizeof(float) * nb * nmax, st);
     hipMemsetAsync(f->power, 0, sizeof(float) * nb, st);
     e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
@@ -449,32 +447,36 @@ int vfps_field_pad(vfps_field* f)
 int vfps_field_get_padded(vfps_field* f, float* out)
 {
     VFPS_CHECK_ARG(f && out, "getPaddedBunchProfiles: NULL argument");
-    VFPS_HIP(hipMemcpyAsync(out, f->padded, sizeof(float) * f->nmax,
-                            hipMemcpyDeviceToHost, f->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(f->dev->stream));
-    return VFPS_OK;
+    const ReadBack r{out, f->padded, sizeof(float) * f->nmax};
+    return read_back(f->dev, &r, 1);
 }
 
 int vfps_field_get_padded_wake(vfps_field* f, float* out)
 {
     VFPS_CHECK_ARG(f && out, "getPaddedWakePotential: NULL argument");
-    VFPS_HIP(hipMemcpyAsync(out, f->wake_padded, sizeof(float) * f->nmax,
-                            hipMemcpyDeviceToHost, f->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(f->dev->stream));
-    return VFPS_OK;
+    const ReadBack r{out, f->wake_padded, sizeof(float) * f->nmax};
+    return read_back(f->dev, &r, 1);
 }
 
 int vfps_field_wake_potential(vfps_field* f, float* wp)
 {
     VFPS_CHECK_ARG(f, "wakePotential: NULL field");
-    int rc = launch_wake_potential(f, nullptr);
+    VFPS_TRY_BEGIN
+    if (!wp) return launch_wake_potential(f, nullptr);
+    // the kernel writes the wake to the pinned buffer beside f->wake
+    const size_t bytes = sizeof(float) * f->nb * f->ps->n;
+    DevStage stage(f->dev);
+    float* out = bytes <= DEV_STAGE_BYTES ? stage.get<float>() : nullptr;
+    int rc = launch_wake_potential(f, out);
     if (rc != VFPS_OK) return rc;
-    if (wp) {
-        VFPS_HIP(hipMemcpyAsync(wp, f->wake, sizeof(float) * f->nb * f->ps->n,
-                                hipMemcpyDeviceToHost, f->dev->stream));
-        VFPS_HIP(hipStreamSynchronize(f->dev->stream));
+    if (!out) {
+        VFPS_HIP(hipMemcpyAsync(wp, f->wake, bytes, hipMemcpyDeviceToHost,
+                                f->dev->stream));
     }
+    VFPS_HIP(hipStreamSynchronize(f->dev->stream));
+    if (out) std::memcpy(wp, out, bytes);
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 int vfps_field_get_wakescaling(const vfps_field* f, float* s)
@@ -499,8 +501,31 @@ int vfps_field_update_csr(vfps_field* f, float fc, float* power,
         f->csr_fc = fc;
     }
     FieldParams p = field_params(f);
-    p.spectrum = f->spectrum;
     p.power = f->power;
+    if (!power && !spectrum) {
+        return launch_field(p, false, true, f->nb, f->dev->stream);
+    }
+    // the kernel writes what is asked for to the pinned buffer, or, where
+    // that is too small, to the device and the runtime copies it
+    const size_t nspec = spectrum ? (size_t)f->nb * f->nmax : 0;
+    DevStage stage(f->dev);
+    float* out = sizeof(float) * (f->nb + nspec) <= DEV_STAGE_BYTES
+                     ? stage.get<float>()
+                     : nullptr;
+    if (out) {
+        p.power = out;
+        if (spectrum) p.spectrum = out + f->nb;
+        int rc = launch_field(p, false, true, f->nb, f->dev->stream);
+        if (rc != VFPS_OK) return rc;
+        VFPS_HIP(hipStreamSynchronize(f->dev->stream));
+        if (power) std::memcpy(power, out, sizeof(float) * f->nb);
+        if (spectrum) std::memcpy(spectrum, out + f->nb, sizeof(float) * nspec);
+        return VFPS_OK;
+    }
+    if (nspec && !f->spectrum) {
+        VFPS_HIP(hipMalloc(&f->spectrum, sizeof(float) * nspec));
+    }
+    p.spectrum = spectrum ? f->spectrum : nullptr;
     int rc = launch_field(p, false, true, f->nb, f->dev->stream);
     if (rc != VFPS_OK) return rc;
     if (power) {
@@ -508,13 +533,10 @@ int vfps_field_update_csr(vfps_field* f, float fc, float* power,
                                 hipMemcpyDeviceToHost, f->dev->stream));
     }
     if (spectrum) {
-        VFPS_HIP(hipMemcpyAsync(spectrum, f->spectrum,
-                                sizeof(float) * f->nb * f->nmax,
+        VFPS_HIP(hipMemcpyAsync(spectrum, f->spectrum, sizeof(float) * nspec,
                                 hipMemcpyDeviceToHost, f->dev->stream));
     }
-    if (power || spectrum) {
-        VFPS_HIP(hipStreamSynchronize(f->dev->stream));
-    }
+    VFPS_HIP(hipStreamSynchronize(f->dev->stream));
     return VFPS_OK;
     VFPS_TRY_END
 }

@@ -557,10 +557,7 @@ int vfps_map_set_offset(vfps_map* map, const float* offset, size_t n)
     VFPS_CHECK_ARG(map->kind == MAP_KICK_X || map->kind == MAP_KICK_Y,
                    "swapOffset: not a KickMap");
     VFPS_CHECK_ARG(n == map->noff, "swapOffset: expected nx*nb offsets");
-    VFPS_HIP(hipMemcpyAsync(map->offset, offset, sizeof(float) * n,
-                            hipMemcpyHostToDevice, map->in->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(map->in->dev->stream));
-    return VFPS_OK;
+    return upload_floats(map->in->dev, map->offset, offset, n);
 }
 
 int vfps_map_get_offset(vfps_map* map, float* offset, size_t n)
@@ -569,10 +566,8 @@ int vfps_map_get_offset(vfps_map* map, float* offset, size_t n)
     VFPS_CHECK_ARG(map->kind == MAP_KICK_X || map->kind == MAP_KICK_Y,
                    "getForce: not a KickMap");
     VFPS_CHECK_ARG(n == map->noff, "getForce: expected nx*nb offsets");
-    VFPS_HIP(hipMemcpyAsync(offset, map->offset, sizeof(float) * n,
-                            hipMemcpyDeviceToHost, map->in->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(map->in->dev->stream));
-    return VFPS_OK;
+    const ReadBack r{offset, map->offset, sizeof(float) * n};
+    return read_back(map->in->dev, &r, 1);
 }
 
 int vfps_map_create_drift(vfps_mesh* in, vfps_mesh* out, const float* slip,
@@ -736,7 +731,8 @@ int vfps_map_update(vfps_map* map)
 
 // DynamicRFKickMap::apply (src/SM/DynamicRFKickMap.cpp:103-111): the RF
 // offsets of the next queue entry (computed on the host in the reference's
-// float arithmetic, staged through pinned memory), then the kick
+// float arithmetic; upload_floats, so the loop does not wait for the step
+// before), then the kick
 static int dynrf_stage(vfps_map* m)
 {
     VFPS_CHECK_ARG((size_t)m->mod_next * 2 < m->modulation.size(),
@@ -752,15 +748,9 @@ static int dynrf_stage(vfps_map* m)
             : rfkick_offsets_at(ps->ax0, ps->ax1, m->rf_revolutionpart,
                                 m->rf_V, m->rf_f, m->rf_V0, ps->qscale,
                                 (float)ps->pscale, phase, ampl);
-    hipStream_t st = ps->dev->stream;
-    // the previous upload from the staging buffer has finished reading it
-    VFPS_HIP(hipEventSynchronize(m->stage_done));
-    std::memcpy(m->stage_h, off.data(), sizeof(float) * off.size());
-    VFPS_HIP(hipMemcpyAsync(m->offset, m->stage_h, sizeof(float) * off.size(),
-                            hipMemcpyHostToDevice, st));
-    VFPS_HIP(hipEventRecord(m->stage_done, st));
-    m->mod_next++;
-    return VFPS_OK;
+    const int rc = upload_floats(ps->dev, m->offset, off.data(), off.size());
+    if (rc == VFPS_OK) m->mod_next++;
+    return rc;
 }
 
 int vfps_map_apply(vfps_map* map)
@@ -801,15 +791,6 @@ static int dynrf_create(vfps_mesh* in, vfps_mesh* out, bool linear,
     m->modulation = dynrf_modulation(steps, seed, m->rf_syncphase,
                                      revolutionpart, phasespread,
                                      amplspread, modampl, modtimeincrement);
-    if (hipHostMalloc(&m->stage_h, sizeof(float) * in->n,
-                      hipHostMallocDefault) != hipSuccess ||
-        hipEventCreateWithFlags(&m->stage_done, hipEventDisableTiming) !=
-            hipSuccess) {
-        vfps_map_destroy(m);
-        *map = nullptr;
-        return fail(VFPS_ERR_NOMEM, "DynamicRFKickMap: staging buffer");
-    }
-    VFPS_HIP(hipEventRecord(m->stage_done, in->dev->stream));
     // the static RF kick of the constructor (RFKickMap::_calcKick(_syncphase))
     const auto off =
         linear ? rfkick_offsets_linear(in->ax0, angle, in->qscale, f_RF)
@@ -883,11 +864,6 @@ int vfps_map_destroy(vfps_map* map)
     hipFree(map->offset);
     hipFree(map->fp_w);
     hipFree(map->fp_i);
-    if (map->stage_done) {
-        hipEventSynchronize(map->stage_done);
-        hipEventDestroy(map->stage_done);
-    }
-    if (map->stage_h) hipHostFree(map->stage_h);
     delete map;
     return VFPS_OK;
 }

@@ -154,6 +154,11 @@ int launch_wake_potential(vfps_field* f, float* dst);
 // updateXProjection / integrate on a mesh (runtime.hip)
 int launch_project_x(vfps_mesh* m, const float* src, float* proj);
 int launch_integrate(vfps_mesh* m);
+// y projection, charge integral, mean/variance/root of both projections
+// (mom[6]) and both projections of a one-bunch mesh (src/main.cpp:961-967),
+// on the host
+int mesh_moments(vfps_mesh* m, float* xproj, float* yproj, double* fill,
+                 float* mom);
 
 // constructor tables
 std::vector<float> drift_offsets(const Ruler& ax0, const Ruler& ax1,

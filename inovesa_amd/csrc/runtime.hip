@@ -193,48 +193,88 @@ project_x_kernel(uint32_t rows, uint32_t n, uint32_t rows_per_wg,
 }
 
 // updateYProjection (src/PS/PhaseSpace.cpp:325-340): for each column y,
-// proj[y] = proj[y] + data[x][y]*ws[x] for x = 0..n-1 in order.  A
-// workgroup takes 64 columns of one bunch, lane y of wave 0 their sums;
-// the other waves stage chunks of PY_ROWS rows (the products) into a
-// double buffer in LDS, one chunk ahead of the sums.
-constexpr uint32_t PY_COLS = 64;
-constexpr uint32_t PY_ROWS = 64;
+// proj[y] = proj[y] + data[x][y]*ws[x] for x = 0..n-1 in order.  A workgroup
+// takes 16 columns of one bunch: its threads load up to PY_ROWS rows of them,
+// all in flight at once, and store the products column by column to LDS
+// (PY_ROWS + 4 words apart); then a lane per column adds them in order, 16
+// bytes a load.  The bound is those dependent additions.  (64 columns a
+// workgroup, one word a load, took 51 us at 512^2; the outstep moments of a
+// step there went from 200 to 36 us with this and moments_kernel.)
+constexpr uint32_t PY_COLS = 16;
+constexpr uint32_t PY_ROWS = 512;
 constexpr uint32_t PY_THREADS = 256;
+constexpr uint32_t PY_STRIDE = PY_ROWS + 4;
 
 __global__ void __launch_bounds__(PY_THREADS)
 project_y_kernel(uint32_t nb, uint32_t n, const float* __restrict__ data,
                  const float* __restrict__ ws, float* __restrict__ proj)
 {
-    __shared__ float buf[2][PY_ROWS][PY_COLS + 1];
+    __shared__ __align__(16) float buf[PY_COLS * PY_STRIDE];
     const uint32_t b = blockIdx.y;
     const uint32_t c0 = blockIdx.x * PY_COLS;
     const uint32_t ncol = min(PY_COLS, n - c0);
-    const float* d = data + (size_t)b * n * n;
-    const uint32_t tid = threadIdx.x, wave = tid >> 6;
-    const uint32_t nchunks = (n + PY_ROWS - 1) / PY_ROWS;
-    // stage chunk k by the threads [t0, t0 + nt)
-    auto stage = [&](uint32_t k, uint32_t t0, uint32_t nt) {
-        const uint32_t x0 = k * PY_ROWS;
+    const float* d = data + (size_t)b * n * n + c0;
+    const uint32_t tid = threadIdx.x;
+    float acc = 0.0f;
+    for (uint32_t x0 = 0; x0 < n; x0 += PY_ROWS) {
         const uint32_t nr = min(PY_ROWS, n - x0);
-        float(*dst)[PY_COLS + 1] = buf[k & 1u];
-        for (uint32_t i = tid - t0; i < nr * PY_COLS; i += nt) {
-            const uint32_t r = i / PY_COLS, c = i % PY_COLS;
-            if (c < ncol) {
-                dst[r][c] = d[(size_t)(x0 + r) * n + c0 + c] * ws[x0 + r];
+        const uint32_t np = (nr + 15u) & ~15u;  // filled up with +0
+        if ((n & 3u) == 0u) {
+            // four columns a load; a load past the last row or column reads
+            // the strip's first words instead
+            constexpr uint32_t LOADS = PY_ROWS * PY_COLS / 4 / PY_THREADS;
+            const uint32_t cg = (tid & 3u) * 4u, r0 = tid >> 2;
+            const bool col = cg < ncol;
+            float4 v[LOADS];
+            float w[LOADS];
+#pragma unroll
+            for (uint32_t k = 0; k < LOADS; k++) {
+                const uint32_t r = r0 + k * (PY_THREADS / 4);
+                const bool in = col && r < nr;
+                v[k] = *reinterpret_cast<const float4*>(
+                    d + (in ? (size_t)(x0 + r) * n + cg : 0u));
+                w[k] = ws[x0 + (r < nr ? r : 0u)];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < LOADS; k++) {
+                const uint32_t r = r0 + k * (PY_THREADS / 4);
+                if (r < np) {
+                    const bool in = r < nr;
+                    float* o = buf + cg * PY_STRIDE + r;
+                    o[0] = in ? v[k].x * w[k] : 0.0f;
+                    o[PY_STRIDE] = in ? v[k].y * w[k] : 0.0f;
+                    o[2 * PY_STRIDE] = in ? v[k].z * w[k] : 0.0f;
+                    o[3 * PY_STRIDE] = in ? v[k].w * w[k] : 0.0f;
+                }
+            }
+        } else {
+            for (uint32_t i = tid; i < np * PY_COLS; i += PY_THREADS) {
+                const uint32_t r = i / PY_COLS, c = i % PY_COLS;
+                buf[c * PY_STRIDE + r] =
+                    r < nr && c < ncol ? d[(size_t)(x0 + r) * n + c] * ws[x0 + r]
+                                       : 0.0f;
             }
         }
-    };
-    stage(0, 0, blockDim.x);
-    __syncthreads();
-    float acc = 0.0f;
-    for (uint32_t k = 0; k < nchunks; k++) {
-        if (wave != 0) {
-            if (k + 1 < nchunks) stage(k + 1, 64, blockDim.x - 64);
-        } else if (tid < ncol) {
-            const uint32_t nr = min(PY_ROWS, n - k * PY_ROWS);
-            float(*src)[PY_COLS + 1] = buf[k & 1u];
-            for (uint32_t r = 0; r < nr; r++) {
-                acc = acc + src[r][tid];
+        __syncthreads();
+        if (tid < ncol) {
+            const float4* p4 =
+                reinterpret_cast<const float4*>(buf + tid * PY_STRIDE);
+            float4 q[4], nq[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) q[k] = p4[k];
+            for (uint32_t y = 0; y < np; y += 16) {
+                const uint32_t yn = y + 16 < np ? y + 16 : y;
+#pragma unroll
+                for (int k = 0; k < 4; k++) nq[k] = p4[(yn >> 2) + k];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    acc = acc + q[k].x;
+                    acc = acc + q[k].y;
+                    acc = acc + q[k].z;
+                    acc = acc + q[k].w;
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++) q[k] = nq[k];
             }
         }
         __syncthreads();
@@ -244,27 +284,37 @@ project_y_kernel(uint32_t nb, uint32_t n, const float* __restrict__ data,
     }
 }
 
-// integrate (src/PS/PhaseSpace.cpp:200-239), FP64 accumulation
-__global__ void integrate_kernel(uint32_t nb, uint32_t n, const float* proj,
-                                 const float* ws, double* filling,
-                                 double* integral)
+// charge integral of one bunch's x projection (src/PS/PhaseSpace.cpp:200-239),
+// FP64; every thread of the workgroup receives it
+__device__ __forceinline__ double filling_of(uint32_t n, const float* proj,
+                                             const float* ws, double* part)
+{
+    double acc = 0.0;
+    for (uint32_t x = threadIdx.x; x < n; x += blockDim.x) {
+        acc += (double)proj[x] * (double)ws[x];
+    }
+    return block_sum(acc, part);
+}
+
+// out (optional, pinned): the fillings and the integral
+__global__ void __launch_bounds__(256)
+integrate_kernel(uint32_t nb, uint32_t n, const float* proj, const float* ws,
+                 double* filling, double* integral, double* out)
 {
     __shared__ double part[16];
     double total = 0.0;
     for (uint32_t b = 0; b < nb; b++) {
-        double acc = 0.0;
-        for (uint32_t x = threadIdx.x; x < n; x += blockDim.x) {
-            acc += (double)proj[(size_t)b * n + x] * (double)ws[x];
-        }
-        acc = block_sum(acc, part);
+        const double acc = filling_of(n, proj + (size_t)b * n, ws, part);
         if (threadIdx.x == 0) {
             filling[b] = acc;
+            if (out) out[b] = acc;
         }
         total += acc;
         __syncthreads();
     }
     if (threadIdx.x == 0) {
         *integral = total;
+        if (out) out[nb] = total;
     }
 }
 
@@ -286,35 +336,96 @@ __global__ void normalize_kernel(uint32_t nb, size_t nxy, float* data,
     }
 }
 
-// average + variance (src/PS/PhaseSpace.cpp:241-289), FP64 accumulation;
-// one block per bunch
-__global__ void variance_kernel(uint32_t n, const float* proj,
-                                const float* axis, float delta,
-                                const float* fill_set, const double* filling,
-                                float* out)
+// average, variance and its root (src/PS/PhaseSpace.cpp:241-289) of one
+// projection, FP64 accumulation; out[3] written by thread 0.  The axis is the
+// Ruler's: min + i delta.
+__device__ __forceinline__ void variance_of(uint32_t n, const float* p,
+                                            float axis_min, float delta,
+                                            bool filled, double filling,
+                                            double* part, float* out)
 {
-    __shared__ double part[16];
-    const uint32_t b = blockIdx.x;
-    const float* p = proj + (size_t)b * n;
-    const bool filled = fill_set[b] > 0.0f;
     double avg = 0.0;
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-        avg += (double)p[i] * (double)axis[i];
+        avg += (double)p[i] * (double)(axis_min + ((float)i * delta));
     }
     avg = block_sum(avg, part);
-    float favg = filled ? (float)(avg * ((double)delta / filling[b])) : 0.0f;
-    __syncthreads();
+    float favg = filled ? (float)(avg * ((double)delta / filling)) : 0.0f;
     double var = 0.0;
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-        double d = (double)(axis[i] - favg);
+        double d = (double)((axis_min + ((float)i * delta)) - favg);
         var += (double)p[i] * d * d;
     }
     var = block_sum(var, part);
     if (threadIdx.x == 0) {
-        float fvar = filled ? (float)(var * ((double)delta / filling[b])) : 0.0f;
-        out[3 * b + 0] = favg;
-        out[3 * b + 1] = fvar;
-        out[3 * b + 2] = sqrtf(fvar);
+        float fvar = filled ? (float)(var * ((double)delta / filling)) : 0.0f;
+        out[0] = favg;
+        out[1] = fvar;
+        out[2] = sqrtf(fvar);
+    }
+}
+
+// one workgroup per bunch; out: [nb][3], pinned
+__global__ void __launch_bounds__(256)
+variance_kernel(uint32_t n, const float* proj, float axis_min, float delta,
+                const float* fill_set, const double* filling, float* out)
+{
+    __shared__ double part[16];
+    const uint32_t b = blockIdx.x;
+    variance_of(n, proj + (size_t)b * n, axis_min, delta, fill_set[b] > 0.0f,
+                filling[b], part, out + 3 * b);
+}
+
+// The outstep quantities of a one-bunch mesh from its projections
+// (proj: x, then y), into pinned memory: the FP64 charge integral, then
+// 2 x (mean, variance, root), then both projections.  The same sums as
+// integrate_kernel and variance_kernel make, in one launch.
+__global__ void __launch_bounds__(256)
+moments_kernel(uint32_t n, const float* proj, const float* ws, float min0,
+               float delta0, float min1, float delta1, const float* fill_set,
+               double* filling, double* integral, double* out)
+{
+    __shared__ double part[16];
+    float* of = reinterpret_cast<float*>(out + 1);
+    for (uint32_t i = threadIdx.x; i < 2 * n; i += blockDim.x) {
+        of[6 + i] = proj[i];
+    }
+    const double f = filling_of(n, proj, ws, part);
+    if (threadIdx.x == 0) {
+        *filling = f;
+        *integral = f;
+        out[0] = f;
+    }
+    const bool filled = fill_set[0] > 0.0f;
+    variance_of(n, proj, min0, delta0, filled, f, part, of);
+    variance_of(n, proj + n, min1, delta1, filled, f, part, of + 3);
+}
+
+struct UploadArgs {
+    float v[UPLOAD_ARGS];
+};
+
+__global__ void __launch_bounds__(256)
+upload_kernel(UploadArgs a, float* dst, uint32_t n)
+{
+    for (uint32_t i = threadIdx.x; i < n; i += 256u) {
+        dst[i] = a.v[i];
+    }
+}
+
+struct ReadBackArgs {
+    const uint32_t* src[READ_BACK_ARRAYS];
+    uint32_t words[READ_BACK_ARRAYS];
+};
+
+__global__ void __launch_bounds__(256)
+read_back_kernel(ReadBackArgs a, uint32_t* out)
+{
+    for (uint32_t k = 0; k < READ_BACK_ARRAYS; k++) {
+        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < a.words[k];
+             i += gridDim.x * 256u) {
+            out[i] = a.src[k][i];
+        }
+        out += a.words[k];
     }
 }
 
@@ -346,8 +457,90 @@ int launch_project_x(vfps_mesh* m, const float* src, float* proj)
 int launch_integrate(vfps_mesh* m)
 {
     hipLaunchKernelGGL(integrate_kernel, dim3(1), dim3(256), 0, m->dev->stream,
-                       m->nb, m->n, m->proj, m->ws, m->filling, m->integral);
+                       m->nb, m->n, m->proj, m->ws, m->filling, m->integral,
+                       (double*)nullptr);
     VFPS_HIP(hipGetLastError());
+    return VFPS_OK;
+}
+
+int read_back(vfps_dev* dev, const ReadBack* arrays, size_t count)
+{
+    hipStream_t st = dev->stream;
+    size_t bytes = 0;
+    for (size_t k = 0; k < count; k++) bytes += arrays[k].bytes;
+    DevStage stage(dev);
+    char* buf = bytes <= READ_BACK_MAX && count <= READ_BACK_ARRAYS
+                    ? stage.get<char>()
+                    : nullptr;
+    if (!buf) {
+        for (size_t k = 0; k < count; k++) {
+            VFPS_HIP(hipMemcpyAsync(arrays[k].dst, arrays[k].src,
+                                    arrays[k].bytes, hipMemcpyDeviceToHost, st));
+        }
+        VFPS_HIP(hipStreamSynchronize(st));
+        return VFPS_OK;
+    }
+    ReadBackArgs a{};
+    for (size_t k = 0; k < count; k++) {
+        a.src[k] = static_cast<const uint32_t*>(arrays[k].src);
+        a.words[k] = (uint32_t)(arrays[k].bytes / 4u);
+    }
+    hipLaunchKernelGGL(read_back_kernel,
+                       dim3(std::max(1u, std::min(32u, ceil_div(bytes, 1024u)))),
+                       dim3(256), 0, st, a, reinterpret_cast<uint32_t*>(buf));
+    VFPS_HIP(hipGetLastError());
+    VFPS_HIP(hipStreamSynchronize(st));
+    for (size_t k = 0; k < count; k++) {
+        std::memcpy(arrays[k].dst, buf, arrays[k].bytes);
+        buf += arrays[k].bytes;
+    }
+    return VFPS_OK;
+}
+
+int upload_floats(vfps_dev* dev, float* dst, const float* src, size_t n)
+{
+    hipStream_t st = dev->stream;
+    if (n > UPLOAD_MAX) {
+        VFPS_HIP(hipMemcpyAsync(dst, src, sizeof(float) * n,
+                                hipMemcpyHostToDevice, st));
+        VFPS_HIP(hipStreamSynchronize(st));
+        return VFPS_OK;
+    }
+    UploadArgs a;
+    for (size_t i = 0; i < n; i += UPLOAD_ARGS) {
+        const size_t k = std::min(UPLOAD_ARGS, n - i);
+        std::memcpy(a.v, src + i, sizeof(float) * k);
+        hipLaunchKernelGGL(upload_kernel, dim3(1), dim3(256), 0, st, a, dst + i,
+                           (uint32_t)k);
+    }
+    VFPS_HIP(hipGetLastError());
+    return VFPS_OK;
+}
+
+int mesh_moments(vfps_mesh* m, float* xproj, float* yproj, double* fill,
+                 float* mom)
+{
+    const uint32_t n = m->n;
+    VFPS_CHECK_ARG(m->nb == 1 && sizeof(double) + sizeof(float) * (6 + 2 * (size_t)n) <=
+                                     DEV_STAGE_BYTES,
+                   "moments: one bunch");
+    int rc = vfps_mesh_project_y(m);
+    if (rc != VFPS_OK) return rc;
+    DevStage stage(m->dev);
+    double* out = stage.get<double>();
+    if (!out) return fail(VFPS_ERR_NOMEM, "moments: pinned memory");
+    hipStream_t st = m->dev->stream;
+    hipLaunchKernelGGL(moments_kernel, dim3(1), dim3(256), 0, st, n, m->proj,
+                       m->ws, m->ax0.min, m->ax0.delta, m->ax1.min,
+                       m->ax1.delta, m->fill_set_d, m->filling, m->integral,
+                       out);
+    VFPS_HIP(hipGetLastError());
+    VFPS_HIP(hipStreamSynchronize(st));
+    const float* of = reinterpret_cast<const float*>(out + 1);
+    *fill = out[0];
+    std::memcpy(mom, of, 6 * sizeof(float));
+    if (xproj) std::memcpy(xproj, of + 6, sizeof(float) * n);
+    if (yproj) std::memcpy(yproj, of + 6 + n, sizeof(float) * n);
     return VFPS_OK;
 }
 
@@ -617,43 +810,52 @@ int vfps_mesh_get_projection(vfps_mesh* m, int axis, float* out)
 {
     VFPS_CHECK_ARG(m && out && (axis == 0 || axis == 1),
                    "vfps_mesh_get_projection: bad argument");
-    VFPS_HIP(hipMemcpyAsync(out, m->proj + (size_t)axis * m->nb * m->n,
-                            sizeof(float) * m->nb * m->n,
-                            hipMemcpyDeviceToHost, m->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(m->dev->stream));
-    return VFPS_OK;
+    const ReadBack r{out, m->proj + (size_t)axis * m->nb * m->n,
+                     sizeof(float) * m->nb * m->n};
+    return read_back(m->dev, &r, 1);
 }
 
 int vfps_mesh_set_projection(vfps_mesh* m, int axis, const float* proj)
 {
     VFPS_CHECK_ARG(m && proj && (axis == 0 || axis == 1),
                    "vfps_mesh_set_projection: bad argument");
-    VFPS_HIP(hipMemcpyAsync(m->proj + (size_t)axis * m->nb * m->n, proj,
-                            sizeof(float) * m->nb * m->n,
-                            hipMemcpyHostToDevice, m->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(m->dev->stream));
-    return VFPS_OK;
+    return upload_floats(m->dev, m->proj + (size_t)axis * m->nb * m->n, proj,
+                         (size_t)m->nb * m->n);
 }
 
 int vfps_mesh_integrate(vfps_mesh* m, double* filling, double* integral)
 {
     VFPS_CHECK_ARG(m, "vfps_mesh_integrate: NULL mesh");
-    int rc = launch_integrate(m);
-    if (rc != VFPS_OK) {
-        return rc;
+    if (!filling && !integral) {
+        return launch_integrate(m);
     }
-    if (filling) {
-        VFPS_HIP(hipMemcpyAsync(filling, m->filling, sizeof(double) * m->nb,
-                                hipMemcpyDeviceToHost, m->dev->stream));
+    VFPS_TRY_BEGIN
+    DevStage stage(m->dev);
+    double* out = sizeof(double) * ((size_t)m->nb + 1) <= DEV_STAGE_BYTES
+                      ? stage.get<double>()
+                      : nullptr;
+    hipStream_t st = m->dev->stream;
+    hipLaunchKernelGGL(integrate_kernel, dim3(1), dim3(256), 0, st, m->nb,
+                       m->n, m->proj, m->ws, m->filling, m->integral, out);
+    VFPS_HIP(hipGetLastError());
+    if (!out) {
+        // (no pinned memory: copies)
+        if (filling) {
+            VFPS_HIP(hipMemcpyAsync(filling, m->filling, sizeof(double) * m->nb,
+                                    hipMemcpyDeviceToHost, st));
+        }
+        if (integral) {
+            VFPS_HIP(hipMemcpyAsync(integral, m->integral, sizeof(double),
+                                    hipMemcpyDeviceToHost, st));
+        }
     }
-    if (integral) {
-        VFPS_HIP(hipMemcpyAsync(integral, m->integral, sizeof(double),
-                                hipMemcpyDeviceToHost, m->dev->stream));
-    }
-    if (filling || integral) {
-        VFPS_HIP(hipStreamSynchronize(m->dev->stream));
+    VFPS_HIP(hipStreamSynchronize(st));
+    if (out) {
+        if (filling) std::memcpy(filling, out, sizeof(double) * m->nb);
+        if (integral) *integral = out[m->nb];
     }
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 int vfps_mesh_normalize(vfps_mesh* m)
@@ -674,22 +876,16 @@ int vfps_mesh_variance(vfps_mesh* m, int axis, float* mean, float* var,
                    "vfps_mesh_variance: bad argument");
     VFPS_TRY_BEGIN
     const Ruler& ax = axis == 0 ? m->ax0 : m->ax1;
-    float* tmp = nullptr;
-    VFPS_HIP(hipMalloc(&tmp, sizeof(float) * (m->n + 3 * m->nb)));
-    hipMemcpyAsync(tmp, ax.data.data(), sizeof(float) * m->n,
-                   hipMemcpyHostToDevice, m->dev->stream);
+    DevStage stage(m->dev);
+    const size_t bytes = sizeof(float) * 3 * (size_t)m->nb;
+    float* h = bytes <= DEV_STAGE_BYTES ? stage.get<float>() : nullptr;
+    if (!h) return fail(VFPS_ERR_NOMEM, "variance: pinned memory");
     hipLaunchKernelGGL(variance_kernel, dim3(m->nb), dim3(256), 0,
                        m->dev->stream, m->n,
-                       m->proj + (size_t)axis * m->nb * m->n, tmp, ax.delta,
-                       m->fill_set_d, m->filling, tmp + m->n);
-    std::vector<float> h(3 * m->nb);
-    hipMemcpyAsync(h.data(), tmp + m->n, sizeof(float) * 3 * m->nb,
-                   hipMemcpyDeviceToHost, m->dev->stream);
-    hipError_t e = hipStreamSynchronize(m->dev->stream);
-    hipFree(tmp);
-    if (e != hipSuccess) {
-        return fail(VFPS_ERR_HIP, hipGetErrorString(e));
-    }
+                       m->proj + (size_t)axis * m->nb * m->n, ax.min, ax.delta,
+                       m->fill_set_d, m->filling, h);
+    VFPS_HIP(hipGetLastError());
+    VFPS_HIP(hipStreamSynchronize(m->dev->stream));
     for (uint32_t b = 0; b < m->nb; b++) {
         if (mean) mean[b] = h[3 * b];
         if (var) var[b] = h[3 * b + 1];

@@ -1126,16 +1126,28 @@ int vfps_step_get_history(vfps_step* s, uint32_t* count, float* csr_power,
                           float* profiles)
 {
     VFPS_CHECK_ARG(s, "vfps_step_get_history: NULL step");
-    VFPS_HIP(hipStreamSynchronize(s->dev->stream));
     uint32_t c = 0;
     const uint32_t at = s->fused ? (s->parity & 1u) : 0u;
-    VFPS_HIP(hipMemcpy(&c, s->counter + at, sizeof(uint32_t),
-                       hipMemcpyDeviceToHost));
+    const bool csr = csr_power && s->csr_hist && s->hist_cap;
+    VFPS_TRY_BEGIN
+    // a short history comes with the counter, whole (what lies past the
+    // recorded steps is not handed out)
+    std::vector<float> all(csr && sizeof(float) * s->hist_cap < READ_BACK_MAX
+                               ? s->hist_cap
+                               : 0);
+    ReadBack r[2] = {{&c, s->counter + at, sizeof(uint32_t)},
+                     {all.data(), s->csr_hist, sizeof(float) * all.size()}};
+    int rc = read_back(s->dev, r, all.empty() ? 1 : 2);
+    if (rc != VFPS_OK) return rc;
     c = std::min(c, s->hist_cap);
     if (count) *count = c;
-    if (csr_power && s->csr_hist && c) {
-        VFPS_HIP(hipMemcpy(csr_power, s->csr_hist, sizeof(float) * c,
-                           hipMemcpyDeviceToHost));
+    if (csr && c) {
+        if (!all.empty()) {
+            std::copy(all.begin(), all.begin() + c, csr_power);
+        } else {
+            VFPS_HIP(hipMemcpy(csr_power, s->csr_hist, sizeof(float) * c,
+                               hipMemcpyDeviceToHost));
+        }
     }
     if (profiles && s->prof_hist && c) {
         VFPS_HIP(hipMemcpy(profiles, s->prof_hist,
@@ -1143,6 +1155,7 @@ int vfps_step_get_history(vfps_step* s, uint32_t* count, float* csr_power,
                            hipMemcpyDeviceToHost));
     }
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 int vfps_step_get_mesh(vfps_step* s, float* mesh, float* proj, float* wake)
@@ -1156,19 +1169,12 @@ int vfps_step_get_mesh(vfps_step* s, float* mesh, float* proj, float* wake)
         VFPS_HIP(hipMemcpy(mesh, cur->data, sizeof(float) * n * n,
                            hipMemcpyDeviceToHost));
     }
-    if (proj) {
-        VFPS_HIP(hipMemcpy(proj, cur->proj, sizeof(float) * n,
-                           hipMemcpyDeviceToHost));
-    }
-    if (wake) {
-        if (s->wfield) {
-            VFPS_HIP(hipMemcpy(wake, s->wfield->wake, sizeof(float) * n,
-                               hipMemcpyDeviceToHost));
-        } else {
-            std::fill(wake, wake + n, 0.0f);
-        }
-    }
-    return VFPS_OK;
+    ReadBack r[2];
+    size_t k = 0;
+    if (proj) r[k++] = {proj, cur->proj, sizeof(float) * n};
+    if (wake && s->wfield) r[k++] = {wake, s->wfield->wake, sizeof(float) * n};
+    if (wake && !s->wfield) std::fill(wake, wake + n, 0.0f);
+    return k ? read_back(s->dev, r, k) : VFPS_OK;
 }
 
 int vfps_step_set_particles(vfps_step* s, const float* pos, uint32_t n,
@@ -1234,33 +1240,21 @@ int vfps_step_moments(vfps_step* s, float* xproj, float* yproj,
                       float* average, float* spread)
 {
     VFPS_CHECK_ARG(s, "vfps_step_moments: NULL step");
-    VFPS_HIP(hipStreamSynchronize(s->dev->stream));
     vfps_mesh* cur = (s->fused && (s->parity & 1u)) ? s->t2 : s->t1;
-    double fill = 0.0;
     // src/main.cpp:961-967: integrate(); variance(0); updateYProjection();
     // variance(1)
-    int rc = vfps_mesh_integrate(cur, &fill, nullptr);
+    double fill = 0.0;
+    float mom[6] = {};
+    VFPS_TRY_BEGIN
+    int rc = mesh_moments(cur, xproj, yproj, &fill, mom);
     if (rc != VFPS_OK) return rc;
-    float mean = 0.0f, var = 0.0f, rms = 0.0f;
-    if ((rc = vfps_mesh_variance(cur, 0, &mean, &var, &rms)) != VFPS_OK) {
-        return rc;
-    }
-    if (position) *position = mean;
-    if (length) *length = rms;
-    if ((rc = vfps_mesh_project_y(cur)) != VFPS_OK) return rc;
-    if ((rc = vfps_mesh_variance(cur, 1, &mean, &var, &rms)) != VFPS_OK) {
-        return rc;
-    }
-    if (average) *average = mean;
-    if (spread) *spread = rms;
     if (population) *population = (float)fill;
-    if (xproj && (rc = vfps_mesh_get_projection(cur, 0, xproj)) != VFPS_OK) {
-        return rc;
-    }
-    if (yproj && (rc = vfps_mesh_get_projection(cur, 1, yproj)) != VFPS_OK) {
-        return rc;
-    }
+    if (position) *position = mom[0];
+    if (length) *length = mom[2];
+    if (average) *average = mom[3];
+    if (spread) *spread = mom[5];
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 int vfps_step_set_mesh(vfps_step* s, const float* mesh)
