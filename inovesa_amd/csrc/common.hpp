@@ -128,6 +128,54 @@ constexpr size_t UPLOAD_ARGS = 960;   // floats in the arguments of one launch
 constexpr size_t UPLOAD_MAX = 4 * UPLOAD_ARGS;
 int upload_floats(vfps_dev* dev, float* dst, const float* src, size_t n);
 
+// While a fused step is built, the device arrays of its meshes, field and
+// maps come from one block, whose initial contents are assembled in a host
+// copy (zeros where nothing is put) and uploaded once: about 40 allocations
+// and 30 copies, fills and waits of a few to 10 us each were 0.4 ms of a
+// step's construction, which a scan pays per run.  Outside (the block is
+// null) every array is an allocation and a copy of its own.
+struct StepBlock {
+    char* base = nullptr;
+    size_t used = 0;
+    std::vector<char> host;   // contents of [base, base + host.size())
+    hipError_t take(void** p, size_t bytes)
+    {
+        const size_t at = (used + 255u) & ~(size_t)255u;
+        if (at + bytes > host.size()) return hipErrorOutOfMemory;
+        *p = base + at;
+        used = at + bytes;
+        return hipSuccess;
+    }
+};
+extern thread_local StepBlock* step_block;
+
+template <typename T>
+hipError_t setup_alloc(T** p, size_t count)
+{
+    if (step_block) {
+        return step_block->take(reinterpret_cast<void**>(p), sizeof(T) * count);
+    }
+    return hipMalloc(p, sizeof(T) * count);
+}
+inline hipError_t setup_put(void* dst, const void* src, size_t bytes,
+                            hipStream_t st)
+{
+    if (step_block) {
+        std::memcpy(step_block->host.data() + ((char*)dst - step_block->base),
+                    src, bytes);
+        return hipSuccess;
+    }
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
+}
+inline hipError_t setup_zero(void* dst, size_t bytes, hipStream_t st)
+{
+    return step_block ? hipSuccess : hipMemsetAsync(dst, 0, bytes, st);
+}
+inline hipError_t setup_sync(hipStream_t st)
+{
+    return step_block ? hipSuccess : hipStreamSynchronize(st);
+}
+
 }  // namespace vfps_impl
 
 struct vfps_mesh {
@@ -137,6 +185,7 @@ struct vfps_mesh {
     double qscale = 0, pscale = 0, charge = 0, current = 0;
     std::vector<float> ws_h;         // Simpson weights (host copy)
     std::vector<float> filling_set;  // set bunch populations
+    bool in_block = false;           // device arrays in a step's block
     float* data = nullptr;           // [nb][n][n]
     float* proj = nullptr;           // [2][nb][n]
     float* ws = nullptr;             // [n]
@@ -159,8 +208,10 @@ struct vfps_map {
     vfps_mesh* in = nullptr;
     vfps_mesh* out = nullptr;
     int interp = 4;
+    bool in_block = false;    // device arrays in a step's block
     // kick maps
     float* offset = nullptr;  // device, noff entries
+    std::vector<float> offset_h;  // as constructed (drift, RF kick)
     size_t noff = 0;
     vfps_field* field = nullptr;  // WakePotentialMap
     // rotation
@@ -199,6 +250,7 @@ struct vfps_field {
     vfps_dev* dev = nullptr;
     vfps_mesh* ps = nullptr;
     vfps_impedance* z = nullptr;
+    bool in_block = false;       // device arrays in a step's block
     uint32_t nmax = 0, nb = 0, spacing = 0;
     std::vector<uint32_t> buckets;
     uint32_t* buckets_d = nullptr;

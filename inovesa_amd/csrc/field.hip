@@ -367,32 +367,29 @@ int vfps_field_create(vfps_mesh* ps, vfps_impedance* z,
     f->csr_fc = 0.0f;
     hipError_t e = hipSuccess;
     const uint32_t n = ps->n, nb = ps->nb;
-    e = e ? e : hipMalloc(&f->buckets_d, sizeof(uint32_t) * nb);
-    e = e ? e : hipMalloc(&f->wake, sizeof(float) * nb * n);
-    e = e ? e : hipMalloc(&f->padded, sizeof(float) * nmax);
-    e = e ? e : hipMalloc(&f->wake_padded, sizeof(float) * nmax);
-    e = e ? e : hipMalloc(&f->tw_m, sizeof(double2) * twm.size());
-    e = e ? e : hipMalloc(&f->tw_n, sizeof(double2) * M);
-    e = e ? e : hipMalloc(&f->csr_renorm, sizeof(float) * nmax);
-    e = e ? e : hipMalloc(&f->power, sizeof(float) * nb);
+    f->in_block = step_block != nullptr;
+    e = e ? e : setup_alloc(&f->buckets_d, nb);
+    e = e ? e : setup_alloc(&f->wake, (size_t)nb * n);
+    e = e ? e : setup_alloc(&f->padded, nmax);
+    e = e ? e : setup_alloc(&f->wake_padded, nmax);
+    e = e ? e : setup_alloc(&f->tw_m, twm.size());
+    e = e ? e : setup_alloc(&f->tw_n, M);
+    e = e ? e : setup_alloc(&f->csr_renorm, nmax);
+    e = e ? e : setup_alloc(&f->power, nb);
     if (e != hipSuccess) {
         vfps_field_destroy(f);
         return fail(VFPS_ERR_NOMEM, hipGetErrorString(e));
     }
     hipStream_t st = ps->dev->stream;
-    hipMemcpyAsync(f->buckets_d, buckets, sizeof(uint32_t) * nb,
-                   hipMemcpyHostToDevice, st);
-    hipMemsetAsync(f->wake, 0, sizeof(float) * nb * n, st);
-    hipMemsetAsync(f->padded, 0, sizeof(float) * nmax, st);
-    hipMemsetAsync(f->wake_padded, 0, sizeof(float) * nmax, st);
-    hipMemcpyAsync(f->tw_m, twm.data(), sizeof(double2) * twm.size(),
-                   hipMemcpyHostToDevice, st);
-    hipMemcpyAsync(f->tw_n, twn.data(), sizeof(double2) * M,
-                   hipMemcpyHostToDevice, st);
-    hipMemcpyAsync(f->csr_renorm, renorm.data(), sizeof(float) * nmax,
-                   hipMemcpyHostToDevice, st);
-    hipMemsetAsync(f->power, 0, sizeof(float) * nb, st);
-    e = hipStreamSynchronize(st);
+    setup_put(f->buckets_d, buckets, sizeof(uint32_t) * nb, st);
+    setup_zero(f->wake, sizeof(float) * nb * n, st);
+    setup_zero(f->padded, sizeof(float) * nmax, st);
+    setup_zero(f->wake_padded, sizeof(float) * nmax, st);
+    setup_put(f->tw_m, twm.data(), sizeof(double2) * twm.size(), st);
+    setup_put(f->tw_n, twn.data(), sizeof(double2) * M, st);
+    setup_put(f->csr_renorm, renorm.data(), sizeof(float) * nmax, st);
+    setup_zero(f->power, sizeof(float) * nb, st);
+    e = setup_sync(st);
     if (e != hipSuccess) {
         vfps_field_destroy(f);
         return fail(VFPS_ERR_HIP, hipGetErrorString(e));
@@ -406,15 +403,17 @@ int vfps_field_destroy(vfps_field* f)
 {
     if (!f) return VFPS_OK;
     hipStreamSynchronize(f->dev->stream);
-    hipFree(f->buckets_d);
-    hipFree(f->wake);
-    hipFree(f->padded);
-    hipFree(f->wake_padded);
-    hipFree(f->tw_m);
-    hipFree(f->tw_n);
-    hipFree(f->csr_renorm);
+    if (!f->in_block) {
+        hipFree(f->buckets_d);
+        hipFree(f->wake);
+        hipFree(f->padded);
+        hipFree(f->wake_padded);
+        hipFree(f->tw_m);
+        hipFree(f->tw_n);
+        hipFree(f->csr_renorm);
+        hipFree(f->power);
+    }
     hipFree(f->spectrum);
-    hipFree(f->power);
     delete f;
     return VFPS_OK;
 }

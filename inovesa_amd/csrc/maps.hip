@@ -521,22 +521,24 @@ static int new_kick(vfps_mesh* in, vfps_mesh* out, int interp, int axis,
     m->out = out;
     m->interp = interp;
     m->noff = (size_t)in->n * in->nb;
-    hipError_t e = hipMalloc(&m->offset, sizeof(float) * m->noff);
+    m->in_block = step_block != nullptr;
+    hipError_t e = setup_alloc(&m->offset, m->noff);
     if (e != hipSuccess) {
         delete m;
         return fail(VFPS_ERR_NOMEM, hipGetErrorString(e));
     }
     // _offset is zero-initialised (src/SM/KickMap.cpp:45-47)
-    hipMemsetAsync(m->offset, 0, sizeof(float) * m->noff, in->dev->stream);
+    setup_zero(m->offset, sizeof(float) * m->noff, in->dev->stream);
     *map = m;
     return VFPS_OK;
 }
 
 static int upload_offset(vfps_map* m, const std::vector<float>& off)
 {
-    VFPS_HIP(hipMemcpyAsync(m->offset, off.data(), sizeof(float) * off.size(),
-                            hipMemcpyHostToDevice, m->in->dev->stream));
-    VFPS_HIP(hipStreamSynchronize(m->in->dev->stream));
+    m->offset_h = off;
+    VFPS_HIP(setup_put(m->offset, off.data(), sizeof(float) * off.size(),
+                       m->in->dev->stream));
+    VFPS_HIP(setup_sync(m->in->dev->stream));
     return VFPS_OK;
 }
 
@@ -676,19 +678,18 @@ int vfps_map_create_fokkerplanck(vfps_mesh* in, vfps_mesh* out, int fptype,
     m->ip = ip;
     m->fptrack = fptrack;
     m->fp_e1 = e1;
-    hipError_t e = hipMalloc(&m->fp_w, sizeof(float) * wt.size());
-    if (e == hipSuccess) e = hipMalloc(&m->fp_i, sizeof(uint32_t) * ixt.size());
+    m->in_block = step_block != nullptr;
+    hipError_t e = setup_alloc(&m->fp_w, wt.size());
+    if (e == hipSuccess) e = setup_alloc(&m->fp_i, ixt.size());
     if (e != hipSuccess) {
-        hipFree(m->fp_w);
+        if (!m->in_block) hipFree(m->fp_w);
         delete m;
         return fail(VFPS_ERR_NOMEM, hipGetErrorString(e));
     }
     hipStream_t st = in->dev->stream;
-    hipMemcpyAsync(m->fp_w, wt.data(), sizeof(float) * wt.size(),
-                   hipMemcpyHostToDevice, st);
-    hipMemcpyAsync(m->fp_i, ixt.data(), sizeof(uint32_t) * ixt.size(),
-                   hipMemcpyHostToDevice, st);
-    VFPS_HIP(hipStreamSynchronize(st));
+    setup_put(m->fp_w, wt.data(), sizeof(float) * wt.size(), st);
+    setup_put(m->fp_i, ixt.data(), sizeof(uint32_t) * ixt.size(), st);
+    VFPS_HIP(setup_sync(st));
     *map = m;
     return VFPS_OK;
     VFPS_TRY_END
@@ -861,9 +862,11 @@ int vfps_map_destroy(vfps_map* map)
 {
     if (!map) return VFPS_OK;
     hipStreamSynchronize(map->in->dev->stream);
-    hipFree(map->offset);
-    hipFree(map->fp_w);
-    hipFree(map->fp_i);
+    if (!map->in_block) {
+        hipFree(map->offset);
+        hipFree(map->fp_w);
+        hipFree(map->fp_i);
+    }
     delete map;
     return VFPS_OK;
 }

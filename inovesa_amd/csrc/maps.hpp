@@ -151,6 +151,12 @@ int launch_map(const vfps_map* m, hipStream_t st, const float* in, float* out);
 // WakePotentialMap::update: wake potential of the field into dst (nb*n)
 int launch_wake_potential(vfps_field* f, float* dst);
 
+// a one-bunch mesh of the step being built (its arrays in the step's block,
+// its data at `data`); nothing is launched
+int mesh_in_block(vfps_dev* dev, uint32_t n, float qmin, float qmax,
+                  double qscale, float pmin, float pmax, double pscale,
+                  float* data, vfps_mesh** out);
+
 // updateXProjection / integrate on a mesh (runtime.hip)
 int launch_project_x(vfps_mesh* m, const float* src, float* proj);
 int launch_integrate(vfps_mesh* m);

@@ -10,6 +10,7 @@
 namespace vfps_impl {
 
 static thread_local std::string g_last_error;
+thread_local StepBlock* step_block = nullptr;
 
 void set_error(const std::string& msg) { g_last_error = msg; }
 
@@ -613,12 +614,14 @@ static void mesh_free(vfps_mesh* m)
     if (!m) {
         return;
     }
-    hipFree(m->data);
-    hipFree(m->proj);
-    hipFree(m->ws);
-    hipFree(m->fill_set_d);
-    hipFree(m->filling);
-    hipFree(m->integral);
+    if (!m->in_block) {
+        hipFree(m->data);
+        hipFree(m->proj);
+        hipFree(m->ws);
+        hipFree(m->fill_set_d);
+        hipFree(m->filling);
+        hipFree(m->integral);
+    }
     delete m;
 }
 
@@ -653,23 +656,23 @@ static int mesh_alloc(vfps_dev* dev, uint32_t nb, uint32_t n, float qmin,
     m->filling_set.assign(filling, filling + nb);
     hipSetDevice(dev->ordinal);
     hipError_t e = hipSuccess;
-    e = (e == hipSuccess) ? hipMalloc(&m->data, sizeof(float) * m->cells()) : e;
-    e = (e == hipSuccess) ? hipMalloc(&m->proj, sizeof(float) * 2 * nb * n) : e;
-    e = (e == hipSuccess) ? hipMalloc(&m->ws, sizeof(float) * n) : e;
-    e = (e == hipSuccess) ? hipMalloc(&m->fill_set_d, sizeof(float) * nb) : e;
-    e = (e == hipSuccess) ? hipMalloc(&m->filling, sizeof(double) * nb) : e;
-    e = (e == hipSuccess) ? hipMalloc(&m->integral, sizeof(double)) : e;
+    // (a step's meshes get their data from the step)
+    m->in_block = step_block != nullptr;
+    e = m->in_block ? e : hipMalloc(&m->data, sizeof(float) * m->cells());
+    e = e ? e : setup_alloc(&m->proj, 2 * (size_t)nb * n);
+    e = e ? e : setup_alloc(&m->ws, n);
+    e = e ? e : setup_alloc(&m->fill_set_d, nb);
+    e = e ? e : setup_alloc(&m->filling, nb);
+    e = e ? e : setup_alloc(&m->integral, 1);
     if (e != hipSuccess) {
         mesh_free(m);
         return fail(VFPS_ERR_NOMEM, std::string("PhaseSpace allocation: ") +
                                         hipGetErrorString(e));
     }
-    hipMemsetAsync(m->proj, 0, sizeof(float) * 2 * nb * n, dev->stream);
-    hipMemcpyAsync(m->ws, m->ws_h.data(), sizeof(float) * n,
-                   hipMemcpyHostToDevice, dev->stream);
-    hipMemcpyAsync(m->fill_set_d, filling, sizeof(float) * nb,
-                   hipMemcpyHostToDevice, dev->stream);
-    e = hipStreamSynchronize(dev->stream);
+    setup_zero(m->proj, sizeof(float) * 2 * nb * n, dev->stream);
+    setup_put(m->ws, m->ws_h.data(), sizeof(float) * n, dev->stream);
+    setup_put(m->fill_set_d, filling, sizeof(float) * nb, dev->stream);
+    e = setup_sync(dev->stream);
     if (e != hipSuccess) {
         mesh_free(m);
         return fail(VFPS_ERR_HIP, hipGetErrorString(e));
@@ -677,6 +680,28 @@ static int mesh_alloc(vfps_dev* dev, uint32_t nb, uint32_t n, float qmin,
     *out = m;
     return VFPS_OK;
 }
+
+}  // extern "C"
+
+namespace vfps_impl {
+
+int mesh_in_block(vfps_dev* dev, uint32_t n, float qmin, float qmax,
+                  double qscale, float pmin, float pmax, double pscale,
+                  float* data, vfps_mesh** out)
+{
+    const float one = 1.0f;
+    int rc = mesh_alloc(dev, 1, n, qmin, qmax, qscale, pmin, pmax, pscale, &one,
+                        out);
+    if (rc != VFPS_OK) return rc;
+    (*out)->charge = 1.0;
+    (*out)->current = 1.0;
+    (*out)->data = data;
+    return VFPS_OK;
+}
+
+}  // namespace vfps_impl
+
+extern "C" {
 
 int vfps_mesh_create(vfps_dev* dev, uint32_t nb, uint32_t n, float qmin,
                      float qmax, double qscale, float pmin, float pmax,

@@ -498,21 +498,26 @@ static void step_free(vfps_step* s)
     vfps_mesh_destroy(s->t1);
     vfps_mesh_destroy(s->t2);
     vfps_mesh_destroy(s->t3);
-    hipFree(s->csr_renorm);
-    hipFree(s->csr_tw);
-    hipFree(s->filling);
-    hipFree(s->counter);
-    hipFree(s->err);
     if (s->err_h) hipHostFree(s->err_h);
     hipFree(s->csr_hist);
     hipFree(s->prof_hist);
-    hipFree(s->wake_g);
-    hipFree(s->csr_h);
-    hipFree(s->csr_part);
-    hipFree(s->csr_valid);
-    hipFree(s->csr_power);
-    hipFree(s->inst_d);
-    hipFree(s->fparams_d);
+    if (s->block) {
+        // the meshes', maps' and step's arrays
+        hipFree(s->block);
+    } else {
+        hipFree(s->csr_renorm);
+        hipFree(s->csr_tw);
+        hipFree(s->filling);
+        hipFree(s->counter);
+        hipFree(s->err);
+        hipFree(s->wake_g);
+        hipFree(s->csr_h);
+        hipFree(s->csr_part);
+        hipFree(s->csr_valid);
+        hipFree(s->csr_power);
+        hipFree(s->inst_d);
+        hipFree(s->fparams_d);
+    }
     delete s;
 }
 
@@ -555,10 +560,7 @@ static int step_upload_desc(vfps_step* s)
     // the halo depends on the maps only: computed once
     if (!s->halo_valid) {
         if (s->desc.scheme == 0) {
-            std::vector<float> off(t1->n);
-            VFPS_HIP(hipMemcpy(off.data(), s->drm->offset, sizeof(float) * t1->n,
-                               hipMemcpyDeviceToHost));
-            kick_halo(off, t1->n, s->desc.interp, &s->halo_lo, &s->halo_hi);
+            kick_halo(s->drm->offset_h, t1->n, s->desc.interp, &s->halo_lo, &s->halo_hi);
         } else {
             rotation_halo(d.rot, t1->n, s->desc.interp, &s->halo_lo, &s->halo_hi);
         }
@@ -696,34 +698,71 @@ static int step_graph(vfps_step* s, uint32_t steps, uint32_t p, bool fin,
     return VFPS_OK;
 }
 
-// Toeplitz tables and scratch of the direct wake / CSR forms
+// arrays of the direct wake / CSR forms
+static int step_alloc_direct(vfps_step* s)
+{
+    const size_t n = s->desc.n, nd = 2 * n - 1;
+    hipStream_t st = s->dev->stream;
+    if (s->desc.use_wake) VFPS_HIP(setup_alloc(&s->wake_g, nd));
+    if (s->desc.use_csr) VFPS_HIP(setup_alloc(&s->csr_h, nd));
+    const uint32_t none[2] = {0xFFFFFFFFu, 0xFFFFFFFFu};
+    VFPS_HIP(setup_alloc(&s->csr_part, 2 * n));
+    VFPS_HIP(setup_alloc(&s->csr_valid, 2));
+    VFPS_HIP(setup_zero(s->csr_part, sizeof(double) * 2 * n, st));
+    VFPS_HIP(setup_put(s->csr_valid, none, sizeof(none), st));
+    return VFPS_OK;
+}
+
+// their Toeplitz tables, in stream order after the uploads they read
 static int step_setup_direct(vfps_step* s)
 {
     const uint32_t n = s->desc.n;
-    const uint32_t M = s->M;
     const bool wake = s->desc.use_wake != 0, csr = s->desc.use_csr != 0;
-    const size_t nd = 2 * (size_t)n - 1;
-    if (wake) VFPS_HIP(hipMalloc(&s->wake_g, sizeof(double) * nd));
-    if (csr) VFPS_HIP(hipMalloc(&s->csr_h, sizeof(double) * nd));
-    if (wake || csr) {
-        // impedances of another handle: its stream may still be at them
-        for (const vfps_impedance* z : {s->zwake, s->zcsr}) {
-            if (z && z->dev != s->dev) {
-                VFPS_HIP(hipStreamSynchronize(z->dev->stream));
-            }
+    if (!wake && !csr) return VFPS_OK;
+    // impedances of another handle: its stream may still be at them
+    for (const vfps_impedance* z : {s->zwake, s->zcsr}) {
+        if (z && z->dev != s->dev) {
+            VFPS_HIP(hipStreamSynchronize(z->dev->stream));
         }
-        hipLaunchKernelGGL(toeplitz_kernel, dim3((uint32_t)nd), dim3(256), 0,
-                           s->dev->stream, n, M, wake ? s->zwake->z : nullptr,
-                           csr ? s->zcsr->z : nullptr, s->csr_renorm,
-                           s->csr_fdelta,
-                           wake ? s->wfield->tw_n : s->csr_tw + s->csr_tw_m,
-                           s->wake_g, s->csr_h);
-        VFPS_HIP(hipGetLastError());
     }
-    VFPS_HIP(hipMalloc(&s->csr_part, sizeof(double) * 2 * n));
-    VFPS_HIP(hipMemset(s->csr_part, 0, sizeof(double) * 2 * n));
-    VFPS_HIP(hipMalloc(&s->csr_valid, sizeof(uint32_t) * 2));
-    VFPS_HIP(hipMemset(s->csr_valid, 0xFF, sizeof(uint32_t) * 2));
+    hipLaunchKernelGGL(toeplitz_kernel, dim3(2 * n - 1), dim3(256), 0,
+                       s->dev->stream, n, s->M, wake ? s->zwake->z : nullptr,
+                       csr ? s->zcsr->z : nullptr, s->csr_renorm, s->csr_fdelta,
+                       wake ? s->wfield->tw_n : s->csr_tw + s->csr_tw_m,
+                       s->wake_g, s->csr_h);
+    VFPS_HIP(hipGetLastError());
+    return VFPS_OK;
+}
+
+// Bytes of the block of a fused step (StepBlock): at least what its arrays
+// take, each from a 256-byte boundary.
+static size_t step_block_bytes(size_t n, size_t nmax)
+{
+    const size_t M = nmax / 2;
+    const size_t tw = fft_pow2((uint32_t)M) ? M : chirp_table((uint32_t)M);
+    const size_t mesh = sizeof(float) * (3 * n + 1) + 2 * sizeof(double);
+    const size_t field = sizeof(float) * (n + 3 * nmax + 2) +
+                         sizeof(double2) * (tw + M);
+    const size_t maps = sizeof(float) * (3 * n + 2 * 5 * n);
+    const size_t step = sizeof(float) * nmax + sizeof(double2) * (tw + M) +
+                        sizeof(double) * (2 * (2 * n - 1) + 2 * n + 4) +
+                        sizeof(InstDesc) + sizeof(FieldParams) + 64;
+    return 3 * mesh + field + maps + step + 64 * 256;
+}
+
+// step_block for the duration of a scope
+struct BlockScope {
+    explicit BlockScope(StepBlock* b) { step_block = b; }
+    ~BlockScope() { step_block = nullptr; }
+};
+
+// the pinned copy of the error flag a run returns with
+static int step_err_flag(vfps_step* s)
+{
+    if (!s->err_h) {
+        VFPS_HIP(hipHostMalloc(&s->err_h, sizeof(uint32_t), hipHostMallocDefault));
+        *s->err_h = 0;
+    }
     return VFPS_OK;
 }
 
@@ -852,6 +891,7 @@ int vfps_step_create(vfps_dev* dev, const vfps_step_desc* desc,
                        (desc->threads % 64 == 0 && desc->threads <= STEP_MAX_THREADS),
                    "vfps_step_create: threads must be a multiple of 64 up to 512");
     VFPS_TRY_BEGIN
+    StepBlock blk;  // (outlives the step if its construction fails)
     auto* s = new vfps_step();
     std::unique_ptr<vfps_step, void (*)(vfps_step*)> guard(s, step_free);
     s->dev = dev;
@@ -866,13 +906,40 @@ int vfps_step_create(vfps_dev* dev, const vfps_step_desc* desc,
     const uint32_t n = desc->n;
     const float one = 1.0f;
     int rc;
-    // three grids (src/main.cpp:470-535)
-    rc = vfps_mesh_create(dev, 1, n, desc->qmin, desc->qmax, desc->qscale,
-                          desc->pmin, desc->pmax, desc->pscale, 1.0, 1.0,
-                          &one, 1.0, init, &s->t1);
-    if (rc != VFPS_OK) return rc;
-    if ((rc = vfps_mesh_clone(s->t1, &s->t2)) != VFPS_OK) return rc;
-    if ((rc = vfps_mesh_clone(s->t1, &s->t3)) != VFPS_OK) return rc;
+    VFPS_HIP(hipSetDevice(dev->ordinal));
+    // three grids (src/main.cpp:470-535); the fused step uses two
+    BlockScope scope(nullptr);
+    const size_t cells = (size_t)n * n;
+    if (s->fused && n >= 3 && n <= STEP_MAX_THREADS * STEP_MAX_COLS) {
+        const uint32_t nmax = std::min(
+            8192u, std::max({4u, zwake ? zwake->n : 0u, zcsr ? zcsr->n : 0u, 2 * n}));
+        const size_t small = (step_block_bytes(n, nmax) + 255u) & ~(size_t)255u;
+        const size_t mesh = (sizeof(float) * cells + 255u) & ~(size_t)255u;
+        if (hipMalloc(&s->block, small + 2 * mesh) != hipSuccess) {
+            return fail(VFPS_ERR_NOMEM, "vfps_step_create: device memory");
+        }
+        blk.base = s->block;
+        blk.host.assign(small, 0);
+        step_block = &blk;
+        float* data[3] = {reinterpret_cast<float*>(s->block + small),
+                          reinterpret_cast<float*>(s->block + small + mesh),
+                          nullptr};
+        vfps_mesh** grids[3] = {&s->t1, &s->t2, &s->t3};
+        for (int k = 0; k < 3; k++) {
+            rc = mesh_in_block(dev, n, desc->qmin, desc->qmax, desc->qscale,
+                               desc->pmin, desc->pmax, desc->pscale, data[k],
+                               grids[k]);
+            if (rc != VFPS_OK) return rc;
+        }
+    } else {
+        rc = vfps_mesh_create(dev, 1, n, desc->qmin, desc->qmax, desc->qscale,
+                              desc->pmin, desc->pmax, desc->pscale, 1.0, 1.0,
+                              &one, 1.0, init, &s->t1);
+        if (rc != VFPS_OK) return rc;
+        if ((rc = vfps_mesh_clone(s->t1, &s->t2)) != VFPS_OK) return rc;
+        if ((rc = vfps_mesh_clone(s->t1, &s->t3)) != VFPS_OK) return rc;
+    }
+    hipStream_t st = dev->stream;
     const int it = (int)desc->interp;
     if (desc->use_wake) {
         const uint32_t bucket0 = 0;
@@ -924,34 +991,44 @@ int vfps_step_create(vfps_dev* dev, const vfps_step_desc* desc,
         const uint32_t nmax = zcsr->n;
         auto renorm = csr_renorm(nmax, s->t1->ax0.delta, desc->qscale, desc->fc,
                                  &s->csr_fdelta);
+        VFPS_HIP(setup_alloc(&s->csr_renorm, nmax));
+        VFPS_HIP(setup_put(s->csr_renorm, renorm.data(), sizeof(float) * nmax, st));
         std::vector<double2> twm, twn;
-        make_twiddles(s->M, twm, twn);
-        // twiddles of their own, used when there is no wake field
-        VFPS_HIP(hipMalloc(&s->csr_renorm, sizeof(float) * nmax));
-        VFPS_HIP(hipMemcpy(s->csr_renorm, renorm.data(), sizeof(float) * nmax,
-                           hipMemcpyHostToDevice));
-        s->csr_tw_m = twm.size();
-        VFPS_HIP(hipMalloc(&s->csr_tw, sizeof(double2) * (twm.size() + s->M)));
-        VFPS_HIP(hipMemcpy(s->csr_tw, twm.data(), sizeof(double2) * twm.size(),
-                           hipMemcpyHostToDevice));
-        VFPS_HIP(hipMemcpy(s->csr_tw + s->csr_tw_m, twn.data(),
-                           sizeof(double2) * s->M, hipMemcpyHostToDevice));
+        if (!s->wfield) {
+            // twiddles of their own
+            make_twiddles(s->M, twm, twn);
+            s->csr_tw_m = twm.size();
+            VFPS_HIP(setup_alloc(&s->csr_tw, twm.size() + s->M));
+            VFPS_HIP(setup_put(s->csr_tw, twm.data(),
+                               sizeof(double2) * twm.size(), st));
+            VFPS_HIP(setup_put(s->csr_tw + s->csr_tw_m, twn.data(),
+                               sizeof(double2) * s->M, st));
+        }
+        VFPS_HIP(setup_sync(st));
     }
-    VFPS_HIP(hipMalloc(&s->filling, sizeof(double) * 2));
-    VFPS_HIP(hipMalloc(&s->counter, sizeof(uint32_t) * 2));
-    VFPS_HIP(hipMalloc(&s->err, sizeof(uint32_t)));
-    VFPS_HIP(hipHostMalloc(&s->err_h, sizeof(uint32_t), hipHostMallocDefault));
-    *s->err_h = 0;
-    VFPS_HIP(hipMalloc(&s->csr_power, sizeof(float)));
-    VFPS_HIP(hipMemset(s->filling, 0, sizeof(double) * 2));
-    VFPS_HIP(hipMemset(s->counter, 0, sizeof(uint32_t) * 2));
-    VFPS_HIP(hipMemset(s->err, 0, sizeof(uint32_t)));
-    VFPS_HIP(hipMemset(s->csr_power, 0, sizeof(float)));
-    VFPS_HIP(hipMalloc(&s->inst_d, sizeof(InstDesc)));
-    VFPS_HIP(hipMalloc(&s->fparams_d, sizeof(FieldParams)));
-    VFPS_HIP(hipSetDevice(dev->ordinal));
+    VFPS_HIP(setup_alloc(&s->filling, 2));
+    VFPS_HIP(setup_alloc(&s->counter, 2));
+    VFPS_HIP(setup_alloc(&s->err, 1));
+    VFPS_HIP(setup_alloc(&s->csr_power, 1));
+    VFPS_HIP(setup_zero(s->filling, sizeof(double) * 2, st));
+    VFPS_HIP(setup_zero(s->counter, sizeof(uint32_t) * 2, st));
+    VFPS_HIP(setup_zero(s->err, sizeof(uint32_t), st));
+    VFPS_HIP(setup_zero(s->csr_power, sizeof(float), st));
+    VFPS_HIP(setup_alloc(&s->inst_d, 1));
+    VFPS_HIP(setup_alloc(&s->fparams_d, 1));
     VFPS_CHECK_ARG(field_lds_bytes(s->M) <= dev->lds_max,
                    "vfps_step_create: FFT length exceeds the LDS of one CU");
+    if (s->direct && (rc = step_alloc_direct(s)) != VFPS_OK) return rc;
+    if (step_block) {
+        // everything so far in one copy, the mesh in another
+        step_block = nullptr;
+        VFPS_HIP(hipMemcpyAsync(blk.base, blk.host.data(), blk.used,
+                                hipMemcpyHostToDevice, st));
+        VFPS_HIP(hipMemcpyAsync(s->t1->data, init, sizeof(float) * cells,
+                                hipMemcpyHostToDevice, st));
+        rc = launch_project_x(s->t1, s->t1->data, s->t1->proj);
+        if (rc != VFPS_OK) return rc;
+    }
     if (s->direct && (rc = step_setup_direct(s)) != VFPS_OK) return rc;
     // fused kernel variant, tile and workgroup
     s->variant.scheme = (int)desc->scheme;
@@ -1029,6 +1106,7 @@ int vfps_step_run(vfps_step* s, uint32_t nsteps)
     uint32_t left = nsteps;
     int rc = step_flush_desc(s);
     if (rc != VFPS_OK) return rc;
+    if ((rc = step_err_flag(s)) != VFPS_OK) return rc;
     bool closed = false;
     if (!s->desc.no_graph) {
         // captured runs: full ones of STEP_GRAPH steps (even, so the parity
@@ -1077,6 +1155,7 @@ int vfps_step_prepare(vfps_step* s, uint32_t nsteps)
     VFPS_CHECK_ARG(s, "vfps_step_prepare: NULL step");
     int rc = step_flush_desc(s);
     if (rc != VFPS_OK) return rc;
+    if ((rc = step_err_flag(s)) != VFPS_OK) return rc;
     if (s->desc.no_graph || nsteps == 0) {
         return VFPS_OK;
     }

@@ -135,6 +135,8 @@ void rotation_halo(const RotGeom& g, uint32_t n, int it, uint32_t* hlo,
 struct vfps_step {
     vfps_dev* dev = nullptr;
     vfps_step_desc desc{};
+    char* block = nullptr;     // fused: the device arrays below, the meshes
+                               // included (StepBlock)
     vfps_mesh *t1 = nullptr, *t2 = nullptr, *t3 = nullptr;
     vfps_map *wm = nullptr, *rfm = nullptr, *drm = nullptr, *rot = nullptr,
              *fpm = nullptr;
