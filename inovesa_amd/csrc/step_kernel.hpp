@@ -148,6 +148,9 @@ constexpr int STEP_LOAD_BATCH = 8;
 // float4 loads of the input rows per thread issued before the wake products
 // (one-mesh launches)
 constexpr int STEP_EARLY_LOADS = 2;
+// most rows whose direct-form dot products a wavefront of a batch sums
+// together
+constexpr int STEP_DOT_ROWS = 4;
 // largest workgroup
 constexpr uint32_t STEP_MAX_THREADS = 512;
 // block-map entry of a padding workgroup
@@ -728,8 +731,95 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     // row 0 of the wake-kicked input (scheme 1 reads it for taps out of
     // range); tiles that do not hold row 0 compute it themselves
     const bool need_s00 = SCHEME == 1 && rbase > 0;
+    // kick row 0 by its wake offset (from its dot product): sample y = 0
+    auto row0_sample = [&](double acc) {
+        const float* row0 = lds + L.row0;
+        const float off = d.wake_scale * (float)acc;
+        uint32_t idx[IT];
+        float w[IT];
+        kick_taps<IT>(off, n, idx, w);
+        float v = 0.0f;
+#pragma unroll
+        for (int t = 0; t < IT; t++) {
+            const uint32_t ys = (uint32_t)((int32_t)idx[t] - half);
+            if (ys < n) {
+                v = v + row0[ys] * w[t];
+            }
+        }
+        return v;
+    };
     double csr_q = 0.0;
-    if (DIRECT && (wake || csr)) {
+    if (!ONE_MESH && DIRECT && (wake || csr)) {
+        // A batch reads the windows from the tables in global memory.  A job
+        // is up to STEP_DOT_ROWS consecutive rows of one table, sized so that
+        // the jobs spread over the wavefronts: their loads go out together and
+        // each value of the profile serves all of them.  (One row at a time,
+        // the two wavefronts of a 128^2 tile of two rows waited for four
+        // trips to L2 one after the other: 128 steps of 64 meshes of 128^2
+        // took 1.96 ms, now 1.85.)  A row's sum keeps its order.
+        const int nwk = wake ? lr1 - lr0 : 0;
+        const int ncsr = csr ? rows_out : 0;
+        const int ns00 = need_s00 && wake ? 1 : 0;
+        const int rj = min(STEP_DOT_ROWS,
+                           max(1, (nwk + ncsr + ns00 + (int)nw - 1) / (int)nw));
+        const int nwj = (nwk + rj - 1) / rj, ncj = (ncsr + rj - 1) / rj;
+        for (int job = (int)wave; job < nwj + ncj + ns00; job += (int)nw) {
+            const int which = job < nwj ? 0 : (job < nwj + ncj ? 1 : 2);
+            const int first = which == 0 ? job * rj : (job - nwj) * rj;
+            const int rows = which == 2 ? 1
+                             : which == 0 ? min(rj, nwk - first)
+                                          : min(rj, ncsr - first);
+            const gdouble* win =
+                (which == 0 ? wake_g + g0 + first
+                            : (which == 1 ? csr_h + (uint32_t)x0 + first : wake_g)) +
+                (n - 1);
+            double acc[STEP_DOT_ROWS];
+            uint32_t at[STEP_DOT_ROWS];
+#pragma unroll
+            for (int i = 0; i < STEP_DOT_ROWS; i++) {
+                acc[i] = 0.0;
+                at[i] = (uint32_t)min(i, rows - 1);  // (slots past the last
+                                                     // row repeat it, unused)
+            }
+#pragma unroll 2
+            for (uint32_t x = lane; x < n; x += 64) {
+                const double p = (double)pprev[x];
+                double w[STEP_DOT_ROWS];
+#pragma unroll
+                for (int i = 0; i < STEP_DOT_ROWS; i++) {
+                    w[i] = (win - x)[at[i]];
+                }
+#pragma unroll
+                for (int i = 0; i < STEP_DOT_ROWS; i++) {
+                    acc[i] += w[i] * p;
+                }
+            }
+            // every lane receives the sums; lane i finishes row i
+            double mine = 0.0;
+#pragma unroll
+            for (int i = 0; i < STEP_DOT_ROWS; i++) {
+                if (i < rows) {
+                    const double v = wave_sum_dpp(acc[i]);
+                    mine = lane == (uint32_t)i ? v : mine;
+                }
+            }
+            if (lane >= (uint32_t)rows) {
+                continue;
+            }
+            if (which == 0) {
+                const int row = lr0 + first + (int)lane;
+                const float off = d.wake_scale * (float)mine;
+                offw[row] = off;
+                store_row_taps<IT>(off, n, tapw + row * STEP_TAP_WORDS);
+            } else if (which == 1) {
+                const int o = first + (int)lane;
+                csr_rows[o] = (double)pprev[x0 + o] * mine;
+            } else {
+                s00_sh = row0_sample(mine);
+            }
+        }
+    }
+    if (ONE_MESH && DIRECT && (wake || csr)) {
         const int nwk = wake ? lr1 - lr0 : 0;
         const int ncsr = csr ? rows_out : 0;
         const int J = nwk + ncsr + ((need_s00 && wake) ? 1 : 0);
@@ -745,25 +835,14 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                 which = 2;
             }
             double acc = 0.0;
-            if constexpr (ONE_MESH) {
-                const double* win =
-                    which == 0 ? gwin
-                               : (which == 1 ? hwin
-                                             : reinterpret_cast<const double*>(
-                                                   lds + L.g0win));
+            const double* win =
+                which == 0 ? gwin
+                           : (which == 1 ? hwin
+                                         : reinterpret_cast<const double*>(
+                                               lds + L.g0win));
 #pragma unroll 4
-                for (uint32_t x = lane; x < n; x += 64) {
-                    acc += win[base + n - 1 - x] * (double)pprev[x];
-                }
-            } else {
-                // the same windows, read from the tables in global memory
-                const gdouble* win =
-                    which == 0 ? wake_g + g0
-                               : (which == 1 ? csr_h + (uint32_t)x0 : wake_g);
-#pragma unroll 4
-                for (uint32_t x = lane; x < n; x += 64) {
-                    acc += win[base + n - 1 - x] * (double)pprev[x];
-                }
+            for (uint32_t x = lane; x < n; x += 64) {
+                acc += win[base + n - 1 - x] * (double)pprev[x];
             }
             acc = wave_sum_dpp(acc);
             if (lane != 0) {
@@ -778,21 +857,7 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                 const int o = job - nwk;
                 csr_rows[o] = (double)pprev[x0 + o] * acc;
             } else {
-                // kick row 0 by its wake offset; s00 is its sample y = 0
-                const float* row0 = lds + L.row0;
-                const float off = d.wake_scale * (float)acc;
-                uint32_t idx[IT];
-                float w[IT];
-                kick_taps<IT>(off, n, idx, w);
-                float v = 0.0f;
-#pragma unroll
-                for (int t = 0; t < IT; t++) {
-                    const uint32_t ys = (uint32_t)((int32_t)idx[t] - half);
-                    if (ys < n) {
-                        v = v + row0[ys] * w[t];
-                    }
-                }
-                s00_sh = v;
+                s00_sh = row0_sample(acc);
             }
         }
     }
