@@ -247,17 +247,22 @@ int build_groups(vfps_batch* b)
     return build_fields(b);
 }
 
-// one step of every instance: the first group on the device stream, the
+int launch_group(const Group& g, uint32_t parity, hipStream_t st)
+{
+    return g.strip
+               ? launch_strip_kernel(g.variant, g.descs_d, g.blockmap_d,
+                                     g.nblocks, g.lds, g.threads, g.maxn,
+                                     parity, st)
+               : launch_step_kernel(g.variant, g.descs_d, g.blockmap_d,
+                                    g.nblocks, g.lds, g.threads, g.maxn, parity,
+                                    st, nullptr, g.grid);
+}
+
+// `steps` steps of every group: the first group on the device stream, the
 // others on branch streams forked from and joined back into it
-int launch_step(vfps_batch* b, uint32_t parity)
+int launch_chains(vfps_batch* b, uint32_t parity, uint32_t steps)
 {
     hipStream_t main = b->dev->stream;
-    // the FFT-wake members' wake potentials, CSR powers and step counts
-    for (const auto& f : b->fields) {
-        int rc = launch_fields(f.wake, f.csr, f.params_d, f.ninst, f.lds,
-                               parity, main);
-        if (rc != VFPS_OK) return rc;
-    }
     if (b->groups.size() > 1) {
         VFPS_HIP(hipEventRecord(b->fork, main));
     }
@@ -267,20 +272,49 @@ int launch_step(vfps_batch* b, uint32_t parity)
         if (k > 0) {
             VFPS_HIP(hipStreamWaitEvent(st, b->fork, 0));
         }
-        int rc = g.strip
-                     ? launch_strip_kernel(g.variant, g.descs_d, g.blockmap_d,
-                                           g.nblocks, g.lds, g.threads, g.maxn,
-                                           parity, st)
-                     : launch_step_kernel(g.variant, g.descs_d, g.blockmap_d,
-                                          g.nblocks, g.lds, g.threads, g.maxn,
-                                          parity, st, nullptr, g.grid);
-        if (rc != VFPS_OK) return rc;
+        for (uint32_t i = 0; i < steps; i++) {
+            int rc = launch_group(g, (parity + i) & 1u, st);
+            if (rc != VFPS_OK) return rc;
+        }
         if (k > 0) {
             VFPS_HIP(hipEventRecord(g.done, st));
         }
     }
     for (size_t k = 1; k < b->groups.size(); k++) {
         VFPS_HIP(hipStreamWaitEvent(main, b->groups[k].done, 0));
+    }
+    return VFPS_OK;
+}
+
+// one step of every instance, the FFT-wake members' wake potentials, CSR
+// powers and step counts first
+int launch_step(vfps_batch* b, uint32_t parity)
+{
+    for (const auto& f : b->fields) {
+        int rc = launch_fields(f.wake, f.csr, f.params_d, f.ninst, f.lds,
+                               parity, b->dev->stream);
+        if (rc != VFPS_OK) return rc;
+    }
+    return launch_chains(b, parity, 1);
+}
+
+// `steps` steps of every instance.  FFT-wake members share one field launch a
+// step, ahead of every group, which keeps the groups together.  Without them
+// nothing does, as the instances are independent: every group runs its steps
+// as a chain of its own and the chains meet once, at the end.  A join of the
+// size classes after each step left them hardly any overlap (64 meshes of
+// 128^2 to 512^2: the four launches alone took 67.5 us, the step 66); as
+// chains, launch gaps and the phases in which a class waits (the projection's
+// serial sums) fall on the other classes' work: 64 steps 4.40 -> 3.54 ms.
+// Dealing one class out over several chains does not pay: on 16 meshes of
+// 128^2 two chains took 8.7 ms and four 13.6 where one takes 7.5, and the
+// mixed batch stayed as it was.
+int launch_steps(vfps_batch* b, uint32_t parity, uint32_t steps)
+{
+    if (b->fields.empty()) return launch_chains(b, parity, steps);
+    for (uint32_t k = 0; k < steps; k++) {
+        int rc = launch_step(b, (parity + k) & 1u);
+        if (rc != VFPS_OK) return rc;
     }
     return VFPS_OK;
 }
@@ -361,14 +395,12 @@ int batch_graph(vfps_batch* b, uint32_t steps, uint32_t p, hipGraphExec_t* out)
     }
     hipStream_t st = b->dev->stream;
     VFPS_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    for (uint32_t k = 0; k < steps; k++) {
-        int rc = launch_step(b, (p + k) & 1u);
-        if (rc != VFPS_OK) {
-            hipGraph_t g = nullptr;
-            hipStreamEndCapture(st, &g);
-            if (g) hipGraphDestroy(g);
-            return rc;
-        }
+    int rc = launch_steps(b, p, steps);
+    if (rc != VFPS_OK) {
+        hipGraph_t g = nullptr;
+        hipStreamEndCapture(st, &g);
+        if (g) hipGraphDestroy(g);
+        return rc;
     }
     hipGraph_t def = nullptr;
     hipGraphExec_t exec = nullptr;

@@ -1,0 +1,34 @@
+"""Captured batch runs: every launch group advances as a chain of its own,
+FFT-wake members keep the groups together.  Pinned by the single-mesh step,
+bit for bit, over runs that end on either parity, follow one another and
+reuse a captured run."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sizes,fft_every,runs", [
+    ((64,), 0, (1, 64, 3)),
+    ((64, 128, 256, 512), 0, (65, 1, 63, 65)),
+    ((128, 256, 384), 2, (33, 64, 33)),
+])
+def test_chains_equal_single_steps(sizes, fft_every, runs):
+    import inovesa_amd as V
+    from inovesa_amd.workloads import batched_scan_config, impedances
+    inst = [(dict(desc, wake_method=1 if fft_every and k % fft_every == 0 else 2),
+             init, *impedances(d)) for k, (desc, d, init) in
+            enumerate(batched_scan_config(sizes=sizes, per_size=2, seed=9))]
+    b = V.Batch(*[[i[k] for i in inst] for k in range(4)])
+    assert (b.info()["launch_groups"] > 1) == (len(sizes) > 1)
+    total = sum(runs)
+    b.record(total)
+    for r in runs:
+        b.run(r)
+    for k, (desc, init, zw, zc) in enumerate(inst):
+        s = V.Step(desc, init, zw, zc)
+        s.record(total)
+        s.run(total)
+        for x, y in zip(b.mesh(k), s.mesh()):
+            assert np.array_equal(x, y), k
+        assert np.array_equal(b.history(k)[0], s.history()[0]), k
