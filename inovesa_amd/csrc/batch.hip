@@ -161,7 +161,10 @@ int build_group(vfps_batch* b, Group& g)
     for (uint32_t k : order) {
         const vfps_step* s = b->members[g.members[k]];
         g.maxn = std::max(g.maxn, s->desc.n);
-        const uint32_t units = g.strip ? s->strips() : s->tiles();
+        // (after a direct-wake instance's tiles: the workgroup that closes
+        // its step; a strip form's first strip does that)
+        const uint32_t units = g.strip ? s->strips()
+                                       : s->tiles() + (g.variant.direct ? 1u : 0u);
         for (uint32_t t = 0; t < units; t++) {
             map.push_back((k << 16) | t);
         }

@@ -416,8 +416,7 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                                           uint32_t parity, float* lds,
                                           StepShared& sh)
 {
-    constexpr int EARLY = ONE_MESH ? STEP_EARLY_LOADS : 0;
-    double* red = sh.red;
+    constexpr int EARLY = STEP_EARLY_LOADS;
     float& s00_sh = sh.s00;
     uint32_t& slot_sh = sh.slot;
     uint32_t& cnt_sh = sh.cnt;
@@ -427,7 +426,12 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     const uint32_t stride = d.stride;
     const int x0 = (int)(tile * T);
     if (x0 >= (int)n) {
-        return;  // not launched: grids hold exactly the tiles
+        // (a batch, direct form: the entry after an instance's tiles)
+        if (DIRECT && !ONE_MESH) {
+            step_close(d, parity,
+                       d.counter ? ((const guint*)d.counter)[parity] : 0u, sh.red);
+        }
+        return;
     }
     VFPS_STAMP(0);
     const int rows_out = min((int)T, (int)n - x0);
@@ -691,7 +695,7 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
             }
         }
     };
-    if constexpr (EARLY == 0) {
+    if constexpr (!ONE_MESH) {
         fill_rows();
     }
     __syncthreads();
@@ -861,7 +865,7 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
             }
         }
     }
-    if constexpr (EARLY > 0) {
+    if constexpr (ONE_MESH) {
         fill_rows();
     }
     __syncthreads();
@@ -1235,16 +1239,10 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     }
     VFPS_STAMP(7);
     // ---- H: close the step (direct form) --------------------------------------
-    // Every tile leaves its CSR share.  In a batch, tile 0 of each instance
-    // also closes the step (step_close); a one-mesh launch gives that to a
-    // workgroup of its own.
-    if (DIRECT) {
-        if (csr && tid == 0) {
-            d.csr_part[(size_t)parity * n + tile] = csr_q;
-        }
-        if (!ONE_MESH && tile == 0) {
-            step_close(d, parity, cnt, red);
-        }
+    // Every tile leaves its CSR share; a workgroup of its own closes the step
+    // beside the tiles (step_close).
+    if (DIRECT && csr && tid == 0) {
+        d.csr_part[(size_t)parity * n + tile] = csr_q;
     }
     if (d.tstamp) {
         // per-tile entry and exit times
