@@ -17,10 +17,10 @@
 //      products mesh*weight of the x projection;
 //   G  the x projection of its rows (PhaseSpace::updateXProjection), summed
 //      in std::inner_product order;
-//   H  (direct wake) every tile stores its CSR share; tile 0 (a one-mesh
-//      launch: a workgroup of its own) counts the step, computes the FP64
-//      charge integral and sums the previous step's shares in a fixed order
-//      (the launch boundary orders them).
+//   H  (direct wake) every tile stores its CSR share; a workgroup of its own
+//      beside each mesh's tiles counts the step, computes the FP64 charge
+//      integral and sums the previous step's shares in a fixed order (the
+//      launch boundary orders them).
 // The mesh makes one trip HBM -> LDS -> HBM per step.  The state buffers
 // and the x projections ping-pong (`parity`), so a step reads only what
 // the previous launch wrote.
@@ -146,7 +146,10 @@ constexpr int STEP_MAX_COLS = 4;
 // float4 loads one thread keeps in flight while filling the tile
 constexpr int STEP_LOAD_BATCH = 8;
 // float4 loads of the input rows per thread issued before the wake products
-// (one-mesh launches)
+// (one mesh: they stay in registers until after the products.  A batch stores
+// them before, but sends them ahead of its tables' loads: 16 meshes of 128^2
+// 8.5 -> 8.1 us a step, 16 each of 128^2 to 512^2 in their first tilings 168 ->
+// 153; the occupancy is the same.)
 constexpr int STEP_EARLY_LOADS = 2;
 // most rows whose direct-form dot products a wavefront of a batch sums
 // together
@@ -416,7 +419,6 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                                           uint32_t parity, float* lds,
                                           StepShared& sh)
 {
-    constexpr int EARLY = STEP_EARLY_LOADS;
     float& s00_sh = sh.s00;
     uint32_t& slot_sh = sh.slot;
     uint32_t& cnt_sh = sh.cnt;
@@ -426,7 +428,9 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     const uint32_t stride = d.stride;
     const int x0 = (int)(tile * T);
     if (x0 >= (int)n) {
-        // (a batch, direct form: the entry after an instance's tiles)
+        // (a batch, direct form: the entry after an instance's tiles.  In a
+        // tile the closing lengthened the launch: 16 meshes of 128^2 took
+        // 9.4 us a step, with a workgroup of its own 8.5.)
         if (DIRECT && !ONE_MESH) {
             step_close(d, parity,
                        d.counter ? ((const guint*)d.counter)[parity] : 0u, sh.red);
@@ -474,9 +478,9 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     const bool csr = DIRECT && d.use_csr != 0;
 
     // ---- A: every global read -------------------------------------------
-    //  - the first EARLY float4 of the input rows per thread go out first
-    //    and stay in registers through phase B (stored to LDS after the
-    //    wake products): the tables' stores below wait for them too (the
+    //  - the first float4 loads of the input rows go out first
+    //    and, one mesh, stay in registers through phase B (stored to LDS
+    //    after the wake products): the tables' stores below wait for them too (the
     //    load counter drains in order), but the compiler keeps them here
     //    instead of sinking them to their use after B
     const bool vec_rows = (n & 3u) == 0u;
@@ -484,10 +488,10 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     const uint32_t in_total = (uint32_t)(lr1 - lr0) * n;
     const uint32_t in_total4 = in_total >> 2;
     const gfloat4* in4 = (const gfloat4*)(in + in_first);
-    vec4f early[EARLY > 0 ? EARLY : 1];
+    vec4f early[STEP_EARLY_LOADS];
     if (vec_rows) {
 #pragma unroll
-        for (int b = 0; b < EARLY; b++) {
+        for (int b = 0; b < STEP_EARLY_LOADS; b++) {
             const uint32_t i = tid + (uint32_t)b * bs;
             early[b] = in4[i < in_total4 ? i : in_total4 - 1u];
         }
@@ -655,18 +659,18 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     }
     //  - input rows [rbase+lr0, rbase+lr1) to LDS: the early registers, then
     //    the rest in batches; the kick taps of the RF (and FFT wake) rows.
-    //    Without early loads this runs before the barrier that ends phase A
-    //    (after phase B it would keep the batch registers live through B).
+    //    In a batch this runs before the barrier that ends phase A (after
+    //    phase B it would keep the batch registers live through B).
     auto fill_rows = [&]() {
         float* dst = bufA + (size_t)lr0 * n;
         if (vec_rows) {
             vec4f* a4 = reinterpret_cast<vec4f*>(dst);
 #pragma unroll
-            for (int b = 0; b < EARLY; b++) {
+            for (int b = 0; b < STEP_EARLY_LOADS; b++) {
                 const uint32_t i = tid + (uint32_t)b * bs;
                 if (i < in_total4) a4[i] = early[b];
             }
-            for (uint32_t base = (uint32_t)EARLY * bs; base < in_total4;
+            for (uint32_t base = (uint32_t)STEP_EARLY_LOADS * bs; base < in_total4;
                  base += bs * STEP_LOAD_BATCH) {
                 // unconditional loads (clamped index) keep v in registers
                 vec4f v[STEP_LOAD_BATCH];
