@@ -28,6 +28,8 @@
 // kernel, so the two forms give the same bits (pinned by the batch tests).
 #pragma once
 
+#include <type_traits>
+
 #include "step_kernel.hpp"
 
 namespace vfps_impl {
@@ -685,19 +687,19 @@ __device__ __forceinline__ void strip_body(const InstDesc& d, uint32_t strip,
             const int r0 = x0 + (int)col_d0[c] - half;
             const bool win_ok = ((dcons >> c) & 1u) && r0 >= wlo &&
                                 r0 + rows_out + IT - 2 < whi;
-            auto window = [&]() {
-                // every slot is read, so that the loads go out together
-                // (one past the window reads some ring row, in bounds, and
-                // is not used)
-                float win[STRIP_MAX_T + IT - 1];
+            // the window of TT output rows from row first on: its TT + IT - 1
+            // loads go out together
+            auto window = [&](auto tt, int first) {
+                constexpr int TT = decltype(tt)::value;
+                float win[TT + IT - 1];
 #pragma unroll
-                for (int t = 0; t < (int)STRIP_MAX_T + IT - 1; t++) {
+                for (int t = 0; t < TT + IT - 1; t++) {
                     const uint32_t slot =
-                        ((uint32_t)(r0 + t) + (uint32_t)hlo) & rmask;
+                        ((uint32_t)(first + t) + (uint32_t)hlo) & rmask;
                     win[t] = ring[__umul24(slot, n) + y];
                 }
 #pragma unroll
-                for (int o = 0; o < (int)STRIP_MAX_T; o++) {
+                for (int o = 0; o < TT; o++) {
                     if (o < rows_out) {
                         float v = 0.0f;
 #pragma unroll
@@ -708,14 +710,32 @@ __device__ __forceinline__ void strip_body(const InstDesc& d, uint32_t strip,
                     }
                 }
             };
+            using Four = std::integral_constant<int, 4>;
+            // (fewer rows than the largest tile: the slots past the window
+            // read some ring row, in bounds, and are not used)
+            using Any = std::integral_constant<int, (int)STRIP_MAX_T>;
             // a wavefront whose columns all read windows takes no per-lane
             // branch
             if (__all(win_ok)) {
-                window();
+                if (rows_out == 4) {
+                    // the tile height of the production workload: 7 loads
+                    // for 4 rows where the largest height takes 11, and with
+                    // one first row their ring slots are scalar arithmetic
+                    // (the sub-tiles are VALU-bound: 16 meshes of 1024^2,
+                    // 64 steps, 4.72 -> 4.54 ms)
+                    const int r0u = __builtin_amdgcn_readfirstlane(r0);
+                    if (__all(r0 == r0u)) {
+                        window(Four{}, r0u);
+                    } else {
+                        window(Four{}, r0);
+                    }
+                } else {
+                    window(Any{}, r0);
+                }
                 continue;
             }
             if (win_ok) {
-                window();
+                window(Any{}, r0);
                 continue;
             }
             // taps not consecutive, or beyond the window (an error)
