@@ -216,8 +216,8 @@ struct vfps_mlp {
     uint16_t* WT = nullptr;
     uint16_t* AT = nullptr;         // layer inputs and dZ [feature][sample]
     uint16_t* GT = nullptr;
-    float* dbp = nullptr;           // bias and loss partials
-    double* lossp = nullptr;
+    float* dz = nullptr;            // FP32 dZ [sample][column]
+    double* terms = nullptr;        // loss terms [sample][output]
     // training data kept between calls of train (grown as needed)
     void* data = nullptr;
     size_t data_bytes = 0;
@@ -249,7 +249,7 @@ void mlp_free(vfps_mlp* m)
                     (void*)m->dyb, (void*)m->dz2, (void*)m->dzb2,
                     (void*)m->tgt, (void*)m->lab, (void*)m->loss,
                     (void*)m->W, (void*)m->WT, (void*)m->AT, (void*)m->GT,
-                    (void*)m->dbp, (void*)m->lossp, m->data}) {
+                    (void*)m->dz, (void*)m->terms, m->data}) {
         (void)hipFree(q);
     }
     for (auto* q : m->z) (void)hipFree(q);
@@ -363,9 +363,9 @@ struct Batch {
     uint32_t B;
 };
 
-// the rows kernel; returns its workgroups
+// the rows kernel
 template <bool TRAIN>
-uint32_t launch_rows(vfps_mlp* m, const MlpRowsArgs& a)
+void launch_rows(vfps_mlp* m, const MlpRowsArgs& a)
 {
     const uint32_t rr = mlp_rows_per_lane(a.B, (uint32_t)m->dev->ncu);
     // (training: whole 32s of samples, the depth of the gradient products)
@@ -381,7 +381,6 @@ uint32_t launch_rows(vfps_mlp* m, const MlpRowsArgs& a)
     } else {
         hipLaunchKernelGGL((mlp_rows_kernel<TRAIN, 4>), g, t, lds, st, m->net, a);
     }
-    return blocks;
 }
 
 int fused_forward(vfps_mlp* m, const float* x, uint32_t B, float* y)
@@ -414,21 +413,21 @@ int fused_step(vfps_mlp* m, const Batch& b, float wl, float* loss,
     a.wl = wl;
     a.AT = m->AT;
     a.GT = m->GT;
-    a.dbp = m->dbp;
-    a.lossp = m->lossp;
+    a.dz = m->dz;
+    a.terms = m->terms;
+    launch_rows<true>(m, a);
     MlpGradArgs g{};
-    g.nwg = launch_rows<true>(m, a);
     g.AT = m->AT;
     g.GT = m->GT;
-    g.dbp = m->dbp;
-    g.lossp = m->lossp;
+    g.dz = m->dz;
+    g.terms = m->terms;
     g.B = b.B;
     g.g = m->g;
     g.loss = loss;
     uint32_t tiles = 0;
     for (uint32_t l = 0; l < m->net.L; l++) tiles += mlp_grad_tiles(m->net, l);
     const uint32_t tb = (tiles + 3u) / 4u;
-    const uint32_t bb = (m->net.nbias + MLP_GRAD_THREADS - 1) / MLP_GRAD_THREADS;
+    const uint32_t bb = mlp_grad_sums(m->net);
     if (adam) {
         g.p = m->p;
         g.m = m->m;
@@ -579,13 +578,12 @@ int vfps_mlp_create(vfps_dev* dev, const uint32_t* dims, uint32_t ndims,
                     (int)MLP_LDS_MAX));
             }
         }
-        const size_t nwg = mlp_max_blocks(k.bmax, (uint32_t)dev->ncu);
         VFPS_HIP(hipMalloc(&m->W, sizeof(uint16_t) * k.wsize));
         VFPS_HIP(hipMalloc(&m->WT, sizeof(uint16_t) * k.wsize));
         VFPS_HIP(hipMalloc(&m->AT, sizeof(uint16_t) * k.arows * k.bmax));
         VFPS_HIP(hipMalloc(&m->GT, sizeof(uint16_t) * k.grows * k.bmax));
-        VFPS_HIP(hipMalloc(&m->dbp, sizeof(float) * nwg * k.nbias));
-        VFPS_HIP(hipMalloc(&m->lossp, sizeof(double) * nwg));
+        VFPS_HIP(hipMalloc(&m->dz, sizeof(float) * k.bmax * k.nbias));
+        VFPS_HIP(hipMalloc(&m->terms, sizeof(double) * k.bmax * k.w[k.L]));
         // (the outputs of a forward longer than the staging)
         VFPS_HIP(hipMalloc(&m->dy, sizeof(float) * B * dims[ndims - 1]));
         *out = guard.release();

@@ -7,14 +7,14 @@
 //                     backward products.  Activations never leave the LDS.
 //   mlp_grad_kernel   every layer's weight gradient (a wavefront per 16x16
 //                     tile, the batch as the contraction), the bias
-//                     gradients and, when training, Adam on the parameters
-//                     the gradient belongs to, in the same pass.
+//                     gradients, the loss and, when training, Adam on the
+//                     parameters the gradient belongs to, in the same pass.
 //
 // The layer-by-layer form they replace launched 15 kernels a training step
 // (gathers, products, column sums, loss, Adam), most of them one to a few
 // workgroups long: 422 us a step for 256 samples of 3-256-256-256-65; the two
-// take 20.5 and 5.7 us (an epoch of 8192 samples, uploads included: 13.6 ms
-// before, 1.03 ms).  A forward of 512 samples went from 88.6 to 27.7 us.
+// take 21.2 and 6.4 us (an epoch of 8192 samples, uploads included: 13.5 ms
+// before, 1.07 ms).  A forward of 512 samples went from 88.6 to 27.4 us.
 //
 // Operand layout.  v_mfma_f32_16x16x32_bf16 wants 8 consecutive k per lane
 // from both operands: lane l holds column (or row) l % 16, k = 8 (l / 16) ...
@@ -24,7 +24,8 @@
 // inputs and output gradients of a batch (samples as the contraction).  A
 // fragment load is then 1 KB in a row and needs no bounds check.  With
 // row-major matrices a load touched 16 rows, and the 128 KB of a layer took
-// a workgroup 4 us (30 us a launch for the training kernel, 20.5 now).
+// a workgroup 4 us (30 us a launch for the training kernel, 20.6 with
+// fragments).
 #pragma once
 
 #include "common.hpp"
@@ -127,15 +128,17 @@ struct MlpNet {
     uint32_t wo[MLP_MAX_LAYERS] = {};     // padded BF16 weights
     uint32_t ao[MLP_MAX_LAYERS] = {};     // rows of a layer's input [feature]
     uint32_t go[MLP_MAX_LAYERS] = {};     // rows of a layer's dZ [feature]
-    uint32_t nbias = 0;                   // bias partials per workgroup
-    uint32_t to[MLP_MAX_LAYERS] = {};     // a layer's bias partials
+    uint32_t nbias = 0;                   // all layers' dZ columns
+    uint32_t to[MLP_MAX_LAYERS] = {};     // a layer's first one
     // LDS (4-byte words)
-    uint32_t zo[MLP_MAX_LAYERS] = {};     // gelu' of the hidden layers [.][wp+4]
-    uint32_t yo = 0;                      // outputs [16][w + 1]
-    uint32_t tgt = 0, lab = 0;            // targets [16][w - 1], labels [16]
+    uint32_t zo[MLP_MAX_LAYERS] = {};     // hidden layers: gelu', then dZ
+                                          // [16][wp + 4]
+    uint32_t yo = 0;                      // outputs, then dZ [16][w + 1]
+    uint32_t tgt = 0;                     // targets, then the outputs'
+                                          // differences from them [16][w - 1]
+    uint32_t lab = 0, logit = 0;          // labels, their outputs [16]
     uint32_t act[2] = {};                 // BF16 activations [16][as]
     uint32_t tr = 0;                      // layer inputs, then dZ [feature][.]
-    uint32_t db = 0;                      // bias partials [nbias]
     uint32_t as = 0;                      // their row stride (halves)
     uint32_t lds_words = 0;
     uint32_t wsize = 0, arows = 0, grows = 0;
@@ -180,6 +183,8 @@ inline MlpNet mlp_net(const uint32_t* dims, uint32_t ndims, uint32_t max_batch)
     z += MLP_ROWS * (out - 1);
     n.lab = z;
     z += MLP_ROWS;
+    n.logit = z;
+    z += MLP_ROWS;
     z = (z + 3u) & ~3u;
     n.as = widest + 8;  // rows 4 banks apart, 16-byte aligned
     for (uint32_t k = 0; k < 2; k++) {
@@ -188,8 +193,6 @@ inline MlpNet mlp_net(const uint32_t* dims, uint32_t ndims, uint32_t max_batch)
     }
     n.tr = z;
     z += (n.arows + n.grows) * MLP_ROWS / 2;
-    n.db = z;
-    z += n.nbias;
     n.lds_words = z;
     n.bmax = up32(max_batch);
     if ((size_t)z * 4 > MLP_LDS_MAX) return MlpNet{};
@@ -210,8 +213,8 @@ struct MlpRowsArgs {
     float wl;                // weight of the label's loss
     uint16_t* AT;            // layer inputs: columns features, k samples
     uint16_t* GT;            // layer dZ, the same way
-    float* dbp;              // bias partials [workgroup][nbias]
-    double* lossp;           // loss partials [workgroup]
+    float* dz;               // FP32 dZ [sample][nbias]
+    double* terms;           // loss terms [sample][out]
 };
 
 // up to MLP_FRAGS fragments from q on, of `count` (one past them rereads the
@@ -256,8 +259,8 @@ __device__ __forceinline__ f32x4 mlp_tile(const uint16_t* act, uint32_t as,
 // (mlp_rows_per_lane).  The products cost a CU 1 us whatever of their 16 rows
 // is in use, but a GELU with its derivative is about 130 instructions: with
 // 16 samples a workgroup's four wavefronts per SIMD spend 3 us a layer on
-// them, and a batch of 256 is 16 workgroups; with 4 samples it is 64 (256
-// samples: 34 us a launch before, 30 after).
+// them, and a batch of 256 is 16 workgroups; with 4 samples it is 64 (a
+// launch of 256 samples, operands still row by row: 34 us with 16, 30 with 4).
 // A lane of a product's result holds rows 4 q .. 4 q + 3 of one column, so
 // sample s = q RR + r is given MFMA row 4 q + r: every lane then has RR
 // samples (the rows between hold stale values that no other row sees).
@@ -271,7 +274,6 @@ __global__ void __launch_bounds__(MLP_THREADS)
 mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
 {
     extern __shared__ __align__(16) float lds[];
-    __shared__ double red[16];
     constexpr uint32_t R = 4u * RR;  // samples of this workgroup
     typedef uint16_t packed_t __attribute__((ext_vector_type(RR == 1 ? 2 : RR)));
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -417,7 +419,6 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
     // weight wl); loss = (1/B) sum_b [ (1/S) sum_k (y-t)^2 + wl BCE ].
     {
         const uint32_t S = out - 1, NP = n.wp[L];
-        double loss = 0.0;
         for (uint32_t t = tid; t < R * NP; t += MLP_THREADS) {
             const uint32_t s = t / NP, k = t % NP;
             float g = 0.0f;
@@ -425,38 +426,30 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
                 const float v = y[s * (out + 1u) + k];
                 if (k < S) {
                     const float d = v - lds[n.tgt + s * S + k];
-                    loss += (double)d * (double)d / (double)S;
+                    lds[n.tgt + s * S + k] = d;
                     g = 2.0f * d / (float)(S * a.B);
                 } else {
-                    const float lab = lds[n.lab + s];
-                    // BCE with logits: max(y,0) - y*lab + log(1 + exp(-|y|))
-                    loss += (double)a.wl *
-                            ((double)fmaxf(v, 0.0f) - (double)v * lab +
-                             log1p(exp(-fabs((double)v))));
                     const float sg = 1.0f / (1.0f + expf(-v));
-                    g = a.wl * (sg - lab) / (float)a.B;
+                    lds[n.logit + s] = v;
+                    g = a.wl * (sg - lds[n.lab + s]) / (float)a.B;
                 }
             }
             if (k < out) y[s * (out + 1u) + k] = g;
             act[row(s) * n.as + k] = f2bf(g);
         }
-        loss = block_sum(loss, red);  // (its barriers order act and y too)
-        if (tid == 0) red[0] = loss;
+        __syncthreads();
         for (uint32_t k = tid; k < NP; k += MLP_THREADS) {
-            float sum = 0.0f;
 #pragma unroll
             for (uint32_t s = 0; s < R; s++) {
                 tr[(n.arows + n.go[L - 1] + k) * R + s] = act[row(s) * n.as + k];
-                if (k < out) sum += y[s * (out + 1u) + k];
             }
-            lds[n.db + n.to[L - 1] + k] = sum;
         }
     }
 
     // ---- backward: dZ of layer l - 1 from dZ of layer l ---------------------------
     for (uint32_t l = L - 1; l > 0; l--) {
         const uint32_t NP = n.wp[l];
-        const float* grad = lds + n.zo[l - 1];
+        float* grad = lds + n.zo[l - 1];
         auto next = [&]() {
             if (l > 1) fetch_backward(l - 1, wave * 16u);
         };
@@ -464,21 +457,16 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
                 [&](uint32_t tj) { fetch_backward(l, tj); }, next,
                 [&](f32x4 acc, uint32_t j, float) {
             packed_t packed;
-            float sum = 0.0f;
 #pragma unroll
             for (uint32_t r = 0; r < (uint32_t)RR; r++) {
                 const uint32_t s = s0 + r;
-                const float dz = r0 + s < a.B
-                                     ? acc[r] * grad[s * (NP + 4u) + j]
-                                     : 0.0f;
-                sum += dz;
+                float& g = grad[s * (NP + 4u) + j];
+                const float dz = r0 + s < a.B ? acc[r] * g : 0.0f;
+                g = dz;
                 packed[r] = f2bf(dz);
                 nxt[row(s) * n.as + j] = packed[r];
             }
             keep(n.arows + n.go[l - 1] + j, packed);
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
-            if (q4 == 0) lds[n.db + n.to[l - 1] + j] = sum;
         });
         __syncthreads();
         uint16_t* t = act;
@@ -495,11 +483,30 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
             mlp_frag(in ? feature : feature - n.arows, r0 + 4u * c, n.bmax)) =
             *reinterpret_cast<const u16x4*>(tr + feature * R + 4u * c);
     }
-    if (tid == 0) {
-        a.lossp[blockIdx.x] = red[0];
+    for (uint32_t l = 0; l < L; l++) {
+        const uint32_t NP = n.wp[l + 1];
+        for (uint32_t t = tid; t < R * NP; t += MLP_THREADS) {
+            const uint32_t s = t / NP, j = t % NP;
+            a.dz[(size_t)(r0 + s) * n.nbias + n.to[l] + j] =
+                l + 1 < L  ? lds[n.zo[l] + s * (NP + 4u) + j]
+                : j < out  ? y[s * (out + 1u) + j]
+                           : 0.0f;
+        }
     }
-    for (uint32_t t = tid; t < n.nbias; t += MLP_THREADS) {
-        a.dbp[(size_t)blockIdx.x * n.nbias + t] = lds[n.db + t];
+    for (uint32_t t = tid; t < R * out; t += MLP_THREADS) {
+        const uint32_t s = t / out, k = t % out, S = out - 1;
+        double e = 0.0;
+        if (k < S) {
+            const float d = lds[n.tgt + s * S + k];
+            e = (double)d * (double)d / (double)S;
+        } else {
+            // BCE with logits: max(y,0) - y*lab + log(1 + exp(-|y|))
+            const float v = lds[n.logit + s];
+            e = (double)a.wl * ((double)fmaxf(v, 0.0f) -
+                                (double)v * lds[n.lab + s] +
+                                log1p(exp(-fabs((double)v))));
+        }
+        if (r0 + s < a.B) a.terms[(size_t)(r0 + s) * out + k] = e;
     }
 }
 
@@ -509,18 +516,12 @@ inline uint32_t mlp_rows_per_lane(uint32_t B, uint32_t ncu)
     const uint32_t rows = (B + 31u) & ~31u;
     return rows <= 4u * ncu ? 1u : rows <= 8u * ncu ? 2u : 4u;
 }
-// most workgroups of the rows kernel for any batch of at most bmax samples
-inline uint32_t mlp_max_blocks(uint32_t bmax, uint32_t ncu)
-{
-    return std::max(std::min(bmax / 4u, ncu), bmax / MLP_ROWS);
-}
 
 struct MlpGradArgs {
     const uint16_t* AT;
     const uint16_t* GT;
-    const float* dbp;
-    const double* lossp;
-    uint32_t nwg;            // workgroups of the rows kernel
+    const float* dz;
+    const double* terms;
     uint32_t B;
     float* g;                // gradients
     float* loss;             // [1] the batch's loss
@@ -541,8 +542,24 @@ __host__ __device__ inline uint32_t mlp_grad_tiles(const MlpNet& n, uint32_t l)
 
 constexpr uint32_t MLP_GRAD_THREADS = 256;
 
+constexpr uint32_t MLP_BIAS_COLS = 32;   // (a layer's columns are whole 32s)
+constexpr uint32_t MLP_BIAS_ROWS = 256;  // samples staged at once
+constexpr uint32_t MLP_BIAS_STRIDE = MLP_BIAS_ROWS + 4;
+
+// workgroups beside the tiles': the biases' and one for the loss
+__host__ __device__ inline uint32_t mlp_grad_sums(const MlpNet& n)
+{
+    return n.nbias / MLP_BIAS_COLS + 1u;
+}
+
 // Workgroups [0, tiles/4): a tile of dW = dZ^T A per wavefront; then the
-// biases, a thread each; the last workgroup's last thread adds the loss.
+// biases, 32 columns of dZ each; the last workgroup adds the loss.
+// The sums that no matrix product fixes keep one order whatever the batch's
+// split over workgroups: a bias gradient adds its samples one after another
+// in FP32 (as colsum_kernel), the loss its terms as loss_kernel does.  So a
+// training run gives the same bits as layer by layer.  (Partial sums of the
+// rows kernel's workgroups took 1.3 us less a step of 256 samples, 27.6 in
+// all, in other last bits.)
 // Bound: the operands' trip from L2 (608 tiles of 16 KB for the surrogate
 // at 256 samples).
 template <bool ADAM>
@@ -551,7 +568,6 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
 {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t K = (a.B + 31u) & ~31u;
-    const uint32_t nwg = a.nwg;
     if (blockIdx.x < tile_blocks) {
         uint32_t tile = blockIdx.x * (MLP_GRAD_THREADS / 64u) + wave;
         uint32_t l = 0;
@@ -613,28 +629,90 @@ mlp_grad_kernel(MlpNet n, MlpGradArgs a, uint32_t tile_blocks)
         }
         return;
     }
-    const uint32_t t = (blockIdx.x - tile_blocks) * MLP_GRAD_THREADS + tid;
-    if (t < n.nbias) {
+    const uint32_t c0 = (blockIdx.x - tile_blocks) * MLP_BIAS_COLS;
+    if (c0 < n.nbias) {
+        __shared__ __align__(16) float cols[MLP_BIAS_COLS * MLP_BIAS_STRIDE];
         uint32_t l = 0;
-        while (l + 1 < n.L && t >= n.to[l + 1]) l++;
-        const uint32_t j = t - n.to[l];
-        if (j < n.w[l + 1]) {
-            float s = 0.0f;
-#pragma unroll 16
-            for (uint32_t w = 0; w < nwg; w++) {
-                s += a.dbp[(size_t)w * n.nbias + t];
+        while (l + 1 < n.L && c0 >= n.to[l + 1]) l++;
+        const uint32_t j = c0 - n.to[l] + tid;
+        const bool mine = tid < MLP_BIAS_COLS && j < n.w[l + 1];
+        const uint32_t o = n.bo[l] + (mine ? j : 0u);
+        float pv = 0.0f, mv = 0.0f, vv = 0.0f;
+        if (ADAM) {
+            pv = a.p[o];
+            mv = a.m[o];
+            vv = a.v[o];
+        }
+        float s = 0.0f;
+        for (uint32_t b0 = 0; b0 < K; b0 += MLP_BIAS_ROWS) {
+            // (samples from the batch's end to K are zeros, which change no
+            // sum that starts at +0)
+            const uint32_t nr = min(MLP_BIAS_ROWS, K - b0);
+            constexpr uint32_t QUADS = MLP_BIAS_COLS / 4;
+            constexpr uint32_t STEP = MLP_GRAD_THREADS / QUADS;
+            constexpr uint32_t LOADS = MLP_BIAS_ROWS / STEP;
+            const uint32_t q = tid % QUADS, r = tid / QUADS;
+            f32x4 v[LOADS];
+#pragma unroll
+            for (uint32_t i = 0; i < LOADS; i++) {
+                const uint32_t b = b0 + min(r + i * STEP, nr - 1u);
+                v[i] = *reinterpret_cast<const f32x4*>(
+                    a.dz + (size_t)b * n.nbias + c0 + q * 4u);
             }
-            const uint32_t o = n.bo[l] + j;
+#pragma unroll
+            for (uint32_t i = 0; i < LOADS; i++) {
+#pragma unroll
+                for (uint32_t e = 0; e < 4; e++) {
+                    cols[(q * 4u + e) * MLP_BIAS_STRIDE + r + i * STEP] = v[i][e];
+                }
+            }
+            __syncthreads();
+            if (tid < MLP_BIAS_COLS) {
+                const f32x4* p4 = reinterpret_cast<const f32x4*>(
+                    cols + tid * MLP_BIAS_STRIDE);
+                for (uint32_t b = 0; b < nr; b += 32u) {
+                    f32x4 x[8];
+#pragma unroll
+                    for (uint32_t i = 0; i < 8; i++) x[i] = p4[b / 4u + i];
+#pragma unroll
+                    for (uint32_t i = 0; i < 8; i++) {
+                        s = s + x[i].x;
+                        s = s + x[i].y;
+                        s = s + x[i].z;
+                        s = s + x[i].w;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (mine) {
             a.g[o] = s;
             if (ADAM) {
-                adam_update(a.adam, s, a.p + o, a.m + o, a.v + o);
+                adam_update(a.adam, s, &pv, &mv, &vv);
+                a.p[o] = pv;
+                a.m[o] = mv;
+                a.v[o] = vv;
             }
         }
+        return;
     }
-    if (blockIdx.x == gridDim.x - 1 && tid == MLP_GRAD_THREADS - 1) {
-        double s = 0.0;
-#pragma unroll 16
-        for (uint32_t w = 0; w < nwg; w++) s += a.lossp[w];
+    __shared__ double red[16];
+    const uint32_t total = a.B * n.w[n.L];
+    double s = 0.0;
+    constexpr uint32_t AHEAD = 16;
+    for (uint32_t t = tid; t < total; t += AHEAD * MLP_GRAD_THREADS) {
+        double e[AHEAD];
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; i++) {
+            e[i] = a.terms[min(t + i * MLP_GRAD_THREADS, total - 1u)];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; i++) {
+            if (t + i * MLP_GRAD_THREADS < total) s += e[i];
+        }
+    }
+    s = block_sum(s, red);
+    if (tid == 0) {
         *a.loss = (float)(s / (double)a.B);
     }
 }

@@ -99,3 +99,27 @@ def test_train_is_gradients_and_adam(V, dims):
     c = V.MLP(dims, max_batch=48, seed=1)
     c.set_params(a.params())
     np.testing.assert_array_equal(a.forward(x), c.forward(x))
+
+
+@pytest.mark.parametrize("dims,B", [((3, 40, 17, 9), 32), ((2, 33, 2), 64),
+                                    ((5, 7), 256), ((3, 64, 40, 5), 512),
+                                    ((3, 40, 17, 9), 2048),
+                                    ((3, 32, 9), 4096),
+                                    ((3, 1200, 1100, 9), 64)])
+def test_bias_gradients_add_the_samples_in_order(V, dims, B):
+    """A bias gradient is the FP32 sum of its column of dZ over the samples,
+    one after another, in either form and for any split of the batch over
+    workgroups.  dZ of a batch of B = 2^k samples is 1/B times the bias
+    gradient of each sample alone, exactly: the scale enters at the outputs
+    and every later operation carries a power of two through unchanged."""
+    net = V.MLP(dims, max_batch=B, seed=9)
+    x, t, lab = _data(B, dims, seed=B)
+    rows = []
+    for k in range(B):
+        net.loss_grad(x[k:k + 1], t[k:k + 1], lab[k:k + 1], 0.5)
+        rows.append(np.concatenate([db for _, db in net.layers(net.grads())]))
+    dz = np.array(rows, np.float32) / np.float32(B)
+    ref = np.add.accumulate(dz, axis=0, dtype=np.float32)[-1]
+    net.loss_grad(x, t, lab, 0.5)
+    got = np.concatenate([db for _, db in net.layers(net.grads())])
+    np.testing.assert_array_equal(got, ref)
