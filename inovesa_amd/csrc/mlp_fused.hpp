@@ -388,7 +388,10 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
                     } else {
                         h = gelu(z);
                     }
-                    const uint16_t hb = f2bf(h);
+                    // (columns up to whole fragments stay zero: 0 times an
+                    // infinite activation is no number, and the next
+                    // product's zero weights would carry it to every output)
+                    const uint16_t hb = j < N ? f2bf(h) : (uint16_t)0;
                     nxt[row(s) * n.as + j] = hb;
                     // (samples past the batch add nothing to the gradients)
                     packed[r] = r0 + s < a.B ? hb : (uint16_t)0;
@@ -461,7 +464,8 @@ mlp_rows_kernel(MlpNet n, MlpRowsArgs a)
             for (uint32_t r = 0; r < (uint32_t)RR; r++) {
                 const uint32_t s = s0 + r;
                 float& g = grad[s * (NP + 4u) + j];
-                const float dz = r0 + s < a.B ? acc[r] * g : 0.0f;
+                // (columns up to whole fragments: zeros, as forward)
+                const float dz = r0 + s < a.B && j < n.w[l] ? acc[r] * g : 0.0f;
                 g = dz;
                 packed[r] = f2bf(dz);
                 nxt[row(s) * n.as + j] = packed[r];

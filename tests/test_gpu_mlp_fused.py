@@ -123,3 +123,33 @@ def test_bias_gradients_add_the_samples_in_order(V, dims, B):
     net.loss_grad(x, t, lab, 0.5)
     got = np.concatenate([db for _, db in net.layers(net.grads())])
     np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("dims", [(3, 48, 33, 9), (3, 40, 64, 40, 5),
+                                  (3, 64, 32, 9), (3, 1200, 1100, 9)])
+def test_overflow_stays_infinite(V, dims):
+    """An activation or gradient that overflows is an infinity in what
+    follows from it, also where a width is no whole number of fragments and
+    zero weights meet it in the columns between.  All weights, inputs and
+    biases are positive, so no infinity meets its opposite or a zero."""
+    net = V.MLP(dims, max_batch=40, seed=1)
+    rng = np.random.default_rng(2)
+    p = (0.01 + 0.01 * rng.random(net.params().size)).astype(np.float32)
+    big = p.copy()
+    big[:dims[0]] = 3e38            # the first hidden unit's weights
+    net.set_params(big)
+    x = np.full((20, dims[0]), 1e-30, np.float32)
+    x[7] = 1.0
+    y = net.forward(x)
+    assert np.all(np.isposinf(y[7]))
+    assert np.all(np.isfinite(np.delete(y, 7, axis=0)))
+    # a target far away: the output gradient overflows
+    net.set_params(p)
+    x[:] = 0.5
+    t = np.zeros((20, dims[-1] - 1), np.float32)
+    t[7] = -3e38
+    net.loss_grad(x, t, np.zeros(20, np.float32))
+    for l, (dW, db) in enumerate(net.layers(net.grads())):
+        # (not the row of the label, whose gradient is finite)
+        out = slice(None, -1 if l + 2 == len(dims) else None)
+        assert np.all(np.isposinf(dW[out])) and np.all(np.isposinf(db[out]))
