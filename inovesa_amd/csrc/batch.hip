@@ -368,14 +368,27 @@ int ensure_all(vfps_batch* b)
         start[i] = o;
         o += descs[i].n;
     }
-    VFPS_HIP(hipMalloc(&b->start_d, sizeof(uint32_t) * k));
-    VFPS_HIP(hipMemcpy(b->start_d, start.data(), sizeof(uint32_t) * k,
-                       hipMemcpyHostToDevice));
+    // (the batch gets them when both are whole: a kernel follows the pointers
+    // in the descriptors)
+    uint32_t* st = nullptr;
     InstDesc* d = nullptr;
-    VFPS_HIP(hipMalloc(&d, sizeof(InstDesc) * k));
+    hipError_t e = hipMalloc(&st, sizeof(uint32_t) * k);
+    if (e == hipSuccess) e = hipMalloc(&d, sizeof(InstDesc) * k);
+    if (e == hipSuccess) {
+        e = hipMemcpy(st, start.data(), sizeof(uint32_t) * k,
+                      hipMemcpyHostToDevice);
+    }
+    if (e == hipSuccess) {
+        e = hipMemcpy(d, descs.data(), sizeof(InstDesc) * k,
+                      hipMemcpyHostToDevice);
+    }
+    if (e != hipSuccess) {
+        hipFree(st);
+        hipFree(d);
+        return fail(VFPS_ERR_HIP, hipGetErrorString(e));
+    }
+    b->start_d = st;
     b->all_d = d;
-    VFPS_HIP(hipMemcpy(d, descs.data(), sizeof(InstDesc) * k,
-                       hipMemcpyHostToDevice));
     return VFPS_OK;
 }
 

@@ -1,5 +1,6 @@
 """Build the C++ test program of the reference-shaped interface
-(include/inovesa_amd.hpp) against the in-tree libvfps.so with g++."""
+(include/inovesa_amd.hpp) against the in-tree libvfps.so with g++, and the
+library of failing allocations (hip_faults.c) with gcc."""
 import os
 import subprocess
 
@@ -7,6 +8,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
 SRC = os.path.join(HERE, "test_reference_api.cpp")
 BIN = os.path.join(HERE, "test_reference_api.bin")
+FAULTS = os.path.join(HERE, "libhip_faults.so")
 
 
 def command(out=BIN, syntax_only=False):
@@ -21,6 +23,9 @@ def command(out=BIN, syntax_only=False):
 
 def build(out=BIN):
     subprocess.run(command(out), check=True)
+    subprocess.run(["gcc", "-O2", "-Wall", "-Wextra", "-shared", "-fPIC",
+                    os.path.join(HERE, "hip_faults.c"), "-ldl", "-o", FAULTS],
+                   check=True)
     return out
 
 
