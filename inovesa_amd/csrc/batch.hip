@@ -567,22 +567,33 @@ int vfps_batch_run(vfps_batch* b, uint32_t nsteps)
     // its own) and every member's error flag, in one launch
     static_assert(DEV_STAGE_BYTES >= sizeof(uint32_t) * 0xFFFFu,
                   "an error flag per instance");
+    VFPS_TRY_BEGIN
+    const size_t count = b->members.size();
     DevStage stage(b->dev);
     uint32_t* err = stage.get<uint32_t>();
-    if (!err) return fail(VFPS_ERR_NOMEM, "batch: pinned memory");
-    if ((rc = launch_step_finalize(b->all_d, (uint32_t)b->members.size(),
-                                   b->parity, st, err, nsteps > 0)) != VFPS_OK) {
+    if ((rc = launch_step_finalize(b->all_d, (uint32_t)count, b->parity, st, err,
+                                   nsteps > 0)) != VFPS_OK) {
         return rc;
+    }
+    std::vector<uint32_t> copied(err ? 0 : count);
+    if (!err) {
+        // (no pinned memory: copies)
+        for (size_t i = 0; i < count; i++) {
+            VFPS_HIP(hipMemcpyAsync(&copied[i], b->members[i]->err,
+                                    sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        }
+        err = copied.data();
     }
     VFPS_HIP(hipStreamSynchronize(st));
     sync_parity(b);
-    for (size_t i = 0; i < b->members.size(); i++) {
+    for (size_t i = 0; i < count; i++) {
         if (err[i]) {
             return fail(VFPS_ERR_INVALID, "batch step: a tap fell outside the "
                                           "halo rows (internal error)");
         }
     }
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 int vfps_batch_prepare(vfps_batch* b, uint32_t nsteps)
@@ -642,8 +653,18 @@ int vfps_batch_get_projections(vfps_batch* b, float* out)
     constexpr size_t most = DEV_STAGE_BYTES / sizeof(float);
     DevStage stage(b->dev);
     float* buf = stage.get<float>();
-    if (!buf) return fail(VFPS_ERR_NOMEM, "batch: pinned memory");
     const uint32_t k = (uint32_t)b->members.size();
+    if (!buf) {
+        // (no pinned memory: a copy per instance)
+        for (auto* s : b->members) {
+            const vfps_mesh* cur = (s->parity & 1u) ? s->t2 : s->t1;
+            VFPS_HIP(hipMemcpyAsync(out, cur->proj, sizeof(float) * s->desc.n,
+                                    hipMemcpyDeviceToHost, st));
+            out += s->desc.n;
+        }
+        VFPS_HIP(hipStreamSynchronize(st));
+        return VFPS_OK;
+    }
     for (uint32_t i = 0; i < k;) {
         uint32_t e = i;
         size_t words = 0;
@@ -678,8 +699,11 @@ int vfps_batch_get_csr_histories(vfps_batch* b, uint32_t first, uint32_t count,
     if (rc != VFPS_OK) return rc;
     const uint32_t k = (uint32_t)b->members.size();
     const size_t most = DEV_STAGE_BYTES / sizeof(float) / count;
-    if (most == 0) {
-        // a history longer than the staging: a copy per instance
+    DevStage stage(b->dev);
+    float* buf = most ? stage.get<float>() : nullptr;
+    if (!buf) {
+        // a history longer than the staging, or no staging: a copy per
+        // instance
         for (auto* s : b->members) {
             VFPS_HIP(hipMemcpyAsync(out, s->csr_hist + first,
                                     sizeof(float) * count,
@@ -689,9 +713,6 @@ int vfps_batch_get_csr_histories(vfps_batch* b, uint32_t first, uint32_t count,
         VFPS_HIP(hipStreamSynchronize(st));
         return VFPS_OK;
     }
-    DevStage stage(b->dev);
-    float* buf = stage.get<float>();
-    if (!buf) return fail(VFPS_ERR_NOMEM, "batch: pinned memory");
     for (uint32_t i = 0; i < k;) {
         const uint32_t m = (uint32_t)std::min<size_t>(most, k - i);
         hipLaunchKernelGGL(batch_csr_kernel,

@@ -83,13 +83,14 @@ namespace vfps_impl {
 // launch that fills it to the copy out of it.  A kernel writes its results
 // there itself, so that a call returning a few arrays costs one launch and
 // one wait where a copy per array costs about 10 us each.  Allocated on first
-// use, freed with the handle.
+// use, freed with the handle.  Where it cannot be had (no memory to pin), every
+// call copies its results instead.
 constexpr size_t DEV_STAGE_BYTES = 4u << 20;
 
 class DevStage {
 public:
     explicit DevStage(vfps_dev* dev) : lock_(dev->stage_mu), dev_(dev) {}
-    // null if the allocation failed
+    // null if the allocation failed (tried again by the next call)
     template <typename T>
     T* get()
     {
@@ -97,6 +98,7 @@ public:
             hipHostMalloc(&dev_->stage, DEV_STAGE_BYTES,
                           hipHostMallocDefault) != hipSuccess) {
             dev_->stage = nullptr;
+            (void)hipGetLastError();  // (the launches that follow check it)
         }
         return static_cast<T*>(dev_->stage);
     }

@@ -671,14 +671,14 @@ int vfps_mlp_forward(vfps_mlp* m, const float* x, uint32_t B, float* y)
         // host memory: no copy launches around it (3-256-256-256-65, 512
         // samples: two copies were half of the call)
         DevStage stage(m->dev);
-        float* xs = stage.get<float>();
-        if (!xs) return fail(VFPS_ERR_NOMEM, "vfps_mlp_forward: pinned memory");
-        float* ys = xs + nx;
-        std::memcpy(xs, x, sizeof(float) * nx);
-        if ((rc = fused_forward(m, xs, B, ys)) != VFPS_OK) return rc;
-        VFPS_HIP(hipStreamSynchronize(st));
-        std::memcpy(y, ys, sizeof(float) * ny);
-        return VFPS_OK;
+        if (float* xs = stage.get<float>()) {
+            float* ys = xs + nx;
+            std::memcpy(xs, x, sizeof(float) * nx);
+            if ((rc = fused_forward(m, xs, B, ys)) != VFPS_OK) return rc;
+            VFPS_HIP(hipStreamSynchronize(st));
+            std::memcpy(y, ys, sizeof(float) * ny);
+            return VFPS_OK;
+        }
     }
     VFPS_HIP(hipMemcpyAsync(m->x, x, sizeof(float) * nx, hipMemcpyHostToDevice,
                             st));

@@ -365,7 +365,7 @@ __device__ __forceinline__ void variance_of(uint32_t n, const float* p,
     }
 }
 
-// one workgroup per bunch; out: [nb][3], pinned
+// one workgroup per bunch; out: [nb][3]
 __global__ void __launch_bounds__(256)
 variance_kernel(uint32_t n, const float* proj, float axis_min, float delta,
                 const float* fill_set, const double* filling, float* out)
@@ -377,8 +377,9 @@ variance_kernel(uint32_t n, const float* proj, float axis_min, float delta,
 }
 
 // The outstep quantities of a one-bunch mesh from its projections
-// (proj: x, then y), into pinned memory: the FP64 charge integral, then
-// 2 x (mean, variance, root), then both projections.  The same sums as
+// (proj: x, then y): the FP64 charge integral, then
+// 2 x (mean, variance, root), then both projections (out: that many words,
+// pinned or on the device).  The same sums as
 // integrate_kernel and variance_kernel make, in one launch.
 __global__ void __launch_bounds__(256)
 moments_kernel(uint32_t n, const float* proj, const float* ws, float min0,
@@ -518,26 +519,45 @@ int upload_floats(vfps_dev* dev, float* dst, const float* src, size_t n)
     return VFPS_OK;
 }
 
+// `bytes` of results, written by the kernel that launch(pointer) starts, to
+// host memory: through the pinned buffer, or, where that is too small or
+// missing, through device memory of their own.
+template <typename F>
+static int read_results(vfps_dev* dev, void* host, size_t bytes, F&& launch)
+{
+    DevStage stage(dev);
+    char* buf = bytes <= DEV_STAGE_BYTES ? stage.get<char>() : nullptr;
+    char* tmp = nullptr;
+    if (!buf) VFPS_HIP(hipMalloc(&tmp, bytes));
+    launch(buf ? buf : tmp);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && tmp) {
+        e = hipMemcpyAsync(host, tmp, bytes, hipMemcpyDeviceToHost, dev->stream);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
+    if (tmp) hipFree(tmp);
+    if (e != hipSuccess) return fail(VFPS_ERR_HIP, hipGetErrorString(e));
+    if (buf) std::memcpy(host, buf, bytes);
+    return VFPS_OK;
+}
+
 int mesh_moments(vfps_mesh* m, float* xproj, float* yproj, double* fill,
                  float* mom)
 {
     const uint32_t n = m->n;
-    VFPS_CHECK_ARG(m->nb == 1 && sizeof(double) + sizeof(float) * (6 + 2 * (size_t)n) <=
-                                     DEV_STAGE_BYTES,
-                   "moments: one bunch");
+    VFPS_CHECK_ARG(m->nb == 1, "moments: one bunch");
     int rc = vfps_mesh_project_y(m);
     if (rc != VFPS_OK) return rc;
-    DevStage stage(m->dev);
-    double* out = stage.get<double>();
-    if (!out) return fail(VFPS_ERR_NOMEM, "moments: pinned memory");
-    hipStream_t st = m->dev->stream;
-    hipLaunchKernelGGL(moments_kernel, dim3(1), dim3(256), 0, st, n, m->proj,
-                       m->ws, m->ax0.min, m->ax0.delta, m->ax1.min,
-                       m->ax1.delta, m->fill_set_d, m->filling, m->integral,
-                       out);
-    VFPS_HIP(hipGetLastError());
-    VFPS_HIP(hipStreamSynchronize(st));
-    const float* of = reinterpret_cast<const float*>(out + 1);
+    // the charge integral, then 6 + 2 n floats
+    std::vector<double> out(1 + (6 + 2 * (size_t)n + 1) / 2);
+    rc = read_results(m->dev, out.data(), sizeof(double) * out.size(), [&](char* o) {
+        hipLaunchKernelGGL(moments_kernel, dim3(1), dim3(256), 0, m->dev->stream,
+                           n, m->proj, m->ws, m->ax0.min, m->ax0.delta,
+                           m->ax1.min, m->ax1.delta, m->fill_set_d, m->filling,
+                           m->integral, reinterpret_cast<double*>(o));
+    });
+    if (rc != VFPS_OK) return rc;
+    const float* of = reinterpret_cast<const float*>(out.data() + 1);
     *fill = out[0];
     std::memcpy(mom, of, 6 * sizeof(float));
     if (xproj) std::memcpy(xproj, of + 6, sizeof(float) * n);
@@ -901,16 +921,15 @@ int vfps_mesh_variance(vfps_mesh* m, int axis, float* mean, float* var,
                    "vfps_mesh_variance: bad argument");
     VFPS_TRY_BEGIN
     const Ruler& ax = axis == 0 ? m->ax0 : m->ax1;
-    DevStage stage(m->dev);
-    const size_t bytes = sizeof(float) * 3 * (size_t)m->nb;
-    float* h = bytes <= DEV_STAGE_BYTES ? stage.get<float>() : nullptr;
-    if (!h) return fail(VFPS_ERR_NOMEM, "variance: pinned memory");
-    hipLaunchKernelGGL(variance_kernel, dim3(m->nb), dim3(256), 0,
-                       m->dev->stream, m->n,
-                       m->proj + (size_t)axis * m->nb * m->n, ax.min, ax.delta,
-                       m->fill_set_d, m->filling, h);
-    VFPS_HIP(hipGetLastError());
-    VFPS_HIP(hipStreamSynchronize(m->dev->stream));
+    std::vector<float> h(3 * (size_t)m->nb);
+    int rc = read_results(m->dev, h.data(), sizeof(float) * h.size(), [&](char* o) {
+        hipLaunchKernelGGL(variance_kernel, dim3(m->nb), dim3(256), 0,
+                           m->dev->stream, m->n,
+                           m->proj + (size_t)axis * m->nb * m->n, ax.min,
+                           ax.delta, m->fill_set_d, m->filling,
+                           reinterpret_cast<float*>(o));
+    });
+    if (rc != VFPS_OK) return rc;
     for (uint32_t b = 0; b < m->nb; b++) {
         if (mean) mean[b] = h[3 * b];
         if (var) var[b] = h[3 * b + 1];

@@ -68,3 +68,53 @@ def test_batch_descriptors():
         for a, e in zip(b.projections(), expect[1]):
             np.testing.assert_array_equal(a, e)
     """)
+
+
+def test_results_without_the_pinned_buffer():
+    """Where the 4 MB read-back buffer cannot be pinned, every call copies its
+    results instead and returns the same."""
+    run_alone("""
+    rng = np.random.default_rng(1)
+    x = rng.random((20, 3)).astype(np.float32)
+
+    def everything():
+        out = {}
+        b = make_batch()
+        b.run(7)
+        out["batch csr"] = b.csr_histories(0, 7)
+        out["batch profiles"] = np.concatenate(b.projections())
+        desc, d = kick_drift_config(n=60, steps_per_ts=500)
+        zw, zc = impedances(d)
+        st = V.Step(desc, initial_mesh(60, seed=4), zw, zc)
+        st.record(5)
+        st.run(5)
+        for k, v in st.moments().items():
+            out["moments " + k] = v
+        out["mesh"], out["profile"], out["wake"] = st.mesh()
+        out["history"] = st.history()[0]
+        ps = V.PhaseSpace(40, -6.0, 6.0, 1e-3, -6.0, 6.0, 1e5,
+                          filling=[0.25, 0.75])
+        out["variance"] = np.concatenate(
+            [np.ravel(v) for axis in (0, 1) for v in ps.variance(axis)])
+        out["integral"] = np.append(*ps.integrate())
+        f = V.ElectricField(ps, V.Impedance(256, 1e12,
+                                            table=np.ones(256, np.complex64)),
+                            [0, 1], 50)
+        out["potential"] = f.wakePotential()
+        out["csr"] = f.updateCSR(0.0)[0]
+        net = V.MLP((3, 40, 9), max_batch=20, seed=2)
+        out["net"] = net.forward(x)
+        return out
+
+    faults.hip_faults_pinned(1 << 20)
+    without = everything()
+    seen = faults.hip_faults_refused()
+    assert seen >= 10
+    faults.hip_faults_pinned(0)
+    with_it = everything()
+    assert faults.hip_faults_refused() == seen
+    assert without.keys() == with_it.keys()
+    for k in without:
+        for a, e in zip(np.atleast_1d(without[k]), np.atleast_1d(with_it[k])):
+            np.testing.assert_array_equal(a, e, err_msg=k)
+    """)
