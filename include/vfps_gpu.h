@@ -564,8 +564,9 @@ VFPS_API int vfps_batch_retile_size_strip(vfps_batch* b, uint32_t n,
  * out[7], if nout >= 8: tiles per strip, 0 outside the strip form) */
 VFPS_API int vfps_batch_config(vfps_batch* b, uint32_t inst, uint32_t* out,
                                uint32_t nout);
-/* average time of one batch step (all launches), HIP events on the device
- * stream; advances the state by nsteps */
+/* average time of one batch step (all launches, in the schedule of
+ * vfps_batch_run, captured before), HIP events on the device stream; advances
+ * the state by nsteps */
 VFPS_API int vfps_batch_timing(vfps_batch* b, uint32_t nsteps, float* ms_step);
 /* Autotuner: per mesh size, time every tile height T in {1,2,4,8,16},
  * workgroup size in {128,256,512} and launch form (one workgroup per tile;

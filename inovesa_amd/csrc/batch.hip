@@ -433,6 +433,52 @@ int batch_graph(vfps_batch* b, uint32_t steps, uint32_t p, hipGraphExec_t* out)
     return VFPS_OK;
 }
 
+// whether the members ask for host launches (no_graph)
+bool host_launches(const vfps_batch* b)
+{
+    return !b->members.empty() && b->members[0]->desc.no_graph;
+}
+
+// the captured runs enqueue_steps(b, nsteps) replays, captured now
+int prepare_steps(vfps_batch* b, uint32_t nsteps)
+{
+    hipGraphExec_t g = nullptr;
+    int rc;
+    if (nsteps >= BATCH_GRAPH &&
+        (rc = batch_graph(b, BATCH_GRAPH, b->parity, &g)) != VFPS_OK) {
+        return rc;
+    }
+    if (nsteps % BATCH_GRAPH &&
+        (rc = batch_graph(b, nsteps % BATCH_GRAPH, b->parity, &g)) != VFPS_OK) {
+        return rc;
+    }
+    return VFPS_OK;
+}
+
+// `nsteps` steps of every instance on the device stream, as every run makes
+// them; the parity follows
+int enqueue_steps(vfps_batch* b, uint32_t nsteps)
+{
+    uint32_t left = nsteps;
+    int rc;
+    while (host_launches(b) && left > 0) {
+        if ((rc = launch_step(b, b->parity)) != VFPS_OK) return rc;
+        b->parity ^= 1u;
+        left--;
+    }
+    // captured runs: full ones of BATCH_GRAPH steps (even, so the parity
+    // stays), then one of the remaining steps
+    while (left > 0) {
+        const uint32_t k = left >= BATCH_GRAPH ? BATCH_GRAPH : left;
+        hipGraphExec_t g = nullptr;
+        if ((rc = batch_graph(b, k, b->parity, &g)) != VFPS_OK) return rc;
+        VFPS_HIP(hipGraphLaunch(g, b->dev->stream));
+        left -= k;
+        b->parity ^= (k & 1u);
+    }
+    return VFPS_OK;
+}
+
 void sync_parity(vfps_batch* b)
 {
     for (auto* s : b->members) s->parity = b->parity;
@@ -543,26 +589,9 @@ int vfps_batch_run(vfps_batch* b, uint32_t nsteps)
 {
     VFPS_CHECK_ARG(b, "vfps_batch_run: NULL batch");
     hipStream_t st = b->dev->stream;
-    uint32_t left = nsteps;
     int rc = ensure_all(b);
     if (rc != VFPS_OK) return rc;
-    // host launches when the members ask for them (no_graph)
-    const bool host = !b->members.empty() && b->members[0]->desc.no_graph;
-    while (host && left > 0) {
-        if ((rc = launch_step(b, b->parity)) != VFPS_OK) return rc;
-        b->parity ^= 1u;
-        left--;
-    }
-    // captured runs: full ones of BATCH_GRAPH steps (even, so the parity
-    // stays), then one of the remaining steps
-    while (left > 0) {
-        const uint32_t k = left >= BATCH_GRAPH ? BATCH_GRAPH : left;
-        hipGraphExec_t g = nullptr;
-        if ((rc = batch_graph(b, k, b->parity, &g)) != VFPS_OK) return rc;
-        VFPS_HIP(hipGraphLaunch(g, st));
-        left -= k;
-        b->parity ^= (k & 1u);
-    }
+    if ((rc = enqueue_steps(b, nsteps)) != VFPS_OK) return rc;
     // the last step's CSR powers (the FFT form's field kernel has recorded
     // its own) and every member's error flag, in one launch
     static_assert(DEV_STAGE_BYTES >= sizeof(uint32_t) * 0xFFFFu,
@@ -600,16 +629,8 @@ int vfps_batch_prepare(vfps_batch* b, uint32_t nsteps)
 {
     VFPS_CHECK_ARG(b, "vfps_batch_prepare: NULL batch");
     VFPS_TRY_BEGIN
-    hipGraphExec_t g = nullptr;
-    int rc;
-    if (nsteps >= BATCH_GRAPH &&
-        (rc = batch_graph(b, BATCH_GRAPH, b->parity, &g)) != VFPS_OK) {
-        return rc;
-    }
-    if (nsteps % BATCH_GRAPH &&
-        (rc = batch_graph(b, nsteps % BATCH_GRAPH, b->parity, &g)) != VFPS_OK) {
-        return rc;
-    }
+    int rc = prepare_steps(b, nsteps);
+    if (rc != VFPS_OK) return rc;
     VFPS_HIP(hipStreamSynchronize(b->dev->stream));
     return VFPS_OK;
     VFPS_TRY_END
@@ -839,28 +860,28 @@ int vfps_batch_retile_size_strip(vfps_batch* b, uint32_t n, uint32_t tile_rows,
 int vfps_batch_timing(vfps_batch* b, uint32_t nsteps, float* ms_step)
 {
     VFPS_CHECK_ARG(b && nsteps > 0 && ms_step, "vfps_batch_timing: bad argument");
+    VFPS_TRY_BEGIN
     hipStream_t st = b->dev->stream;
+    // the steps as a run makes them (a join of the launch groups after each
+    // would be another time: 16 each of 128^2 to 512^2, 66 us against 52)
+    int rc = host_launches(b) ? VFPS_OK : prepare_steps(b, nsteps);
+    if (rc != VFPS_OK) return rc;
     hipEvent_t e0, e1;
     VFPS_HIP(hipEventCreate(&e0));
     VFPS_HIP(hipEventCreate(&e1));
-    double tot = 0;
-    int rc = VFPS_OK;
-    for (uint32_t k = 0; k < nsteps && rc == VFPS_OK; k++) {
-        hipEventRecord(e0, st);
-        rc = launch_step(b, b->parity);
-        hipEventRecord(e1, st);
-        hipEventSynchronize(e1);
-        float ms = 0;
-        hipEventElapsedTime(&ms, e0, e1);
-        tot += ms;
-        b->parity ^= 1u;
-    }
+    float ms = 0;
+    hipEventRecord(e0, st);
+    rc = enqueue_steps(b, nsteps);
+    hipEventRecord(e1, st);
+    hipEventSynchronize(e1);
+    hipEventElapsedTime(&ms, e0, e1);
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     sync_parity(b);
     if (rc != VFPS_OK) return rc;
-    *ms_step = (float)(tot / nsteps);
+    *ms_step = ms / (float)nsteps;
     return VFPS_OK;
+    VFPS_TRY_END
 }
 
 // Choose the tile height and workgroup size per mesh size: for each size
@@ -1074,27 +1095,30 @@ int vfps_batch_autotune(vfps_batch* b, uint32_t steps, float* table,
     }
     // A persistent launch holds every resident slot, so it can starve the
     // other size classes' launches, which run beside it: with several
-    // classes, a persistent choice must also win on the whole batch.
+    // classes, a persistent choice must also win on the whole batch, in the
+    // schedule that runs have (every group a captured chain).
     if (rc == VFPS_OK && choices.size() > 1) {
         auto time_all = [&](float* us) -> int {
             vfps_batch sub;
             sub.dev = b->dev;
             sub.fork = b->fork;
             sub.members = b->members;
+            sub.parity = par;
             int r1 = build_groups(&sub);
             float ms = 0;
+            // warm up (and capture), then time; an even number of steps, so
+            // both start at the same parity
+            if (r1 == VFPS_OK) r1 = enqueue_steps(&sub, 4 * even);
             if (r1 == VFPS_OK) {
-                for (uint32_t k = 0; k < 2 && r1 == VFPS_OK; k++) {
-                    r1 = launch_step(&sub, (par + k) & 1u);
-                }
                 hipEventRecord(e0, st);
-                for (uint32_t k = 0; k < 4 * even && r1 == VFPS_OK; k++) {
-                    r1 = launch_step(&sub, (par + k) & 1u);
-                }
+                r1 = enqueue_steps(&sub, 4 * even);
                 hipEventRecord(e1, st);
                 hipEventSynchronize(e1);
                 hipEventElapsedTime(&ms, e0, e1);
             }
+            hipStreamSynchronize(st);
+            const int r2 = drop_graph(&sub);
+            if (r1 == VFPS_OK) r1 = r2;
             free_groups(&sub);
             sub.fork = nullptr;
             sub.members.clear();

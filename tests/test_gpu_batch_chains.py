@@ -32,3 +32,33 @@ def test_chains_equal_single_steps(sizes, fft_every, runs):
         for x, y in zip(b.mesh(k), s.mesh()):
             assert np.array_equal(x, y), k
         assert np.array_equal(b.history(k)[0], s.history()[0]), k
+
+
+def test_timing_is_the_time_of_a_run():
+    """Batch.timing gives the step time that a run has (launch groups as
+    chains), not that of steps joined one by one: over many groups these lie
+    far apart, so the bound on wall-clock times can be wide.  It advances the
+    state by as many steps."""
+    import time
+
+    import inovesa_amd as V
+    from inovesa_amd.workloads import batched_scan_config, impedances
+    sizes = (64, 96, 128, 160, 192, 256, 320, 384, 448, 512)
+    inst = [(desc, init, *impedances(d)) for desc, d, init in
+            batched_scan_config(sizes=sizes, per_size=1, seed=4)]
+    a, b = (V.Batch(*[[i[k] for i in inst] for k in range(4)])
+            for _ in range(2))
+    groups = a.info()["launch_groups"]
+    steps = 192
+    a.run(steps)
+    b.timing(steps)
+    for k in range(len(inst)):
+        assert np.array_equal(a.mesh(k)[0], b.mesh(k)[0]), k
+    run, timing = [], []
+    for _ in range(3):
+        t0 = time.perf_counter()
+        a.run(steps)
+        run.append((time.perf_counter() - t0) / steps * 1e6)
+        timing.append(b.timing(steps) * 1e3)
+    print(f"{groups} groups: run {min(run):.1f}, timing {min(timing):.1f} us")
+    assert min(timing) <= 1.5 * min(run)
