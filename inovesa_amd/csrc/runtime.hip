@@ -109,7 +109,8 @@ project_x_kernel(uint32_t rows, uint32_t n, uint32_t rows_per_wg,
                  const float* __restrict__ data,
                  const float* __restrict__ ws, float* __restrict__ proj)
 {
-    extern __shared__ __align__(16) float px[];   // rows_per_wg * px_stride(n)
+    extern __shared__ __align__(16) float px[];   // (the last row: without
+                                                  // the 4 words after it)
     const uint32_t r0 = blockIdx.x * rows_per_wg;
     const uint32_t nr = min(rows_per_wg, rows - r0);
     const uint32_t stride = px_stride(n);
@@ -437,13 +438,15 @@ int launch_project_x(vfps_mesh* m, const float* src, float* proj)
     const uint32_t rows = m->nb * m->n;
     // rows per workgroup: enough workgroups for the CUs (two meshes of 256^2
     // in rows of 16 were 32 of them), at most PX_ROWS and what the LDS holds
-    const size_t row_bytes = sizeof(float) * px_stride(m->n);
+    // (the longest row of all fills it: n = 40960)
+    const size_t stride = px_stride(m->n), words = m->dev->lds_max / sizeof(float);
+    const size_t last = stride - 4;
+    VFPS_CHECK_ARG(last <= words,
+                   "updateXProjection: a mesh row exceeds the LDS");
     const size_t share = ceil_div(rows, (size_t)std::max(m->dev->ncu, 1));
     const uint32_t rpw = (uint32_t)std::max<size_t>(
-        1, std::min({share, (size_t)PX_ROWS, m->dev->lds_max / row_bytes}));
-    const size_t lds = row_bytes * rpw;
-    VFPS_CHECK_ARG(lds <= m->dev->lds_max,
-                   "updateXProjection: a mesh row exceeds the LDS");
+        1, std::min({share, (size_t)PX_ROWS, (words - last) / stride + 1}));
+    const size_t lds = sizeof(float) * ((rpw - 1) * stride + last);
     if (lds > 65536) {
         VFPS_HIP(hipFuncSetAttribute(
             reinterpret_cast<const void*>(&project_x_kernel),

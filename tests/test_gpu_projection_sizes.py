@@ -47,3 +47,24 @@ def test_step_and_batch_projection(n):
     bm, bp, _ = b.mesh(0)
     np.testing.assert_array_equal(bm, mesh)
     np.testing.assert_array_equal(bp, proj)
+
+
+@pytest.mark.parametrize("n", [8180, 13641, 40956])
+def test_longest_rows(n):
+    """Rows that fill a workgroup's LDS: several to one, and the longest row
+    that leaves no room beside it (6.7 GB of mesh)."""
+    import inovesa_amd as V
+    ps = V.PhaseSpace(n, -6.0, 6.0, 1e-3, -6.0, 6.0, 1e6)
+    ps.updateXProjection()
+    proj, ws, mesh = ps.getProjection(0)[0], ps.simpsonWeights(), ps.getData()[0]
+    for r in (0, 1, n // 2 - 1, n // 2, n - 2, n - 1):
+        seq = np.add.accumulate(np.append(np.float32(0), mesh[r] * ws),
+                                dtype=np.float32)
+        assert proj[r] == seq[-1], r
+    assert proj[n // 2] > 0
+
+
+def test_a_row_beyond_the_lds_is_refused():
+    import inovesa_amd as V
+    with pytest.raises(V.VfpsInvalid):
+        V.PhaseSpace(40961, -6.0, 6.0, 1e-3, -6.0, 6.0, 1e6)
