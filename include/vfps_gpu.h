@@ -485,6 +485,10 @@ VFPS_API int vfps_step_phases(vfps_step* s, double* ns_out, uint32_t nout);
  * [2] tile rows, [3] threads, [4] LDS buffer rows, [5] LDS bytes (nout >= 6),
  * [6] persistent launch in a batch (nout >= 7) */
 VFPS_API int vfps_step_config(vfps_step* s, uint32_t* out, uint32_t nout);
+/* the FP64 Toeplitz kernels of a direct-wake step as its device made them
+ * (g and h of vfps_toeplitz_kernels, 2n-1 doubles each; either may be NULL,
+ * and must be where the step has no wake or no CSR) */
+VFPS_API int vfps_step_get_toeplitz(vfps_step* s, double* g, double* h);
 
 /* ---- batch of independent meshes ------------------------------------- *
  * No reference counterpart: a scan over currents or chamber gaps runs the

@@ -179,6 +179,7 @@ _SIGS = {
     "vfps_step_timing": (_int, [_vp, _u32, _vp, _vp, _vp]),
     "vfps_step_phases": (_int, [_vp, _vp, _u32]),
     "vfps_step_config": (_int, [_vp, _vp, _u32]),
+    "vfps_step_get_toeplitz": (_int, [_vp, _vp, _vp]),
     "vfps_batch_create": (_int, [_vp, _u32, C.POINTER(StepDesc), _vp, _vp,
                                  _vp, _vp]),
     "vfps_batch_destroy": (_int, [_vp]),

@@ -231,7 +231,8 @@ void toeplitz_tables(uint32_t n, uint32_t M, const float2* Z,
 // The same tables on the device: a workgroup per entry d, its threads the
 // terms k = t, t + 256, ... (FP64, summed per thread and then over the
 // workgroup, so the rounding error is no larger than the host's running
-// sum).  tw_n[t] = exp(-2 pi i t/N), t < M.  On the host the tables were half
+// sum; 1e-13 of the largest entry, tests/test_gpu_toeplitz.py).
+// tw_n[t] = exp(-2 pi i t/N), t < M.  On the host the tables were half
 // of a step's construction: 0.3 ms of 0.74 at n = 128 with 512 frequencies;
 // here 5.6 us of device time that nothing waits for.
 __global__ void __launch_bounds__(256)
@@ -1369,6 +1370,19 @@ int vfps_step_config(vfps_step* s, uint32_t* out, uint32_t nout)
         out[7] = s->strip;
     }
     return VFPS_OK;
+}
+
+int vfps_step_get_toeplitz(vfps_step* s, double* g, double* h)
+{
+    VFPS_CHECK_ARG(s, "vfps_step_get_toeplitz: NULL step");
+    VFPS_CHECK_ARG((!g || s->wake_g) && (!h || s->csr_h),
+                   "vfps_step_get_toeplitz: the step has no such table");
+    const size_t bytes = sizeof(double) * (2 * (size_t)s->desc.n - 1);
+    ReadBack r[2];
+    size_t k = 0;
+    if (g) r[k++] = {g, s->wake_g, bytes};
+    if (h) r[k++] = {h, s->csr_h, bytes};
+    return k ? read_back(s->dev, r, k) : VFPS_OK;
 }
 
 int vfps_step_phases(vfps_step* s, double* ns_out, uint32_t nout)

@@ -719,6 +719,16 @@ class Step:
         return dict(zip(("fused", "wake_method", "tile_rows", "threads",
                          "stride", "lds_bytes"), (int(v) for v in out)))
 
+    def toeplitz(self, wake=True, csr=True):
+        """The FP64 Toeplitz kernels (g, h) of a direct-wake step as its
+        device made them, index d + n - 1 for |d| < n; None where not asked
+        for."""
+        g = np.zeros(2 * self.n - 1, np.float64) if wake else None
+        h = np.zeros(2 * self.n - 1, np.float64) if csr else None
+        call("vfps_step_get_toeplitz", self.h,
+             _p(g) if wake else None, _p(h) if csr else None)
+        return g, h
+
     def __del__(self):
         h = getattr(self, "h", None)
         if h:
