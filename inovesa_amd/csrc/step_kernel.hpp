@@ -114,7 +114,7 @@ __host__ __device__ inline StepLds step_lds(uint32_t n, uint32_t T, uint32_t str
         L.tile_out = STEP_TILE_IN_BUF;
     } else {
         L.tile_out = w;
-        w += T * (n + 4);
+        w += step_round4(T * (n + 4));
     }
     L.offw = w;
     w += step_round4(stride);
@@ -231,9 +231,26 @@ __device__ __forceinline__ void lds_window16(const float* s, int32_t lo,
     }
 }
 
+// Four consecutive values of an LDS row of n from y on: one 16-byte store,
+// or, where rows are no whole groups (n % 4 != 0), those inside the row word
+// by word.
+__device__ __forceinline__ void store4(float* row, uint32_t n, uint32_t y,
+                                       vec4f o)
+{
+    if ((n & 3u) == 0u) {
+        *reinterpret_cast<vec4f*>(row + y) = o;
+        return;
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < 4; e++) {
+        if (y + e < n) row[y + e] = o[e];
+    }
+}
+
 // KickMap::apply along y (src/SM/KickMap.cpp:244-267) on local rows
 // [r0, r1) of a row buffer: each thread makes four consecutive outputs of
-// a row from IT+3 consecutive inputs, taps in order (n % 4 == 0).
+// a row (the last group may end past it) from IT+3 consecutive inputs, taps
+// in order.
 template <int IT>
 __device__ __forceinline__ void kick_rows(const float* __restrict__ src,
                                           float* __restrict__ dst, uint32_t n,
@@ -244,7 +261,7 @@ __device__ __forceinline__ void kick_rows(const float* __restrict__ src,
         return;
     }
     const uint32_t bs = blockDim.x;
-    const uint32_t ng = n >> 2;
+    const uint32_t ng = (n + 3u) >> 2;
     const uint32_t drow = bs / ng, dg = bs % ng;
     uint32_t row = (uint32_t)r0 + threadIdx.x / ng;
     uint32_t g = threadIdx.x % ng;
@@ -272,7 +289,7 @@ __device__ __forceinline__ void kick_rows(const float* __restrict__ src,
             }
             o[e] = acc;
         }
-        *reinterpret_cast<vec4f*>(dst + (size_t)row * n + 4 * g) = o;
+        store4(dst + (size_t)row * n, n, 4 * g, o);
         g += dg;
         row += drow;
         if (g >= ng) {
@@ -300,7 +317,7 @@ __device__ __forceinline__ void kick2_rows(const float* __restrict__ src,
         return;
     }
     const uint32_t bs = blockDim.x;
-    const uint32_t ng = n >> 2;
+    const uint32_t ng = (n + 3u) >> 2;
     const uint32_t drow = bs / ng, dg = bs % ng;
     uint32_t row = (uint32_t)r0 + threadIdx.x / ng;
     uint32_t g = threadIdx.x % ng;
@@ -340,7 +357,7 @@ __device__ __forceinline__ void kick2_rows(const float* __restrict__ src,
             }
             o[e] = acc;
         }
-        *reinterpret_cast<vec4f*>(dst + (size_t)row * n + 4 * g) = o;
+        store4(dst + (size_t)row * n, n, 4 * g, o);
         g += dg;
         row += drow;
         if (g >= ng) {
