@@ -151,9 +151,6 @@ constexpr int STEP_LOAD_BATCH = 8;
 // 8.5 -> 8.1 us a step, 16 each of 128^2 to 512^2 in their first tilings 168 ->
 // 153; the occupancy is the same.)
 constexpr int STEP_EARLY_LOADS = 2;
-// most rows whose direct-form dot products a wavefront of a batch sums
-// together
-constexpr int STEP_DOT_ROWS = 4;
 // largest workgroup
 constexpr uint32_t STEP_MAX_THREADS = 512;
 // block-map entry of a padding workgroup
@@ -436,6 +433,8 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                                           uint32_t parity, float* lds,
                                           StepShared& sh)
 {
+    // whether the x projection of any row length keeps 32 values ahead (G)
+    constexpr bool AHEAD32 = ONE_MESH || (!DIRECT && MAXC != 2);
     float& s00_sh = sh.s00;
     uint32_t& slot_sh = sh.slot;
     uint32_t& cnt_sh = sh.cnt;
@@ -774,77 +773,7 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
         return v;
     };
     double csr_q = 0.0;
-    if (!ONE_MESH && DIRECT && (wake || csr)) {
-        // A batch reads the windows from the tables in global memory.  A job
-        // is up to STEP_DOT_ROWS consecutive rows of one table, sized so that
-        // the jobs spread over the wavefronts: their loads go out together and
-        // each value of the profile serves all of them.  (One row at a time,
-        // the two wavefronts of a 128^2 tile of two rows waited for four
-        // trips to L2 one after the other: 128 steps of 64 meshes of 128^2
-        // took 1.96 ms, now 1.85.)  A row's sum keeps its order.
-        const int nwk = wake ? lr1 - lr0 : 0;
-        const int ncsr = csr ? rows_out : 0;
-        const int ns00 = need_s00 && wake ? 1 : 0;
-        const int rj = min(STEP_DOT_ROWS,
-                           max(1, (nwk + ncsr + ns00 + (int)nw - 1) / (int)nw));
-        const int nwj = (nwk + rj - 1) / rj, ncj = (ncsr + rj - 1) / rj;
-        for (int job = (int)wave; job < nwj + ncj + ns00; job += (int)nw) {
-            const int which = job < nwj ? 0 : (job < nwj + ncj ? 1 : 2);
-            const int first = which == 0 ? job * rj : (job - nwj) * rj;
-            const int rows = which == 2 ? 1
-                             : which == 0 ? min(rj, nwk - first)
-                                          : min(rj, ncsr - first);
-            const gdouble* win =
-                (which == 0 ? wake_g + g0 + first
-                            : (which == 1 ? csr_h + (uint32_t)x0 + first : wake_g)) +
-                (n - 1);
-            double acc[STEP_DOT_ROWS];
-            uint32_t at[STEP_DOT_ROWS];
-#pragma unroll
-            for (int i = 0; i < STEP_DOT_ROWS; i++) {
-                acc[i] = 0.0;
-                at[i] = (uint32_t)min(i, rows - 1);  // (slots past the last
-                                                     // row repeat it, unused)
-            }
-#pragma unroll 2
-            for (uint32_t x = lane; x < n; x += 64) {
-                const double p = (double)pprev[x];
-                double w[STEP_DOT_ROWS];
-#pragma unroll
-                for (int i = 0; i < STEP_DOT_ROWS; i++) {
-                    w[i] = (win - x)[at[i]];
-                }
-#pragma unroll
-                for (int i = 0; i < STEP_DOT_ROWS; i++) {
-                    acc[i] += w[i] * p;
-                }
-            }
-            // every lane receives the sums; lane i finishes row i
-            double mine = 0.0;
-#pragma unroll
-            for (int i = 0; i < STEP_DOT_ROWS; i++) {
-                if (i < rows) {
-                    const double v = wave_sum_dpp(acc[i]);
-                    mine = lane == (uint32_t)i ? v : mine;
-                }
-            }
-            if (lane >= (uint32_t)rows) {
-                continue;
-            }
-            if (which == 0) {
-                const int row = lr0 + first + (int)lane;
-                const float off = d.wake_scale * (float)mine;
-                offw[row] = off;
-                store_row_taps<IT>(off, n, tapw + row * STEP_TAP_WORDS);
-            } else if (which == 1) {
-                const int o = first + (int)lane;
-                csr_rows[o] = (double)pprev[x0 + o] * mine;
-            } else {
-                s00_sh = row0_sample(mine);
-            }
-        }
-    }
-    if (ONE_MESH && DIRECT && (wake || csr)) {
+    if (DIRECT && (wake || csr)) {
         const int nwk = wake ? lr1 - lr0 : 0;
         const int ncsr = csr ? rows_out : 0;
         const int J = nwk + ncsr + ((need_s00 && wake) ? 1 : 0);
@@ -860,14 +789,30 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                 which = 2;
             }
             double acc = 0.0;
-            const double* win =
-                which == 0 ? gwin
-                           : (which == 1 ? hwin
-                                         : reinterpret_cast<const double*>(
-                                               lds + L.g0win));
+            if constexpr (ONE_MESH) {
+                const double* win =
+                    which == 0 ? gwin
+                               : (which == 1 ? hwin
+                                             : reinterpret_cast<const double*>(
+                                                   lds + L.g0win));
 #pragma unroll 4
-            for (uint32_t x = lane; x < n; x += 64) {
-                acc += win[base + n - 1 - x] * (double)pprev[x];
+                for (uint32_t x = lane; x < n; x += 64) {
+                    acc += win[base + n - 1 - x] * (double)pprev[x];
+                }
+            } else {
+                // the same windows, read from the tables in global memory.
+                // (Up to four rows a wavefront at once save trips to L2 where
+                // rows are many and short, 64 meshes of 128^2 with T = 8: 13.0
+                // -> 12.2 us a step; but their registers and loads cost every
+                // other tiling: 4 of 512^2 with T = 2 17.8 -> 22.8, 4 of
+                // 1024^2 with T = 4 36.3 -> 49.9.)
+                const gdouble* win =
+                    which == 0 ? wake_g + g0
+                               : (which == 1 ? csr_h + (uint32_t)x0 : wake_g);
+#pragma unroll 4
+                for (uint32_t x = lane; x < n; x += 64) {
+                    acc += win[base + n - 1 - x] * (double)pprev[x];
+                }
             }
             acc = wave_sum_dpp(acc);
             if (lane != 0) {
@@ -1171,7 +1116,7 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                         acc = acc + qb[k].w;
                     }
                 }
-            } else if (vec_rows) {
+            } else if (vec_rows && AHEAD32 && n >= 64u) {
                 // other lengths: the same with the loads held inside the row,
                 // and the last n % 64 values' loads together (one word at a
                 // time the last n % 16 took 30 cycles each: the projection of
@@ -1227,6 +1172,67 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                     }
                 }
                 y = n;
+            } else if (vec_rows) {
+                // a batch of direct-wake meshes, where registers are
+                // occupancy, and short rows: the next 16 values load while the
+                // current 16 are added, the last n % 16 together.  (With 32
+                // ahead the resident-grid form kept 133 registers and 3
+                // wavefronts a SIMD, two-column tiles 105 and 4 in place of 88
+                // and 5: 64 meshes of 256^2, T = 2 with 128 threads, 44.3 ->
+                // 49.2 us.  The FFT form has them to spare, but for two columns
+                // a thread, 100 and 4 in place of 88 and 5: 2 meshes of 1000^2,
+                // T = 2 with 256 threads, 48.1 us with 32 ahead, 53.4 with 16;
+                // 4 of 1024^2, T = 2 with 512, 64.2 and 59.6.)
+                const vec4f* r4 = reinterpret_cast<const vec4f*>(r);
+                const uint32_t n4 = n >> 2;
+                vec4f q[4], nq[4];
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) {
+                    q[k] = r4[min(k, n4 - 1u)];
+                }
+                for (; y + 16 <= n; y += 16) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; k++) {
+                        nq[k] = r4[min(((y + 16) >> 2) + k, n4 - 1u)];
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        acc = acc + q[k].x;
+                        acc = acc + q[k].y;
+                        acc = acc + q[k].z;
+                        acc = acc + q[k].w;
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        q[k] = nq[k];
+                    }
+                }
+                const uint32_t left4 = (n - y) >> 2;
+#pragma unroll
+                for (uint32_t k = 0; k < 3; k++) {
+                    if (k < left4) {
+                        acc = acc + q[k].x;
+                        acc = acc + q[k].y;
+                        acc = acc + q[k].z;
+                        acc = acc + q[k].w;
+                    }
+                }
+                y = n;
+            }
+            // n % 4 != 0: words, eight loads at a time (left to the compiler
+            // this loop came out differently wherever the code around it
+            // changed: 8 meshes of 130^2, T = 2 with 128 threads, 14.3 us a
+            // step, 15.4 beside the branches above, 11.2 like this)
+            for (; y + 8 <= n; y += 8) {
+                float q[8];
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    q[k] = r[y + (uint32_t)k];
+                }
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    acc = acc + q[k];
+                }
             }
             for (; y < n; y++) {
                 acc = acc + r[y];

@@ -62,3 +62,30 @@ def test_timing_is_the_time_of_a_run():
         timing.append(b.timing(steps) * 1e3)
     print(f"{groups} groups: run {min(run):.1f}, timing {min(timing):.1f} us")
     assert min(timing) <= 1.5 * min(run)
+
+
+@pytest.mark.parametrize("count,n,T", [(1, 32, 1), (1, 40, 8), (3, 24, 2),
+                                       (7, 17, 4), (8, 8, 8), (9, 20, 16),
+                                       (13, 36, 5)])
+@pytest.mark.parametrize("persistent", [False, True])
+def test_shares_of_the_block_map(count, n, T, persistent):
+    """Tiles and closing workgroups dealt out over eight shares: fewer tiles
+    than shares, equal and uneven shares, more closing workgroups than
+    shares, padding; every instance as on its own."""
+    import inovesa_amd as V
+    from inovesa_amd.workloads import (impedances, initial_mesh,
+                                       kick_drift_config)
+    desc, d = kick_drift_config(n=n, steps_per_ts=4000)
+    zw, zc = impedances(d)
+    inits = [initial_mesh(n, seed=k) for k in range(count)]
+    b = V.Batch([desc] * count, inits, [zw] * count, [zc] * count)
+    b.retile_size(n, T, 128, persistent=persistent)
+    b.record(5)
+    b.run(5)
+    for k in range(count):
+        s = V.Step(desc, inits[k], zw, zc)
+        s.record(5)
+        s.run(5)
+        for x, y in zip(b.mesh(k), s.mesh()):
+            np.testing.assert_array_equal(x, y)
+        np.testing.assert_array_equal(b.history(k)[0], s.history()[0])

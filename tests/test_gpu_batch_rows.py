@@ -1,7 +1,7 @@
-"""The wake and CSR dot products of a batch's tiles: up to four consecutive
-rows of a table share a wavefront.  Pinned by the single-mesh step, which sums
-one row per wavefront: a row's own sum keeps its order, so the meshes and the
-CSR powers are equal bit for bit, wherever the rows of a tile end."""
+"""The wake and CSR dot products of a batch's tiles, whose rows are dealt out
+over the wavefronts.  Pinned by the single-mesh step: a row's sum has the same
+order there, so the meshes and the CSR powers are equal bit for bit, wherever
+the rows of a tile end and however many wavefronts share them."""
 import numpy as np
 import pytest
 

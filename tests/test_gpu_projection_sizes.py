@@ -68,3 +68,31 @@ def test_a_row_beyond_the_lds_is_refused():
     import inovesa_amd as V
     with pytest.raises(V.VfpsInvalid):
         V.PhaseSpace(40961, -6.0, 6.0, 1e-3, -6.0, 6.0, 1e6)
+
+
+@pytest.mark.parametrize("n", [5, 7, 8, 9, 15, 17, 23, 24, 66, 129, 250, 268])
+@pytest.mark.parametrize("wake", [1, 2])
+def test_step_and_batch_projection_in_words(n, wake):
+    """Lengths with every remainder of the eight words a turn, and of the 16
+    and 64 values a turn, in each wake form and with one, two and four columns
+    a thread."""
+    import inovesa_amd as V
+    from inovesa_amd.workloads import (impedances, initial_mesh,
+                                       kick_drift_config, simpson_weights)
+    desc, d = kick_drift_config(n=n, steps_per_ts=2000)
+    desc = dict(desc, wake_method=wake)
+    zw, zc = impedances(d)
+    init = initial_mesh(n, seed=n)
+    ws = simpson_weights(n, np.float32(12.0) / np.float32(n - 1))
+    st = V.Step(desc, init, zw, zc)
+    st.run(2)
+    mesh, proj, _ = st.mesh()
+    np.testing.assert_array_equal(proj, _sequential(mesh, ws))
+    for threads in (64, 128, 512):
+        if threads * 4 < n:
+            continue
+        b = V.Batch([dict(desc, tile_rows=2, threads=threads)], [init], [zw], [zc])
+        b.run(2)
+        bm, bp, _ = b.mesh(0)
+        np.testing.assert_array_equal(bm, mesh)
+        np.testing.assert_array_equal(bp, proj)
