@@ -6,7 +6,7 @@
 // passes (and one radix-4 or radix-2 pass), in place in one LDS buffer
 // with a spare slot after every 8 elements, with no bit reversal.  A length
 // M that is no power of two goes through two transforms of a power-of-two
-// length (Bluestein's chirp algorithm).
+// length (Bluestein's chirp algorithm), a short one through the direct sums.
 //
 // The butterflies run in FP64.  Inputs and outputs stay FP32 exactly where
 // the reference's arrays are float (profile, spectrum F, W = Z F, wake
@@ -233,15 +233,70 @@ __host__ __device__ __forceinline__ uint32_t chirp_table(uint32_t M)
     return M + P + chirp_tw(P);
 }
 
-// Complex DFT of length M (no power of two; M <= FFT_MAX_M) in place in the
+__host__ __device__ __forceinline__ bool fft_pow2(uint32_t M)
+{
+    return M >= 1u && (M & (M - 1u)) == 0u;
+}
+
+// Longest transform made by the direct sums (dft_direct).  Their time grows
+// with M, the chirp's is that of its barriers: FFT-wake steps of M = 50, 127,
+// 170, 190 took 12.5, 19.0, 22.7, 25.5 us with the sums and 22.1, 23.0, 23.9,
+// 23.8 with the chirp.
+constexpr uint32_t DFT_MAX_DIRECT = 176;
+
+// whether the transform of M elements is a chirp DFT
+__host__ __device__ __forceinline__ bool fft_chirp(uint32_t M)
+{
+    return !fft_pow2(M) && M > DFT_MAX_DIRECT;
+}
+
+// entries of the transform's table (tw_m): exp(-2 pi i t / M), t < M, or the
+// chirp table
+__host__ __device__ __forceinline__ uint32_t fft_table(uint32_t M)
+{
+    return fft_chirp(M) ? chirp_table(M) : M;
+}
+
+// Complex DFT of length M (any M) in place in the slots of the LDS buffer
+// `a`, by the sums out[k] = sum_j a[j] w^(j k) in FP64.  tmp: LDS scratch of
+// M entries; tw: the table exp(-2 pi i t / M), t < M (global memory: the
+// powers of w are picked by index, (j k) mod M, so no rounding accumulates
+// across the sum).  Forward uses exp(-i..), INV exp(+i..); unnormalised.
+// Must be called by the whole workgroup.
+template <bool INV>
+__device__ void dft_direct(double2* a, double2* tmp, uint32_t M,
+                           const double2* __restrict__ tw)
+{
+    for (uint32_t i = threadIdx.x; i < M; i += FFT_THREADS) {
+        tmp[i] = a[fft_slot(i)];
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < M; k += FFT_THREADS) {
+        double re = 0.0, im = 0.0;
+        uint32_t t = 0;
+        for (uint32_t j = 0; j < M; j++) {
+            const double2 x = tmp[j];
+            const double2 w = tw[t];
+            const double wy = INV ? -w.y : w.y;
+            re += x.x * w.x - x.y * wy;
+            im += x.x * wy + x.y * w.x;
+            t += k;
+            if (t >= M) t -= M;
+        }
+        a[fft_slot(k)] = make_double2(re, im);
+    }
+    __syncthreads();
+}
+
+// Complex DFT of length M (fft_chirp(M); M <= FFT_MAX_M) in place in the
 // slots of the LDS buffer `a` (chirp_len(M) elements), for the lengths the
 // FFT does not take (the reference's FFTW plans any length, e.g. nmax = 768 =
 // 3 * 256 when RoundPadding is off).  With j k = (j^2 + k^2 - (k - j)^2) / 2,
 //   X_k = c_k sum_j (x_j c_j) conj(c_{k-j}):
 // a convolution, made by an FFT of P >= 2 M - 1 elements, the product with
 // the filter's transform and the inverse FFT, all FP64.  Wake potential and
-// CSR spectra of two bunches with M = 1500: 119 us a call, with the direct
-// sums of M^2 terms it was 1884.
+// CSR spectra of two bunches with M = 1500: 82 us a call; the direct sums of
+// M^2 terms take 1850 us more.
 // The inverse DFT is the conjugate of the DFT of the conjugate.  tw: LDS
 // copy of the table's twiddle factors; tab: the table in global memory (it
 // stays in L2).  Forward uses exp(-i..), INV exp(+i..); unnormalised.
@@ -274,11 +329,6 @@ __device__ void dft_lds(double2* a, uint32_t M, const double2* tw,
         a[fft_slot(j)] = v;
     }
     __syncthreads();
-}
-
-__host__ __device__ __forceinline__ bool fft_pow2(uint32_t M)
-{
-    return M >= 1u && (M & (M - 1u)) == 0u;
 }
 
 // Spectrum F_k (k = 0..M) of the real input from Z = FFT_M(z):

@@ -29,6 +29,9 @@ size_t field_lds_bytes(uint32_t M)
     if (fft_pow2(M)) {
         return sizeof(double2) * (fft_slots(M) + M / 2);
     }
+    if (!fft_chirp(M)) {
+        return sizeof(double2) * (fft_slots(M) + M);
+    }
     const uint32_t P = chirp_len(M);
     return sizeof(double2) * (fft_slots(P) + chirp_tw(P));
 }
@@ -124,7 +127,7 @@ void make_twiddles(uint32_t M, std::vector<double2>& tw_m,
                    std::vector<double2>& tw_n)
 {
     const double pi = 3.141592653589793238462643383279502884;
-    if (fft_pow2(M)) {
+    if (!fft_chirp(M)) {
         tw_m.resize(M);
         for (uint32_t t = 0; t < M; t++) {
             sincos(-2.0 * pi * (double)t / (double)M, &tw_m[t].y, &tw_m[t].x);

@@ -41,8 +41,7 @@ size_t field_lds_bytes(uint32_t M);
 int field_set_lds_limit(size_t bytes);
 int launch_field(const FieldParams& p, bool wake, bool csr, uint32_t blocks,
                  hipStream_t st);
-// the transform's table (e^{-2 pi i t/M}, t < M, or the chirp table where M
-// is no power of two) and e^{-2 pi i k/2M}, k < M
+// the transform's table (fft_table(M) entries) and e^{-2 pi i k/2M}, k < M
 void make_twiddles(uint32_t M, std::vector<double2>& tw_m,
                    std::vector<double2>& tw_n);
 std::vector<float> csr_renorm(uint32_t nmax, float delta0, double qscale,

@@ -18,8 +18,9 @@ namespace vfps_impl {
 // holds them as float, and the float arithmetic on them follows the
 // reference.  lds: field_lds_bytes(M): fft_slots(M) + M/2 double2 (data
 // with a spare slot after every 8 elements, twiddle half table) for a
-// power-of-two M, else those of the chirp transform's length and its twiddle
-// factors.  Runs with FFT_THREADS
+// power-of-two M, those of the chirp transform's length and its twiddle
+// factors, or those of M and M double2 of scratch (direct sums).  Runs with
+// FFT_THREADS
 // threads (the loops step by that constant: blockDim would be a load from
 // the dispatch packet, waited for after every barrier).
 constexpr int FIELD_PAIRS = 3;  // (k, M-k) pairs per thread: M <= 4096
@@ -50,9 +51,9 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     VFPS_FSTAMP(0);
     const uint32_t M = p.M;
     // power-of-two M: radix-8 FFT with the half twiddle table in LDS;
-    // other M: chirp DFT
-    const bool pow2 = fft_pow2(M);
-    const uint32_t P = pow2 ? M : chirp_len(M);
+    // other M: chirp DFT, or direct sums where M is short
+    const bool pow2 = fft_pow2(M), chirp = fft_chirp(M);
+    const uint32_t P = chirp ? chirp_len(M) : M;
     auto slot = [](uint32_t i) { return fft_slot(i); };
     // real sample i of the padded array: element i/2, real part for even i
     auto rslot = [&](uint32_t i) { return 2u * slot(i >> 1) + (i & 1u); };
@@ -89,7 +90,7 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
         A[slot(i)] = make_double2(0.0, 0.0);
     }
     if (WAKE || CSR) {
-        const uint32_t ntw = pow2 ? M / 2 : chirp_tw(P);
+        const uint32_t ntw = pow2 ? M / 2 : (chirp ? chirp_tw(P) : 0u);
         const double2* src = pow2 ? p.tw_m : p.tw_m + M + P;
         for (uint32_t i = threadIdx.x; i < ntw; i += FFT_THREADS) {
             twl[i] = src[i];
@@ -198,8 +199,10 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     VFPS_FSTAMP(1);
     if (pow2) {
         fft_lds<false>(A, M, TwTable{twl});
-    } else {
+    } else if (chirp) {
         dft_lds<false>(A, M, twl, p.tw_m);
+    } else {
+        dft_direct<false>(A, twl, M, p.tw_m);
     }
     VFPS_FSTAMP(2);
     double2* Zf = A;
@@ -290,8 +293,10 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     VFPS_FSTAMP(3);
     if (pow2) {
         fft_lds<true>(A, M, TwTable{twl});
-    } else {
+    } else if (chirp) {
         dft_lds<true>(A, M, twl, p.tw_m);
+    } else {
+        dft_direct<true>(A, twl, M, p.tw_m);
     }
     VFPS_FSTAMP(4);
     const double* yd = reinterpret_cast<const double*>(A);

@@ -740,7 +740,7 @@ static int step_setup_direct(vfps_step* s)
 static size_t step_block_bytes(size_t n, size_t nmax)
 {
     const size_t M = nmax / 2;
-    const size_t tw = fft_pow2((uint32_t)M) ? M : chirp_table((uint32_t)M);
+    const size_t tw = fft_table((uint32_t)M);
     const size_t mesh = sizeof(float) * (3 * n + 1) + 2 * sizeof(double);
     const size_t field = sizeof(float) * (n + 3 * nmax + 2) +
                          sizeof(double2) * (tw + M);

@@ -1,7 +1,7 @@
-"""The field's transforms whose length is no power of two (chirp DFT):
-primes, the smallest and largest lengths, either side of a doubling of the
-inner transform, several bunches, and mixed with power-of-two lengths in one
-batch."""
+"""The field's transforms whose length is no power of two (direct sums, from
+178 on a chirp DFT): primes, the smallest and largest lengths, either side of
+a doubling of the inner transform and of the direct sums' longest, several
+bunches, and mixed with power-of-two lengths in one batch."""
 import numpy as np
 import pytest
 
@@ -76,3 +76,31 @@ def test_batch_of_mixed_lengths(V):
         st.run(9)
         for x, y in zip(b.mesh(i), st.mesh()):
             np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("nmax,n,nb", [(202, 90, 2), (346, 100, 3),
+                                       (352, 176, 2), (354, 120, 2),
+                                       (356, 100, 3), (358, 333, 1)])
+def test_either_side_of_the_direct_sums(V, nmax, n, nb):
+    test_chirp_lengths_match_numpy(V, nmax, n, nb)
+
+
+@pytest.mark.parametrize("nmax", [250, 352, 354, 1000])
+def test_fft_step_beside_a_batch(V, nmax):
+    """A step with its own transform kernel and the batch's shared one."""
+    from inovesa_amd.workloads import initial_mesh, kick_drift_config
+    rng = np.random.default_rng(nmax)
+    z = V.Impedance(nmax, 1e12, table=(1e-3 * rng.random(nmax)).astype(
+        np.complex64))
+    desc, _ = kick_drift_config(n=64, steps_per_ts=4000)
+    desc = dict(desc, wake_method=1)
+    init = initial_mesh(64, seed=1)
+    st = V.Step(desc, init, z, z)
+    st.record(3)
+    st.run(3)
+    b = V.Batch([desc] * 2, [init] * 2, [z] * 2, [z] * 2)
+    b.record(3)
+    b.run(3)
+    for x, y in zip(b.mesh(1), st.mesh()):
+        np.testing.assert_array_equal(x, y)
+    np.testing.assert_array_equal(b.history(1)[0], st.history()[0])
