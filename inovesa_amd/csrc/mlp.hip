@@ -191,8 +191,7 @@ __global__ void adam_kernel(float* __restrict__ p, uint16_t* __restrict__ pb,
 {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x) {
-        const float pi = adam_update(a, g[i], p + i, m + i, v + i);
-        if (pb) pb[i] = f2bf(pi);
+        pb[i] = f2bf(adam_update(a, g[i], p + i, m + i, v + i));
     }
 }
 
@@ -490,11 +489,17 @@ AdamArgs next_adam(vfps_mlp* m, float lr, float b1, float b2, float eps)
 int adam(vfps_mlp* m, float lr, float b1, float b2, float eps)
 {
     const AdamArgs a = next_adam(m, lr, b1, b2, eps);
-    hipLaunchKernelGGL(adam_kernel, dim3(std::min<size_t>((m->nparams + 255) / 256, 1024)),
-                       dim3(256), 0, m->dev->stream, m->p, m->pb, m->g, m->m,
-                       m->v, m->nparams, a);
+    const dim3 blocks(std::min<size_t>((m->nparams + 255) / 256, 1024));
+    if (m->fused()) {
+        hipLaunchKernelGGL(mlp_adam_kernel, blocks, dim3(256), 0, m->dev->stream,
+                           m->net, a, (uint32_t)m->nparams, m->p, m->g, m->m,
+                           m->v, m->W, m->WT);
+    } else {
+        hipLaunchKernelGGL(adam_kernel, blocks, dim3(256), 0, m->dev->stream,
+                           m->p, m->pb, m->g, m->m, m->v, m->nparams, a);
+    }
     VFPS_HIP(hipGetLastError());
-    return m->fused() ? fused_pack(m) : VFPS_OK;
+    return VFPS_OK;
 }
 
 uint64_t splitmix(uint64_t& s)

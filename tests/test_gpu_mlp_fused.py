@@ -153,3 +153,30 @@ def test_overflow_stays_infinite(V, dims):
         # (not the row of the label, whose gradient is finite)
         out = slice(None, -1 if l + 2 == len(dims) else None)
         assert np.all(np.isposinf(dW[out])) and np.all(np.isposinf(db[out]))
+
+
+@pytest.mark.parametrize("dims", [(3, 2), (1, 5, 2), (3, 48, 33, 9),
+                                  (33, 100, 17), (3, 256, 256, 65),
+                                  (3, 1200, 1100, 9)])
+def test_adam_step_updates_the_operands(V, dims):
+    """adam_step alone: the parameters by Adam's formula (two steps, FP32), and
+    the BF16 copies that the products read follow them."""
+    x, t, lab = _data(20, dims, seed=3)
+    net = V.MLP(dims, max_batch=32, seed=2)
+    m = v = np.zeros(net.params().size)
+    for step in (1, 2):
+        net.loss_grad(x, t, lab)
+        p, g = net.params().astype(np.float64), net.grads().astype(np.float64)
+        net.adam_step(lr=1e-2)
+        m, v = 0.9 * m + 0.1 * g, 0.999 * v + 0.001 * g * g
+        ref = p - 1e-2 * (m / (1 - 0.9 ** step)) / (
+            np.sqrt(v / (1 - 0.999 ** step)) + 1e-8)
+        # an update is at most lr here and is made of a dozen FP32 operations
+        # (1 - 0.999^t, a difference of near equals, carries the most: 6e-5)
+        assert np.abs(net.params() - ref).max() <= 1e-2 * 1e-4 + 2.0**-23 * 4
+    other = V.MLP(dims, max_batch=32, seed=5)
+    other.set_params(net.params())
+    np.testing.assert_array_equal(net.forward(x), other.forward(x))
+    net.loss_grad(x, t, lab)
+    other.loss_grad(x, t, lab)
+    np.testing.assert_array_equal(net.grads(), other.grads())
