@@ -71,69 +71,67 @@ int field_set_lds_limit(size_t bytes)
     return VFPS_OK;
 }
 
-// in-place radix-2 FFT (host, exp(-i..)) of a power-of-two length
-static void fft_host(std::vector<double2>& a)
+// The chirp table of dft_lds (fft.hpp), one workgroup.  (Made on the host its
+// sines and its FFT of up to 8192 elements were two fifths of a field's
+// construction: 248 us with nmax = 6000, 114 now.)
+__global__ void __launch_bounds__(FFT_THREADS)
+chirp_table_kernel(uint32_t M, double2* __restrict__ tab)
 {
-    const size_t n = a.size();
-    for (size_t i = 1, j = 0; i < n; i++) {
-        size_t bit = n >> 1;
-        for (; j & bit; bit >>= 1) j ^= bit;
-        j ^= bit;
-        if (i < j) std::swap(a[i], a[j]);
+    extern __shared__ double2 lds[];
+    const uint32_t P = chirp_len(M);
+    double2* a = lds;
+    double2* tw = lds + fft_slots(P);
+    auto turn = [](double half_turns) {  // exp(-i pi half_turns)
+        double2 v;
+        sincospi(-half_turns, &v.y, &v.x);
+        return v;
+    };
+    for (uint32_t k = threadIdx.x; k < chirp_tw(P); k += FFT_THREADS) {
+        const uint32_t e = k < 64u ? k : 64u * (k - 64u);
+        tw[k] = turn(2.0 * (double)e / (double)P);
+        tab[M + P + k] = tw[k];
     }
-    std::vector<double2> w(n / 2);
-    for (size_t t = 0; t < n / 2; t++) {
-        sincos(-2.0 * M_PI * (double)t / (double)n, &w[t].y, &w[t].x);
+    for (uint32_t j = threadIdx.x; j < P; j += FFT_THREADS) {
+        a[fft_slot(j)] = make_double2(0.0, 0.0);
     }
-    for (size_t h = 1; h < n; h <<= 1) {
-        for (size_t i = 0; i < n; i += 2 * h) {
-            for (size_t k = 0; k < h; k++) {
-                const double2 c = w[k * (n / (2 * h))], u = a[i + k],
-                              v = a[i + k + h];
-                const double2 x = make_double2(v.x * c.x - v.y * c.y,
-                                               v.x * c.y + v.y * c.x);
-                a[i + k] = make_double2(u.x + x.x, u.y + x.y);
-                a[i + k + h] = make_double2(u.x - x.x, u.y - x.y);
-            }
-        }
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < M; j += FFT_THREADS) {
+        // j^2 modulo 2 M: the angle stays small and exact
+        const double2 c = turn((double)(j * j % (2u * M)) / (double)M);
+        tab[j] = c;
+        a[fft_slot(j)] = cconj(c);
+        if (j) a[fft_slot(P - j)] = cconj(c);
+    }
+    __syncthreads();
+    fft_lds<false, CHIRP_MAX_P>(a, P, TwFactors{tw});
+    for (uint32_t k = threadIdx.x; k < P; k += FFT_THREADS) {
+        const double2 v = a[fft_slot(k)];
+        tab[M + k] = make_double2(v.x / P, v.y / P);
     }
 }
 
-// the chirp table of dft_lds (fft.hpp)
-static std::vector<double2> chirp_tables(uint32_t M)
+int launch_fft_table(vfps_dev* dev, uint32_t M, double2* tab)
 {
-    const uint32_t P = chirp_len(M);
-    std::vector<double2> t(chirp_table(M)), b(P, make_double2(0.0, 0.0));
-    for (uint32_t j = 0; j < M; j++) {
-        // j^2 modulo 2 M: the angle stays small and exact
-        const uint64_t q = (uint64_t)j * j % (2ull * M);
-        sincos(-M_PI * (double)q / (double)M, &t[j].y, &t[j].x);
-        b[j] = make_double2(t[j].x, -t[j].y);
-        if (j) b[P - j] = b[j];
+    if (!fft_chirp(M)) return VFPS_OK;
+    const size_t lds = field_lds_bytes(M);
+    if (lds > 65536) {
+        VFPS_HIP(hipFuncSetAttribute(
+            reinterpret_cast<const void*>(&chirp_table_kernel),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     }
-    fft_host(b);
-    for (uint32_t k = 0; k < P; k++) {
-        t[M + k] = make_double2(b[k].x / P, b[k].y / P);
-    }
-    double2* f = t.data() + M + P;
-    for (uint32_t k = 0; k < chirp_tw(P); k++) {
-        const uint64_t e = k < 64u ? k : 64ull * (k - 64u);
-        sincos(-2.0 * M_PI * (double)e / (double)P, &f[k].y, &f[k].x);
-    }
-    return t;
+    hipLaunchKernelGGL(chirp_table_kernel, dim3(1), dim3(FFT_THREADS), lds,
+                       dev->stream, M, tab);
+    VFPS_HIP(hipGetLastError());
+    return VFPS_OK;
 }
 
 void make_twiddles(uint32_t M, std::vector<double2>& tw_m,
                    std::vector<double2>& tw_n)
 {
     const double pi = 3.141592653589793238462643383279502884;
-    if (!fft_chirp(M)) {
-        tw_m.resize(M);
-        for (uint32_t t = 0; t < M; t++) {
-            sincos(-2.0 * pi * (double)t / (double)M, &tw_m[t].y, &tw_m[t].x);
-        }
-    } else {
-        tw_m = chirp_tables(M);
+    tw_m.resize(fft_chirp(M) ? 0 : M);
+    for (uint32_t t = 0; t < tw_m.size(); t++) {
+        sincos(-2.0 * pi * (double)t / (double)M, &tw_m[t].y, &tw_m[t].x);
     }
     tw_n.resize(M);
     for (uint32_t t = 0; t < M; t++) {
@@ -375,7 +373,7 @@ int vfps_field_create(vfps_mesh* ps, vfps_impedance* z,
     e = e ? e : setup_alloc(&f->wake, (size_t)nb * n);
     e = e ? e : setup_alloc(&f->padded, nmax);
     e = e ? e : setup_alloc(&f->wake_padded, nmax);
-    e = e ? e : setup_alloc(&f->tw_m, twm.size());
+    e = e ? e : setup_alloc(&f->tw_m, fft_table(M));
     e = e ? e : setup_alloc(&f->tw_n, M);
     e = e ? e : setup_alloc(&f->csr_renorm, nmax);
     e = e ? e : setup_alloc(&f->power, nb);
@@ -388,7 +386,12 @@ int vfps_field_create(vfps_mesh* ps, vfps_impedance* z,
     setup_zero(f->wake, sizeof(float) * nb * n, st);
     setup_zero(f->padded, sizeof(float) * nmax, st);
     setup_zero(f->wake_padded, sizeof(float) * nmax, st);
-    setup_put(f->tw_m, twm.data(), sizeof(double2) * twm.size(), st);
+    if (!twm.empty()) {
+        setup_put(f->tw_m, twm.data(), sizeof(double2) * twm.size(), st);
+    } else if (!f->in_block && (rc = launch_fft_table(f->dev, M, f->tw_m)) != VFPS_OK) {
+        vfps_field_destroy(f);
+        return rc;
+    }
     setup_put(f->tw_n, twn.data(), sizeof(double2) * M, st);
     setup_put(f->csr_renorm, renorm.data(), sizeof(float) * nmax, st);
     setup_zero(f->power, sizeof(float) * nb, st);

@@ -41,9 +41,13 @@ size_t field_lds_bytes(uint32_t M);
 int field_set_lds_limit(size_t bytes);
 int launch_field(const FieldParams& p, bool wake, bool csr, uint32_t blocks,
                  hipStream_t st);
-// the transform's table (fft_table(M) entries) and e^{-2 pi i k/2M}, k < M
+// the transform's table (fft_table(M) entries; none where the device makes
+// it) and e^{-2 pi i k/2M}, k < M
 void make_twiddles(uint32_t M, std::vector<double2>& tw_m,
                    std::vector<double2>& tw_n);
+// the transform's table where the device makes it (chirp lengths), in stream
+// order
+int launch_fft_table(vfps_dev* dev, uint32_t M, double2* tab);
 std::vector<float> csr_renorm(uint32_t nmax, float delta0, double qscale,
                               float fc, float* fdelta);
 

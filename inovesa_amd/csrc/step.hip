@@ -998,10 +998,15 @@ int vfps_step_create(vfps_dev* dev, const vfps_step_desc* desc,
         if (!s->wfield) {
             // twiddles of their own
             make_twiddles(s->M, twm, twn);
-            s->csr_tw_m = twm.size();
-            VFPS_HIP(setup_alloc(&s->csr_tw, twm.size() + s->M));
-            VFPS_HIP(setup_put(s->csr_tw, twm.data(),
-                               sizeof(double2) * twm.size(), st));
+            s->csr_tw_m = fft_table(s->M);
+            VFPS_HIP(setup_alloc(&s->csr_tw, s->csr_tw_m + s->M));
+            if (!twm.empty()) {
+                VFPS_HIP(setup_put(s->csr_tw, twm.data(),
+                                   sizeof(double2) * twm.size(), st));
+            } else if (!step_block &&
+                       (rc = launch_fft_table(dev, s->M, s->csr_tw)) != VFPS_OK) {
+                return rc;
+            }
             VFPS_HIP(setup_put(s->csr_tw + s->csr_tw_m, twn.data(),
                                sizeof(double2) * s->M, st));
         }
@@ -1027,6 +1032,11 @@ int vfps_step_create(vfps_dev* dev, const vfps_step_desc* desc,
                                 hipMemcpyHostToDevice, st));
         VFPS_HIP(hipMemcpyAsync(s->t1->data, init, sizeof(float) * cells,
                                 hipMemcpyHostToDevice, st));
+        // (tables the device makes, after the block's zeros)
+        double2* tab = s->wfield ? s->wfield->tw_m : s->csr_tw;
+        if (tab && !s->direct && (rc = launch_fft_table(dev, s->M, tab)) != VFPS_OK) {
+            return rc;
+        }
         rc = launch_project_x(s->t1, s->t1->data, s->t1->proj);
         if (rc != VFPS_OK) return rc;
     }
