@@ -229,12 +229,13 @@ __device__ __forceinline__ void lds_window16(const float* s, int32_t lo,
 }
 
 // Four consecutive values of an LDS row of n from y on: one 16-byte store,
-// or, where rows are no whole groups (n % 4 != 0), those inside the row word
-// by word.
+// or, where rows are no whole groups (WHOLE: n % 4 == 0), those inside the row
+// word by word.
+template <bool WHOLE>
 __device__ __forceinline__ void store4(float* row, uint32_t n, uint32_t y,
                                        vec4f o)
 {
-    if ((n & 3u) == 0u) {
+    if constexpr (WHOLE) {
         *reinterpret_cast<vec4f*>(row + y) = o;
         return;
     }
@@ -248,7 +249,7 @@ __device__ __forceinline__ void store4(float* row, uint32_t n, uint32_t y,
 // [r0, r1) of a row buffer: each thread makes four consecutive outputs of
 // a row (the last group may end past it) from IT+3 consecutive inputs, taps
 // in order.
-template <int IT>
+template <int IT, bool WHOLE>
 __device__ __forceinline__ void kick_rows(const float* __restrict__ src,
                                           float* __restrict__ dst, uint32_t n,
                                           int r0, int r1,
@@ -258,7 +259,7 @@ __device__ __forceinline__ void kick_rows(const float* __restrict__ src,
         return;
     }
     const uint32_t bs = blockDim.x;
-    const uint32_t ng = (n + 3u) >> 2;
+    const uint32_t ng = (n + (WHOLE ? 0u : 3u)) >> 2;
     const uint32_t drow = bs / ng, dg = bs % ng;
     uint32_t row = (uint32_t)r0 + threadIdx.x / ng;
     uint32_t g = threadIdx.x % ng;
@@ -286,7 +287,7 @@ __device__ __forceinline__ void kick_rows(const float* __restrict__ src,
             }
             o[e] = acc;
         }
-        store4(dst + (size_t)row * n, n, 4 * g, o);
+        store4<WHOLE>(dst + (size_t)row * n, n, 4 * g, o);
         g += dg;
         row += drow;
         if (g >= ng) {
@@ -303,7 +304,7 @@ __device__ __forceinline__ void kick_rows(const float* __restrict__ src,
 // kick_rows makes it (a sample out of range reads as zero in both), so the
 // result equals the two kicks one after the other bit for bit, without the
 // intermediate rows in LDS or the barrier between the two.
-template <int IT>
+template <int IT, bool WHOLE>
 __device__ __forceinline__ void kick2_rows(const float* __restrict__ src,
                                            float* __restrict__ dst, uint32_t n,
                                            int r0, int r1,
@@ -314,7 +315,7 @@ __device__ __forceinline__ void kick2_rows(const float* __restrict__ src,
         return;
     }
     const uint32_t bs = blockDim.x;
-    const uint32_t ng = (n + 3u) >> 2;
+    const uint32_t ng = (n + (WHOLE ? 0u : 3u)) >> 2;
     const uint32_t drow = bs / ng, dg = bs % ng;
     uint32_t row = (uint32_t)r0 + threadIdx.x / ng;
     uint32_t g = threadIdx.x % ng;
@@ -354,7 +355,7 @@ __device__ __forceinline__ void kick2_rows(const float* __restrict__ src,
             }
             o[e] = acc;
         }
-        store4(dst + (size_t)row * n, n, 4 * g, o);
+        store4<WHOLE>(dst + (size_t)row * n, n, 4 * g, o);
         g += dg;
         row += drow;
         if (g >= ng) {
@@ -856,13 +857,21 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     // ---- C, D: wake kick and RF kick along y -------------------------------
     if (SCHEME == 0 && wake) {
         // both kicks in one pass (scheme 0)
-        kick2_rows<IT>(cur, oth, n, lr0, lr1, tapw, tapr);
+        if (vec_rows) {
+            kick2_rows<IT, true>(cur, oth, n, lr0, lr1, tapw, tapr);
+        } else {
+            kick2_rows<IT, false>(cur, oth, n, lr0, lr1, tapw, tapr);
+        }
         __syncthreads();
         float* t = cur;
         cur = oth;
         oth = t;
     } else if (wake) {
-        kick_rows<IT>(cur, oth, n, lr0, lr1, tapw);
+        if (vec_rows) {
+            kick_rows<IT, true>(cur, oth, n, lr0, lr1, tapw);
+        } else {
+            kick_rows<IT, false>(cur, oth, n, lr0, lr1, tapw);
+        }
         __syncthreads();
         float* t = cur;
         cur = oth;
@@ -872,7 +881,11 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
     if constexpr (SCHEME == 0) {
         if (!wake) {
             // ---- D: RF kick along y ----------------------------------------
-            kick_rows<IT>(cur, oth, n, lr0, lr1, tapr);
+            if (vec_rows) {
+                kick_rows<IT, true>(cur, oth, n, lr0, lr1, tapr);
+            } else {
+                kick_rows<IT, false>(cur, oth, n, lr0, lr1, tapr);
+            }
             __syncthreads();
             float* t = cur;
             cur = oth;
