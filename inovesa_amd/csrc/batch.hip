@@ -47,6 +47,7 @@ struct Group {
 // workgroup per member, ahead of the step kernels of the same step.
 struct FieldLaunch {
     bool wake = false, csr = false;
+    FieldKind kind = FIELD_PLAIN;
     uint32_t ninst = 0;
     size_t lds = 0;       // the most any member's transform needs
     FieldParams* params_d = nullptr;
@@ -113,11 +114,14 @@ int build_fields(vfps_batch* b)
         const bool wake = (pair & 1) != 0, csr = (pair & 2) != 0;
         std::vector<FieldParams> ps;
         size_t lds = 0;
+        FieldKind kind = FIELD_PLAIN;
         for (const vfps_step* s : b->members) {
             if (s->direct || (s->desc.use_wake != 0) != wake ||
                 (s->desc.use_csr != 0) != csr) {
                 continue;
             }
+            kind = ps.empty() || kind == field_kind(s->M) ? field_kind(s->M)
+                                                          : FIELD_ANY;
             ps.push_back(s->fparams_h);
             lds = std::max(lds, field_lds_bytes(s->M));
         }
@@ -127,6 +131,7 @@ int build_fields(vfps_batch* b)
         FieldLaunch f;
         f.wake = wake;
         f.csr = csr;
+        f.kind = kind;
         f.ninst = (uint32_t)ps.size();
         f.lds = lds;
         b->fields.push_back(f);
@@ -313,7 +318,7 @@ int launch_chains(vfps_batch* b, uint32_t parity, uint32_t steps)
 int launch_step(vfps_batch* b, uint32_t parity)
 {
     for (const auto& f : b->fields) {
-        int rc = launch_fields(f.wake, f.csr, f.params_d, f.ninst, f.lds,
+        int rc = launch_fields(f.wake, f.csr, f.kind, f.params_d, f.ninst, f.lds,
                                parity, b->dev->stream);
         if (rc != VFPS_OK) return rc;
     }

@@ -16,12 +16,25 @@
 
 namespace vfps_impl {
 
-template <bool WAKE, bool CSR>
+template <bool WAKE, bool CSR, FieldKind KIND>
 __global__ void __launch_bounds__(1024)
 field_kernel(FieldParams p)
 {
     extern __shared__ double2 lds[];
-    field_body<WAKE, CSR>(p, blockIdx.x, lds);
+    field_body<WAKE, CSR, KIND>(p, blockIdx.x, lds);
+}
+
+FieldKind field_kind(uint32_t M)
+{
+    return fft_chirp(M) ? FIELD_CHIRP : FIELD_PLAIN;
+}
+
+template <FieldKind KIND>
+static const void* field_fn(bool wake, bool csr)
+{
+    return wake && csr ? reinterpret_cast<const void*>(&field_kernel<true, true, KIND>)
+           : wake ? reinterpret_cast<const void*>(&field_kernel<true, false, KIND>)
+                  : reinterpret_cast<const void*>(&field_kernel<false, true, KIND>);
 }
 
 size_t field_lds_bytes(uint32_t M)
@@ -39,18 +52,13 @@ size_t field_lds_bytes(uint32_t M)
 int launch_field(const FieldParams& p, bool wake, bool csr, uint32_t blocks,
                  hipStream_t st)
 {
-    const size_t lds = field_lds_bytes(p.M);
-    if (wake && csr) {
-        hipLaunchKernelGGL((field_kernel<true, true>), dim3(1), dim3(FFT_THREADS), lds,
-                           st, p);
-    } else if (wake) {
-        hipLaunchKernelGGL((field_kernel<true, false>), dim3(1), dim3(FFT_THREADS),
-                           lds, st, p);
-    } else {
-        hipLaunchKernelGGL((field_kernel<false, true>), dim3(blocks),
-                           dim3(FFT_THREADS), lds, st, p);
-    }
-    VFPS_HIP(hipGetLastError());
+    const void* fn = field_kind(p.M) == FIELD_CHIRP
+                         ? field_fn<FIELD_CHIRP>(wake, csr)
+                         : field_fn<FIELD_PLAIN>(wake, csr);
+    FieldParams q = p;
+    void* args[] = {(void*)&q};
+    VFPS_HIP(hipLaunchKernel(fn, dim3(wake ? 1u : blocks), dim3(FFT_THREADS), args,
+                             field_lds_bytes(p.M), st));
     return VFPS_OK;
 }
 
@@ -59,15 +67,13 @@ int field_set_lds_limit(size_t bytes)
     if (bytes <= 65536) {
         return VFPS_OK;
     }
-    VFPS_HIP(hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&field_kernel<true, true>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-    VFPS_HIP(hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&field_kernel<true, false>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-    VFPS_HIP(hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&field_kernel<false, true>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    for (int k = 1; k < 4; k++) {
+        for (const void* fn : {field_fn<FIELD_PLAIN>((k & 1) != 0, (k & 2) != 0),
+                               field_fn<FIELD_CHIRP>((k & 1) != 0, (k & 2) != 0)}) {
+            VFPS_HIP(hipFuncSetAttribute(
+                fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+        }
+    }
     return VFPS_OK;
 }
 

@@ -36,6 +36,13 @@ struct FieldParams {
     unsigned long long* tstamp;  // optional phase timestamps (block 0)
 };
 
+// Which transforms a field kernel is made for: powers of two and direct sums,
+// chirps, or all of them (instances of several lengths in one launch).  The
+// chirp's two transforms of twice the length take 120 registers and spill; in
+// one kernel with the others they cost those 0.5 us of 14.6.
+enum FieldKind : int { FIELD_PLAIN = 0, FIELD_CHIRP = 1, FIELD_ANY = 2 };
+
+FieldKind field_kind(uint32_t M);
 FieldParams field_params(vfps_field* f);
 size_t field_lds_bytes(uint32_t M);
 int field_set_lds_limit(size_t bytes);

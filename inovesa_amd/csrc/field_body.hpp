@@ -43,7 +43,7 @@ __device__ __forceinline__ T opaque_after(T v)
     return v;
 }
 
-template <bool WAKE, bool CSR>
+template <bool WAKE, bool CSR, FieldKind KIND>
 __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
                            double2* lds)
 {
@@ -52,7 +52,8 @@ __device__ void field_body(const FieldParams& p, uint32_t block_bunch,
     const uint32_t M = p.M;
     // power-of-two M: radix-8 FFT with the half twiddle table in LDS;
     // other M: chirp DFT, or direct sums where M is short
-    const bool pow2 = fft_pow2(M), chirp = fft_chirp(M);
+    const bool pow2 = KIND != FIELD_CHIRP && fft_pow2(M);
+    const bool chirp = KIND == FIELD_CHIRP || (KIND == FIELD_ANY && fft_chirp(M));
     const uint32_t P = chirp ? chirp_len(M) : M;
     auto slot = [](uint32_t i) { return fft_slot(i); };
     // real sample i of the padded array: element i/2, real part for even i

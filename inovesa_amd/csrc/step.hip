@@ -276,7 +276,7 @@ toeplitz_kernel(uint32_t n, uint32_t M, const float2* __restrict__ Z,
 
 // ---- fields kernel (one workgroup per instance) ------------------------------
 
-template <bool WAKE, bool CSR>
+template <bool WAKE, bool CSR, FieldKind KIND>
 __global__ void __launch_bounds__(1024)
 fields_kernel(const FieldParams* __restrict__ params, uint32_t parity)
 {
@@ -286,12 +286,12 @@ fields_kernel(const FieldParams* __restrict__ params, uint32_t parity)
         p.proj = p.proj_alt;
     }
     p.parity = parity;
-    field_body<WAKE, CSR>(p, 0, flds);
+    field_body<WAKE, CSR, KIND>(p, 0, flds);
 }
 
 // One instance with its parameters by value: the kernel starts from its
 // arguments instead of a load of the parameter block through a pointer.
-template <bool WAKE, bool CSR>
+template <bool WAKE, bool CSR, FieldKind KIND>
 __global__ void __launch_bounds__(1024)
 field_one_kernel(FieldParams p, uint32_t parity)
 {
@@ -300,30 +300,44 @@ field_one_kernel(FieldParams p, uint32_t parity)
         p.proj = p.proj_alt;
     }
     p.parity = parity;
-    field_body<WAKE, CSR>(p, 0, flds);
+    field_body<WAKE, CSR, KIND>(p, 0, flds);
 }
 
 template <bool WAKE, bool CSR>
-static const void* fields_fn(bool one)
+static const void* fields_fn(bool one, FieldKind kind)
 {
-    return one ? reinterpret_cast<const void*>(&field_one_kernel<WAKE, CSR>)
-               : reinterpret_cast<const void*>(&fields_kernel<WAKE, CSR>);
+    if (one) {
+        return kind == FIELD_PLAIN
+                   ? reinterpret_cast<const void*>(
+                         &field_one_kernel<WAKE, CSR, FIELD_PLAIN>)
+                   : reinterpret_cast<const void*>(
+                         &field_one_kernel<WAKE, CSR, FIELD_CHIRP>);
+    }
+    switch (kind) {
+    case FIELD_PLAIN:
+        return reinterpret_cast<const void*>(&fields_kernel<WAKE, CSR, FIELD_PLAIN>);
+    case FIELD_CHIRP:
+        return reinterpret_cast<const void*>(&fields_kernel<WAKE, CSR, FIELD_CHIRP>);
+    default:
+        return reinterpret_cast<const void*>(&fields_kernel<WAKE, CSR, FIELD_ANY>);
+    }
 }
 
-int launch_fields(bool wake, bool csr, const FieldParams* params_d,
-                  uint32_t ninst, size_t lds, uint32_t parity,
+int launch_fields(bool wake, bool csr, FieldKind kind,
+                  const FieldParams* params_d, uint32_t ninst, size_t lds,
+                  uint32_t parity,
                   hipStream_t st, const FieldParams* params_h)
 {
     const bool one = ninst == 1 && params_h;
     const void* fn;
     if (wake && csr) {
-        fn = fields_fn<true, true>(one);
+        fn = fields_fn<true, true>(one, kind);
     } else if (wake) {
-        fn = fields_fn<true, false>(one);
+        fn = fields_fn<true, false>(one, kind);
     } else if (csr) {
-        fn = fields_fn<false, true>(one);
+        fn = fields_fn<false, true>(one, kind);
     } else {
-        fn = fields_fn<false, false>(one);
+        fn = fields_fn<false, false>(one, kind);
     }
     if (lds > 65536) {
         VFPS_HIP(hipFuncSetAttribute(fn,
@@ -413,7 +427,7 @@ static int step_launch_fused(vfps_step* s, uint32_t parity, hipStream_t st)
 {
     if (!s->direct) {
         int rc = launch_fields(s->desc.use_wake != 0, s->desc.use_csr != 0,
-                               s->fparams_d, 1, field_lds_bytes(s->M), parity, st,
+                               field_kind(s->M), s->fparams_d, 1, field_lds_bytes(s->M), parity, st,
                                &s->fparams_h);
         if (rc != VFPS_OK) return rc;
     }
@@ -446,8 +460,8 @@ static int step_launch_maps(vfps_step* s, uint32_t parity)
         return step_launch_fused(s, parity, st);
     }
     // per-map path, the loop body of src/main.cpp:948-1053
-    int rc = launch_fields(wake, csr, s->fparams_d, 1, field_lds_bytes(s->M), 0, st,
-                           &s->fparams_h);
+    int rc = launch_fields(wake, csr, field_kind(s->M), s->fparams_d, 1,
+                           field_lds_bytes(s->M), 0, st, &s->fparams_h);
     if (rc != VFPS_OK) return rc;
     vfps_mesh *t1 = s->t1, *t2 = s->t2, *t3 = s->t3;
     if (wake) {
@@ -1521,7 +1535,7 @@ int vfps_step_timing(vfps_step* s, uint32_t nsteps, float* ms_wake,
             const uint32_t par = s->parity;
             hipEventRecord(e0, st);
             rc = launch_fields(s->desc.use_wake != 0, s->desc.use_csr != 0,
-                               s->fparams_d, 1, field_lds_bytes(s->M), par, st,
+                               field_kind(s->M), s->fparams_d, 1, field_lds_bytes(s->M), par, st,
                                &s->fparams_h);
             hipEventRecord(e1, st);
             if (rc == VFPS_OK) {

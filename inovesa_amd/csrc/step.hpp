@@ -111,8 +111,9 @@ void toeplitz_tables(uint32_t n, uint32_t M, const float2* Z,
 // the longest of their transforms needs.  params_h:
 // the host copy of the parameters of a single instance, passed by value,
 // or null to read them from params_d.
-int launch_fields(bool wake, bool csr, const FieldParams* params_d,
-                  uint32_t ninst, size_t lds, uint32_t parity,
+int launch_fields(bool wake, bool csr, FieldKind kind,
+                  const FieldParams* params_d, uint32_t ninst, size_t lds,
+                  uint32_t parity,
                   hipStream_t st, const FieldParams* params_h = nullptr);
 // close a run: with close_csr, the last step's CSR power from the tiles'
 // shares (direct form; the next step's closing workgroup does this
