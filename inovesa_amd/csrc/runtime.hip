@@ -1,6 +1,7 @@
 // Device handle, errors and the PhaseSpace object (inc/PS/PhaseSpace.hpp).
 #include <algorithm>
 #include <cmath>
+#include <memory>
 #include <numeric>
 #include <stdexcept>
 
@@ -740,6 +741,7 @@ int vfps_mesh_create(vfps_dev* dev, uint32_t nb, uint32_t n, float qmin,
     if (rc != VFPS_OK) {
         return rc;
     }
+    std::unique_ptr<vfps_mesh, void (*)(vfps_mesh*)> guard(m, mesh_free);
     m->charge = charge;
     m->current = current;
     hipStream_t st = dev->stream;
@@ -764,7 +766,7 @@ int vfps_mesh_create(vfps_dev* dev, uint32_t nb, uint32_t n, float qmin,
     if ((rc = vfps_mesh_project_y(m)) != VFPS_OK) return rc;
     if ((rc = launch_integrate(m)) != VFPS_OK) return rc;
     VFPS_HIP(hipStreamSynchronize(st));
-    *out = m;
+    *out = guard.release();
     return VFPS_OK;
     VFPS_TRY_END
 }
@@ -780,6 +782,7 @@ int vfps_mesh_clone(const vfps_mesh* src, vfps_mesh** out)
     if (rc != VFPS_OK) {
         return rc;
     }
+    std::unique_ptr<vfps_mesh, void (*)(vfps_mesh*)> guard(m, mesh_free);
     m->charge = src->charge;
     m->current = src->current;
     hipStream_t st = src->dev->stream;
@@ -789,7 +792,7 @@ int vfps_mesh_clone(const vfps_mesh* src, vfps_mesh** out)
     if ((rc = vfps_mesh_project_y(m)) != VFPS_OK) return rc;
     if ((rc = launch_integrate(m)) != VFPS_OK) return rc;
     VFPS_HIP(hipStreamSynchronize(st));
-    *out = m;
+    *out = guard.release();
     return VFPS_OK;
     VFPS_TRY_END
 }

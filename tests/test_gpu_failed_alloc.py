@@ -118,3 +118,18 @@ def test_results_without_the_pinned_buffer():
         for a, e in zip(np.atleast_1d(without[k]), np.atleast_1d(with_it[k])):
             np.testing.assert_array_equal(a, e, err_msg=k)
     """)
+
+
+def test_refused_meshes_are_freed():
+    """A mesh whose row exceeds the LDS of a CU is refused after its 6.7 GB
+    are allocated; nothing of it stays."""
+    run_alone("""
+    keep = V.PhaseSpace(32, -6.0, 6.0, 1e-3, -6.0, 6.0, 1e6)
+    live = faults.hip_faults_live()
+    try:
+        V.PhaseSpace(40961, -6.0, 6.0, 1e-3, -6.0, 6.0, 1e6)
+        sys.exit("a row beyond the LDS was accepted")
+    except V.VfpsInvalid:
+        pass
+    assert faults.hip_faults_live() == live
+    """)
