@@ -540,9 +540,10 @@ VFPS_API int vfps_batch_set_merge(vfps_batch* b, int merge);
 VFPS_API int vfps_batch_retile_size(vfps_batch* b, uint32_t n,
                                     uint32_t tile_rows, uint32_t threads,
                                     int persistent);
-/* the launches of one step, cap rows of 4: workgroup size, tiles in the
- * block map (with padding), workgroups launched (fewer than the tiles:
- * persistent), dynamic LDS bytes; *ngroups = number of launches */
+/* the launches of one step, cap rows of 4: workgroup size, entries of the
+ * block map (tiles or strips, a closing workgroup per direct-wake instance in
+ * tiles, padding), workgroups launched (fewer than the entries: persistent),
+ * dynamic LDS bytes; *ngroups = number of launches */
 VFPS_API int vfps_batch_launches(vfps_batch* b, uint32_t* out, uint32_t cap,
                                  uint32_t* ngroups);
 /* Set the tiling of one instance by hand: tile rows, workgroup size and

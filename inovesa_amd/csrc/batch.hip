@@ -910,7 +910,8 @@ int vfps_batch_timing(vfps_batch* b, uint32_t nsteps, float* ms_step)
 
 // Choose the tile height and workgroup size per mesh size: for each size
 // class, every candidate (T, threads) is timed on that class's instances
-// alone (one launch per step, HIP events); the fastest is kept.  The state
+// alone (host launches, HIP events); the fastest is kept, a persistent one
+// only if it is also faster in captured runs of the whole batch.  The state
 // of every instance is saved before and restored after, so tuning does not
 // advance the simulation.  table rows: n, T, threads, microseconds per
 // step, chosen (1/0).
@@ -1016,10 +1017,13 @@ int vfps_batch_autotune(vfps_batch* b, uint32_t steps, float* table,
             orig.push_back({m->T, m->threads, m->strip, m->persist});
         }
         // strips exist for the kick-drift maps with the direct wake; below
-        // 1024 rows a size class has too few strips to fill the GPU beside
-        // the other classes of a batch (at 512 rows strips timed alone can
-        // beat tiles, yet the whole ragged batch then runs slower), so the
-        // tuner does not try them there
+        // 1024 rows a size class has few of them, and what they take alone
+        // says little about the whole batch, so the tuner does not try them
+        // there.  (64 meshes of 128^2 to 512^2 as chains, 52.8 us a step in
+        // tiles: of 18 strip forms of the 512^2 class two are faster, 49.5 us
+        // with 32 rows in tiles of 8 and 512 threads, 51.6, and 16 slower, up
+        // to 126.6; of 384^2 and 256^2 the best are 49.5 and 51.5.  To take
+        // them the choice would have to be made on the whole batch.)
         bool direct = true;  // the resident-grid form needs every member
         for (uint32_t i : cl.second) direct = direct && b->members[i]->direct;
         const bool strips_ok =

@@ -810,8 +810,8 @@ __device__ __forceinline__ void step_tile(const InstDesc& d, uint32_t inst,
                 // the same windows, read from the tables in global memory.
                 // (Up to four rows a wavefront at once save trips to L2 where
                 // rows are many and short, 64 meshes of 128^2 with T = 8: 13.0
-                // -> 12.2 us a step; but their registers and loads cost every
-                // other tiling: 4 of 512^2 with T = 2 17.8 -> 22.8, 4 of
+                // -> 12.2 us a step; but their registers and loads cost most
+                // other tilings: 4 of 512^2 with T = 2 17.8 -> 22.8, 4 of
                 // 1024^2 with T = 4 36.3 -> 49.9.)
                 const gdouble* win =
                     which == 0 ? wake_g + g0

@@ -25,7 +25,9 @@
 //      stored;
 //   H  the CSR shares were stored in B; strip 0 closes the step.
 // Every output value is the same sum, in the same order, as in the tile
-// kernel, so the two forms give the same bits (pinned by the batch tests).
+// kernel, so the two forms give the same values (pinned by the batch tests),
+// bit for bit but for the sign of a zero that every tap underflows to
+// (first_tap).
 #pragma once
 
 #include <type_traits>
@@ -728,11 +730,12 @@ __device__ __forceinline__ void strip_body(const InstDesc& d, uint32_t strip,
             // branch
             if (__all(win_ok)) {
                 if (rows_out == 4) {
-                    // the tile height of the production workload: 7 loads
-                    // for 4 rows where the largest height takes 11, and with
-                    // one first row their ring slots are scalar arithmetic
-                    // (the sub-tiles are VALU-bound: 16 meshes of 1024^2,
-                    // 64 steps, 4.72 -> 4.54 ms)
+                    // tiles of four rows, the height that strips of 1024 rows
+                    // are fastest with: 7 loads for 4 rows where the largest
+                    // height takes 11, and with one first row their ring
+                    // slots are scalar arithmetic (the sub-tiles are
+                    // VALU-bound: 16 meshes of 1024^2, 64 steps, 4.72 -> 4.54
+                    // ms).  Other heights read the largest one's window.
                     const int r0u = __builtin_amdgcn_readfirstlane(r0);
                     if (__all(r0 == r0u)) {
                         window(Four{}, r0u);

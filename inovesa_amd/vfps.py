@@ -822,8 +822,9 @@ class Batch:
                         (int(v) for v in out)))
 
     def launches(self):
-        """The launches of one step: threads, tiles, workgroups, LDS bytes
-        (fewer workgroups than tiles: a persistent launch)."""
+        """The launches of one step: threads, tiles (entries of the block map:
+        tiles or strips, closing workgroups, padding), workgroups, LDS bytes
+        (fewer workgroups than entries: a persistent launch)."""
         cap = 64
         out = np.zeros((cap, 4), np.uint32)
         ng = C.c_uint32()
