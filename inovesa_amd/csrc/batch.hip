@@ -314,7 +314,8 @@ int launch_chains(vfps_batch* b, uint32_t parity, uint32_t steps)
 }
 
 // one step of every instance, the FFT-wake members' wake potentials, CSR
-// powers and step counts first
+// powers and step counts first (also how no_graph members run: chains launched
+// from the host would go out one group after the other)
 int launch_step(vfps_batch* b, uint32_t parity)
 {
     for (const auto& f : b->fields) {
@@ -612,6 +613,7 @@ int vfps_batch_destroy(vfps_batch* b)
 int vfps_batch_run(vfps_batch* b, uint32_t nsteps)
 {
     VFPS_CHECK_ARG(b, "vfps_batch_run: NULL batch");
+    VFPS_TRY_BEGIN
     hipStream_t st = b->dev->stream;
     int rc = ensure_all(b);
     if (rc != VFPS_OK) return rc;
@@ -620,7 +622,6 @@ int vfps_batch_run(vfps_batch* b, uint32_t nsteps)
     // its own) and every member's error flag, in one launch
     static_assert(DEV_STAGE_BYTES >= sizeof(uint32_t) * 0xFFFFu,
                   "an error flag per instance");
-    VFPS_TRY_BEGIN
     const size_t count = b->members.size();
     DevStage stage(b->dev);
     uint32_t* err = stage.get<uint32_t>();
